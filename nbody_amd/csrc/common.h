@@ -21,6 +21,21 @@ struct NodeView {
 __device__ __forceinline__ int geo_level(int4 g) { return g.w & 0xff; }
 __device__ __forceinline__ int geo_nchild(int4 g) { return g.w >> 8; }
 
+// Counters that many wavefronts add to.  Atomics on one 128-byte line are
+// served one after the other, ~12 ns each however many XCDs they come from
+// (16,384 wavefronts adding once: 200 us on one line, 42 us on 8, 7 us on 64,
+// the time of the empty launch): every such counter has a line of its own, and
+// the sums that are only read later are kept in CNT_COPIES copies.
+constexpr int CNT_COPIES = 64;
+struct alignas(128) LineU32 {
+    uint32_t v;
+};
+struct alignas(128) LineTotals {
+    unsigned long long m2l, p2p, split;
+    unsigned long long m2lx;       // M2L entries between different levels
+    unsigned long long p2p_inter;  // particle pairs of the P2P kernels
+};
+
 // Device-side counters of one force evaluation.  Written by kernels, read by
 // the host once after the tree build and once after the walk's first phase.
 struct Counters {
@@ -30,16 +45,18 @@ struct Counters {
     uint32_t overflow;                 // bit flags, see OVF_*
     uint32_t level_count[MAX_LEVELS + 1];
     uint32_t level_off[MAX_LEVELS + 2];
-    uint32_t carried[MAX_LEVELS + 2];  // walk: carried leaf rows per depth
-    uint32_t sl_used;                  // walk: split-list entries used
-    uint32_t rows_used;
-    uint32_t m2l_pool_used;            // walk: phase-1 segment pools used
-    uint32_t p2p_pool_used;
-    unsigned long long m2l_total, p2p_total, p2p_inter, split_total;
-    unsigned long long m2lx_total;     // walk: M2L entries between different levels
-    uint32_t far_blocks, far_pairs;    // M2L: deferred pairs (level gap >= 2)
+    // (from here to far_pairs: cleared before each walk)
+    alignas(128) uint32_t carried[MAX_LEVELS + 2];  // walk: carried leaf rows per depth
+    LineU32 sl_used;                   // walk: split-list entries used
+    LineU32 m2l_pool_used;             // walk: phase-1 segment pools used
+    LineU32 p2p_pool_used;
+    LineTotals tot[CNT_COPIES];
+    alignas(128) unsigned long long near_used;  // near field: work items (low half), slots asked for (high half)
+    LineU32 far_pairs;                 // M2L: deferred pairs (level gap >= 2)
     uint32_t nonfinite;
     uint32_t outside;                  // fixed root box: a particle lies outside it
+    // sums over tot, made by the host when it has read the counters
+    unsigned long long m2l_total, p2p_total, p2p_inter, split_total, m2lx_total;
 };
 
 // OVF_GEOM: a same-level M2L block found a pair count or a source position
@@ -73,6 +90,18 @@ template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+    return v;
+}
+
+// inclusive prefix sum over the wavefront
+template <typename T>
+__device__ __forceinline__ T wave_prefix(T v) {
+    const int lane = __lane_id();
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const T y = __shfl_up(v, o, WAVE);
+        if (lane >= o) v += y;
+    }
     return v;
 }
 

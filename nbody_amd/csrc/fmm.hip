@@ -16,6 +16,7 @@
 #include "common.h"
 #include "expansion.h"
 #include "launch.h"
+#include "near.h"
 
 namespace nbh {
 
@@ -89,8 +90,11 @@ __global__ __launch_bounds__(256) void l2p_kernel(FmmParams F, State S, uint32_t
     for (int k = 0; k < NC; ++k) L[k] = Ls[k];
     float phi, gx, gy, gz;
     l2p_eval<P>(me.x, me.y, me.z, L, phi, gx, gy, gz);
-    // the P2P kernel left the raw near-field sums in (ax, ay, az, pot)
-    const float nx = S.ax[i], ny = S.ay[i], nz = S.az[i], nph = S.pot[i];
+    // the P2P kernel left the raw near-field sums in (ax, ay, az, pot), or, of
+    // a leaf whose list was cut, one partial sum per item
+    float4 nr;
+    if (!near_partial_sum(F, F.pleaf[i], i, nr)) nr = make_float4(S.ax[i], S.ay[i], S.az[i], S.pot[i]);
+    const float nx = nr.x, ny = nr.y, nz = nr.z, nph = nr.w;
     const float fac = (float)(S.charge[i] / S.mass[i]) * F.G;
     const float axo = fac * (nx + gx), ayo = fac * (ny + gy), azo = fac * (nz + gz);
     S.ax[i] = axo;
@@ -289,12 +293,93 @@ __global__ __launch_bounds__(256) void p2p_kernel(FmmParams F, State S, uint32_t
             if (POT) S.pot[i] = ph;
         }
     }
-    if (lane == 0 && inter) atomicAdd(F.p2p_inter, inter);
+    if (lane == 0 && inter) atomicAdd(&F.tot[blockIdx.x % CNT_COPIES].p2p_inter, inter);
 }
 
 // ---------------------------------------------------------------------------
-// P2P, staged: one wavefront per target leaf, sources flattened across the
-// leaf's P2P list.  Up to 64 list entries at a time are read by the lanes
+// Near-field work items.  A leaf's list can be hundreds of times the mean (a
+// coarse leaf at the edge of a dense region meets every small leaf of it), and
+// a small system has fewer leaves than the GPU has wavefronts: with one
+// wavefront per leaf the longest list was the kernel's time.  So a list of more
+// than G batches is cut into items of at most G, G = the evaluation's batches
+// / NEAR_BATCHES (about three rounds of resident wavefronts; 1 for small
+// systems), and each item leaves its partial sums in a slot that the join
+// kernel adds up in order (no atomics: the sums do not depend on which item
+// ran first).  P2P kernel, one wavefront per leaf -> items, with the pair
+// count's atomics spread over CNT_COPIES lines: Plummer 5003 100 -> 21 us,
+// 30,011 (p = 5) 682 -> 86 us, two spheres of 150,001 (p = 6, theta = 0.4)
+// 5.65 -> 1.1 ms, the adjoint's kernel at 16,384 590 -> 190 us; 1,048,576
+// beside the M2L kernels 2.06 -> 1.66 ms (there the atomics alone, one per
+// leaf at ~12 ns, took 1.4 ms).
+__global__ __launch_bounds__(256) void near_plan_kernel(FmmParams F, uint32_t num_leaves) {
+    Counters* C = const_cast<Counters*>(F.C);
+    if (C->overflow & OVF_WALK) return;
+    if (num_leaves == DEV_COUNT) num_leaves = C->num_leaves;
+    const int lane = lane_id(), wave = threadIdx.x / WAVE;
+    constexpr int NW = 256 / WAVE;
+    __shared__ uint32_t wsum[NW][2];
+    __shared__ unsigned long long first;
+    static_assert(CNT_COPIES == WAVE, "one copy per lane");
+    const unsigned long long entries = wave_sum(C->tot[lane].p2p);
+    const uint32_t G = (uint32_t)max(1ull, (entries / WAVE + NEAR_BATCHES - 1) / NEAR_BATCHES);
+    for (uint32_t t0 = blockIdx.x * 256; t0 < num_leaves; t0 += gridDim.x * 256) {  // uniform over the workgroup
+        const uint32_t t = t0 + threadIdx.x;
+        int A = 0;
+        uint32_t nb = 0, tc = 0, k = 0;
+        if (t < num_leaves) {
+            A = (int)F.leaf_ids[t];
+            for (uint32_t r = F.lists.first[A]; r != NO_ROW; r = F.lists.next[r])
+                nb += (F.lists.p_cnt[r] + WAVE - 1) / WAVE;
+            tc = ((uint32_t)F.nodes.link[A].y + WAVE - 1) / WAVE;
+            k = max(1u, (nb + G - 1) / G);
+        }
+        // items, and slots for the leaves that are cut; items are reserved for
+        // every leaf as if it found its slots, which is at most what they all
+        // take uncut, and the slots there are
+        uint32_t want = k > 1 ? tc * k : 0u;
+        const uint32_t wpre = wave_prefix(want), ipre = wave_prefix(tc);
+        if (lane == WAVE - 1) {
+            wsum[wave][0] = wpre;
+            wsum[wave][1] = ipre;
+        }
+        __syncthreads();
+        uint32_t wb = wpre - want, ib = ipre - tc, wt = 0, it = 0;
+        for (int w = 0; w < NW; ++w) {
+            if (w < wave) {
+                wb += wsum[w][0];
+                ib += wsum[w][1];
+            }
+            wt += wsum[w][0];
+            it += wsum[w][1];
+        }
+        if (threadIdx.x == 0) first = atomicAdd(&C->near_used, (unsigned long long)wt << 32 | it);
+        __syncthreads();
+        // uncut items from 0 on; the items of a cut leaf stand beside its slots
+        const uint32_t s0 = (uint32_t)(first >> 32) + wb, i0 = (uint32_t)first + ib;
+        if (want && (unsigned long long)s0 + want > F.near_slot_cap) k = 1;
+        if (t < num_leaves) {
+            F.near_k[A] = k;
+            F.near_first[A] = s0;
+            NearItem* uncut = F.near_items + F.near_slot_cap;
+            for (uint32_t c = 0; c < tc; ++c) {
+                // (the leaf's place among the uncut items: empty if it was cut)
+                uncut[i0 + c] = NearItem{A, c * WAVE, 0, k > 1 ? 0u : nb, NO_SLOT, {0, 0, 0}};
+                for (uint32_t j = 0; k > 1 && j < k; ++j) {
+                    const uint32_t b0 = (uint32_t)((unsigned long long)nb * j / k);
+                    const uint32_t b1 = (uint32_t)((unsigned long long)nb * (j + 1) / k);
+                    F.near_items[s0 + c * k + j] = NearItem{A, c * WAVE, b0, b1, s0 + c * k + j, {0, 0, 0}};
+                }
+            }
+            // slots that this leaf asked for beyond the last: nothing to do
+            if (want && k == 1)
+                for (uint32_t j = s0; j < F.near_slot_cap; ++j) F.near_items[j] = NearItem{A, 0, 0, 0, NO_SLOT, {0, 0, 0}};
+        }
+        __syncthreads();
+    }
+}
+
+// P2P, staged: one wavefront per near-field item, sources flattened across the
+// batches.  Up to 64 list entries at a time are read by the lanes
 // (one entry each: centre offset, first particle, count) and prefix-summed;
 // then 64 source particles at a time are gathered (each lane finds its
 // source's entry from a bitmask of the entry starts), shifted into the target
@@ -318,8 +403,7 @@ constexpr int p2p_stage_slots() { return SPL == 1 ? 96 : 160; }
 // potential); else the self pair and the empty slots are skipped by index.
 // POT: the potential sums too (else the accelerations alone).
 template <bool SOFT, int SPL, bool POT>
-__device__ __forceinline__ void p2p_staged_body(const FmmParams& F, const State& S, uint32_t num_leaves) {
-    // (num_leaves == DEV_COUNT: the leaf count of the device counters)
+__device__ __forceinline__ void p2p_staged_body(const FmmParams& F, const State& S) {
     constexpr int P2P_STAGE = p2p_stage_slots<SPL>();
     constexpr int CHUNK = WAVE * SPL;
     __shared__ float4 stage_s[P2P_WAVES][P2P_STAGE];
@@ -336,10 +420,8 @@ __device__ __forceinline__ void p2p_staged_body(const FmmParams& F, const State&
     int* sidx = stage_i[wslot];
     int2* ent = ent_s[wslot];
     float4* entd = entd_s[wslot];
-    if (num_leaves == DEV_COUNT) {
-        if (F.C->overflow & OVF_WALK) return;
-        num_leaves = F.C->num_leaves;
-    }
+    // (a captured step whose tree or walk outgrew its buffers stands down)
+    const NearCount items = near_count(F);
     // slots past the chunk are never staged: zero charges for good
     static_assert(P2P_STAGE - CHUNK <= WAVE, "one slot per lane");
     if (lane < P2P_STAGE - CHUNK) {
@@ -348,13 +430,16 @@ __device__ __forceinline__ void p2p_staged_body(const FmmParams& F, const State&
     }
     const uint32_t nw = gridDim.x * P2P_WAVES;
     unsigned long long inter = 0;  // particle pairs, summed over the lanes at the end
-    for (uint32_t w = blockIdx.x * P2P_WAVES + wslot; w < num_leaves; w += nw) {
-        const int A = (int)F.leaf_ids[w];
+    for (uint32_t w = blockIdx.x * P2P_WAVES + wslot; w < items.cut + items.uncut; w += nw) {
+        const NearItem item = near_item(F, items, w);
+        if (item.b1 == 0) continue;
+        const int A = item.node;
+        const int t0 = (int)item.t0;
         const int4 ga = F.nodes.geo[A];
         const int4 la = F.nodes.link[A];
         const float unit = F.unit[F.nodes.sys[A]];
         const float eps2 = F.eps2;
-        for (int t0 = 0; t0 < la.y; t0 += WAVE) {
+        {
             const int nt = min(WAVE, la.y - t0);
             const int splits = WAVE / nt;
             // ceil(x / splits) = umulhi(x + splits - 1, magic) for x <= 64
@@ -364,8 +449,7 @@ __device__ __forceinline__ void p2p_staged_body(const FmmParams& F, const State&
             const int i = la.x + t0 + ti;
             const float4 me = F.pf[i];
             float ax = 0.f, ay = 0.f, az = 0.f, ph = 0.f;
-            for (uint32_t r = F.lists.first[A]; r != NO_ROW; r = F.lists.next[r])
-            for (uint32_t eb = F.lists.p_start[r], e_end = eb + F.lists.p_cnt[r]; eb < e_end; eb += WAVE) {
+            near_batches(F.lists, A, item.b0, item.b1, [&](uint32_t eb, uint32_t e_end) {
                 const int ne = (int)min((uint32_t)WAVE, e_end - eb);
                 int cnt = 0, beg = 0;
                 float dx = 0.f, dy = 0.f, dz = 0.f;
@@ -470,9 +554,10 @@ __device__ __forceinline__ void p2p_staged_body(const FmmParams& F, const State&
                     }
                     wave_lds_sync();
                 }
-            }
-            // the self term q_i/eps sits in exactly one stride's partial sum
-            if (POT && SOFT && sp == 0) ph -= me.w * __builtin_amdgcn_rsqf(eps2);
+            });
+            // the self term q_i/eps sits in exactly one stride's partial sum of
+            // one item; it is taken from the first item's
+            if (POT && SOFT && sp == 0 && item.b0 == 0) ph -= me.w * __builtin_amdgcn_rsqf(eps2);
             // combine the source strides of each target
             {
                 const float ax0 = ax, ay0 = ay, az0 = az, ph0 = ph;
@@ -485,26 +570,29 @@ __device__ __forceinline__ void p2p_staged_body(const FmmParams& F, const State&
             }
             if (sp == 0) {
                 // raw near-field sums; l2p_kernel adds the far field
-                S.ax[i] = ax;
-                S.ay[i] = ay;
-                S.az[i] = az;
-                if (POT) S.pot[i] = ph;
+                if (item.slot != NO_SLOT) {
+                    F.near_part[(size_t)item.slot * WAVE + ti] = make_float4(ax, ay, az, ph);
+                } else {
+                    S.ax[i] = ax;
+                    S.ay[i] = ay;
+                    S.az[i] = az;
+                    if (POT) S.pot[i] = ph;
+                }
             }
         }
     }
     inter = wave_sum(inter);
-    if (lane == 0 && inter) atomicAdd(F.p2p_inter, inter);
+    if (lane == 0 && inter) atomicAdd(&F.tot[blockIdx.x % CNT_COPIES].p2p_inter, inter);
 }
 
 template <int P, int SPL, bool POT>
-__global__ __launch_bounds__(WAVE * P2P_WAVES) void p2p_staged_kernel(FmmParams F, State S, uint32_t num_leaves) {
-    p2p_staged_body<true, SPL, POT>(F, S, num_leaves);
+__global__ __launch_bounds__(WAVE * P2P_WAVES) void p2p_staged_kernel(FmmParams F, State S) {
+    p2p_staged_body<true, SPL, POT>(F, S);
 }
 
 template <int P, int SPL, bool POT>
-__global__ __launch_bounds__(WAVE * P2P_WAVES) void p2p_staged_unsoftened_kernel(FmmParams F, State S,
-                                                                                 uint32_t num_leaves) {
-    p2p_staged_body<false, SPL, POT>(F, S, num_leaves);
+__global__ __launch_bounds__(WAVE * P2P_WAVES) void p2p_staged_unsoftened_kernel(FmmParams F, State S) {
+    p2p_staged_body<false, SPL, POT>(F, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -892,12 +980,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(P <= 4 ? 4 
         // deferred pairs: one contiguous run per target
         const bool defer = act && nfar > 0;
         if (!__ballot(defer)) continue;  // uniform
+        // (one reservation for both halves)
+        const uint32_t nf0 = __shfl(defer ? nfar : 0u, 0, WAVE), nf1 = __shfl(defer ? nfar : 0u, 32, WAVE);
         uint32_t s0 = 0;
-        if (defer && sub == 0) {
-            atomicAdd(&F.far_cnt[0], 1u);
-            s0 = atomicAdd(&F.far_cnt[1], nfar);
-        }
-        s0 = __shfl(s0, lane & 32, WAVE);
+        if (lane == 0) s0 = atomicAdd(F.far_cnt, nf0 + nf1);
+        s0 = __shfl(s0, 0, WAVE) + (half ? nf0 : 0u);
         // the capacity is the walk's count of other-level entries, which
         // bounds the deferred pairs (a captured step sizes it from the
         // previous step and flags a shortfall)
@@ -945,7 +1032,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
         if (F.C->overflow & OVF_WALK) return;
         num_nodes = F.C->num_nodes;
     }
-    const uint32_t npairs = min(F.far_cnt[1], F.far_cap);
+    const uint32_t npairs = min(*F.far_cnt, F.far_cap);
     const int lane = lane_id();
     const uint32_t w0 = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE * WAVE;
     for (uint32_t base = w0; base < npairs; base += gridDim.x * blockDim.x) {  // uniform
@@ -986,8 +1073,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     }
 }
 
-__global__ void zero_u32x2_kernel(uint32_t* p) {
-    if (threadIdx.x < 2) p[threadIdx.x] = 0u;
+__global__ void zero_word_kernel(uint32_t* p) {
+    if (threadIdx.x == 0) *p = 0u;
 }
 
 __global__ void zero_f32_kernel(float* p, size_t n) {
@@ -1022,7 +1109,6 @@ static void launch_m2l_pq_pot(const FmmParams& F, const M2LPlan& plan, int parts
         return;
     }
     if (parts & M2L_REST) {
-        hipLaunchKernelGGL(zero_u32x2_kernel, dim3(1), dim3(64), 0, st, F.far_cnt);
         // cells above the tabled levels have no same-level pairs: L starts at 0
         if (plan.dev) {
             hipLaunchKernelGGL(zero_top_kernel, dim3(64), dim3(256), 0, st, F.L, F.C, F.dlevel0, F.ncp);
@@ -1137,21 +1223,18 @@ static void launch_p2p_t(const FmmParams& F, const State& S, uint32_t num_leaves
 }
 
 template <int P, int SPL, bool POT>
-static void launch_p2p_staged_pot(const FmmParams& F, const State& S, uint32_t num_leaves, unsigned grid,
-                                  hipStream_t st) {
+static void launch_p2p_staged_pot(const FmmParams& F, const State& S, unsigned grid, hipStream_t st) {
     if (F.eps2 > 0.f)
-        hipLaunchKernelGGL((p2p_staged_kernel<P, SPL, POT>), dim3(grid), dim3(WAVE * P2P_WAVES), 0, st, F, S,
-                           num_leaves);
+        hipLaunchKernelGGL((p2p_staged_kernel<P, SPL, POT>), dim3(grid), dim3(WAVE * P2P_WAVES), 0, st, F, S);
     else
-        hipLaunchKernelGGL((p2p_staged_unsoftened_kernel<P, SPL, POT>), dim3(grid), dim3(WAVE * P2P_WAVES), 0, st,
-                           F, S, num_leaves);
+        hipLaunchKernelGGL((p2p_staged_unsoftened_kernel<P, SPL, POT>), dim3(grid), dim3(WAVE * P2P_WAVES), 0, st, F,
+                           S);
 }
 template <int P, int SPL>
-static void launch_p2p_staged_t(const FmmParams& F, const State& S, uint32_t num_leaves, uint32_t items,
-                                hipStream_t st) {
+static void launch_p2p_staged_t(const FmmParams& F, const State& S, uint32_t items, hipStream_t st) {
     const unsigned grid = std::min<unsigned>(ceil_div(items, P2P_WAVES), 65536u);
-    if (F.pot) launch_p2p_staged_pot<P, SPL, true>(F, S, num_leaves, grid, st);
-    else launch_p2p_staged_pot<P, SPL, false>(F, S, num_leaves, grid, st);
+    if (F.pot) launch_p2p_staged_pot<P, SPL, true>(F, S, grid, st);
+    else launch_p2p_staged_pot<P, SPL, false>(F, S, grid, st);
 }
 #define NBH_DISPATCH_P(p, call)          \
     switch (p) {                         \
@@ -1187,12 +1270,15 @@ void launch_l2l_level(int p, const FmmParams& F, int level, uint32_t count, uint
     if (count == DEV_COUNT) off = (uint32_t)level;
     NBH_DISPATCH_P(p, launch_l2l_t<PP>(F, count, off, items, st));
 }
-void launch_p2p_staged(int p, int chunk, const FmmParams& F, const State& S, uint32_t num_leaves, hipStream_t st,
-                       uint32_t grid_items) {
+void launch_near_plan(const FmmParams& F, uint32_t num_leaves, hipStream_t st, uint32_t grid_items) {
     if (!num_leaves) return;
     const uint32_t items = grid_items_of(num_leaves, grid_items);
-    if (chunk == 128) NBH_DISPATCH_P(p, (launch_p2p_staged_t<PP, 2>(F, S, num_leaves, items, st)))
-    else NBH_DISPATCH_P(p, (launch_p2p_staged_t<PP, 1>(F, S, num_leaves, items, st)))
+    hipLaunchKernelGGL(near_plan_kernel, dim3(ceil_div(items, 256)), dim3(256), 0, st, F, num_leaves);
+}
+void launch_p2p_staged(int p, int chunk, const FmmParams& F, const State& S, hipStream_t st, uint32_t grid_items) {
+    const uint32_t items = std::max<uint32_t>(grid_items, 1u);
+    if (chunk == 128) NBH_DISPATCH_P(p, (launch_p2p_staged_t<PP, 2>(F, S, items, st)))
+    else NBH_DISPATCH_P(p, (launch_p2p_staged_t<PP, 1>(F, S, items, st)))
 }
 void launch_dtable(int q, const FmmParams& F, float* out, int level0, int nlev, int E, int a, int b, int shift,
                    int nsys, const uint32_t* offs, int nrows, hipStream_t st) {
@@ -1230,6 +1316,9 @@ void launch_m2l_parts(int p, int q, const FmmParams& F, const M2LPlan& plan, int
 #undef NBH_M2L
 }
 void launch_m2l(int p, int q, const FmmParams& F, const M2LPlan& plan, hipStream_t st) {
+    // a second M2L on the same lists (the adjoint's): the forward one's
+    // deferred pairs, counted from the walk's zero on, are done
+    if (F.dtab) hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(64), 0, st, F.far_cnt);
     launch_m2l_parts(p, q, F, plan, M2L_LEVELS | M2L_REST, -1, st);
 }
 void launch_p2p(int p, const FmmParams& F, const State& S, uint32_t num_leaves, hipStream_t st) {

@@ -90,6 +90,26 @@ struct ListView {
     const int* p_pool;
 };
 
+// One wavefront's share of the near field: the targets [t0, t0 + 64) of a leaf
+// against batches [b0, b1) of its P2P list.  A batch is up to 64 consecutive
+// entries of one row; batches are numbered along the leaf's row chain.  slot:
+// where the partial sums go (NO_SLOT: the item is the whole list, and its sums
+// are the particles' near field).
+constexpr uint32_t NO_SLOT = 0xffffffffu;
+struct alignas(16) NearItem {
+    int node;
+    uint32_t t0, b0, b1;
+    uint32_t slot;
+    uint32_t pad[3];
+};
+// Batches that an evaluation's lists are cut towards, and the most slots
+// (1 KiB each): the items of a split leaf hold more than half of
+// (batches / NEAR_BATCHES) batches each, so that they stay below NEAR_SLOTS
+// (a leaf that finds no slot left is not split).  The items of split leaves
+// stand at the index of their slot, those of the others from the slot
+// capacity on.
+constexpr uint32_t NEAR_BATCHES = 16384, NEAR_SLOTS = 2 * NEAR_BATCHES;
+
 // ---- particle state in sorted order (FP64 positions/velocities)
 struct State {
     double *x, *y, *z, *vx, *vy, *vz, *mass, *charge;
@@ -116,8 +136,17 @@ struct FmmParams {
     const uint32_t* leaf_ids;
     float4* pf;            // per particle: offset from its leaf centre, charge
     ListView lists;
-    unsigned long long* p2p_inter;  // statistics: particle pairs of the P2P kernels
+    LineTotals* tot;       // statistics: particle pairs of the P2P kernels (CNT_COPIES copies)
     uint32_t* pleaf;       // per particle: its leaf node
+    // near-field work items (null: one wavefront per leaf), and per leaf node
+    // the items its list is cut into and their first slot: item j of target
+    // chunk c has slot near_first + c near_k + j, target t of the chunk the
+    // sums near_part[64 slot + t]
+    NearItem* near_items;
+    uint32_t* near_k;
+    uint32_t* near_first;
+    float4* near_part;
+    uint32_t near_slot_cap;
     float* dtab;           // per system and level, derivative tensors of the same-level offsets (or null);
                            // system s, level l at row ((s dnlev + l - dlevel0) dsz + row)
     int dK, dlevel0, dnlev;
@@ -135,7 +164,7 @@ struct FmmParams {
     int* far_tgt;
     int* far_src;
     uint32_t far_cap;
-    uint32_t* far_cnt;     // [targets, pairs]
+    uint32_t* far_cnt;     // deferred pairs
     double eps2_64;
     int pot;               // 1: potentials too; 0: accelerations only (the tuned P2P and M2L kernels leave
                            // out the potential's terms, l2p_kernel does not write it)
@@ -154,9 +183,11 @@ void launch_l2l_level(int p, const FmmParams& F, int level, uint32_t count, uint
 // az, pot); launch_l2p adds the far field of the leaf's local expansion,
 // applies G q/m and the sign of the potential, and the kick v += a kick_dt
 void launch_p2p(int p, const FmmParams& F, const State& S, uint32_t num_leaves, hipStream_t st);
-// chunk: sources staged per wavefront round, 64 or 128 (the tile shape)
-void launch_p2p_staged(int p, int chunk, const FmmParams& F, const State& S, uint32_t num_leaves, hipStream_t st,
-                       uint32_t grid_items = 0);
+// chunk: sources staged per wavefront round, 64 or 128 (the tile shape);
+// grid_items: at least the items that near_plan makes (the kernel strides)
+void launch_p2p_staged(int p, int chunk, const FmmParams& F, const State& S, hipStream_t st, uint32_t grid_items);
+// cuts the leaves' P2P lists into items (F.near_items), before launch_p2p_staged
+void launch_near_plan(const FmmParams& F, uint32_t num_leaves, hipStream_t st, uint32_t grid_items = 0);
 void launch_l2p(int p, const FmmParams& F, const State& S, uint32_t n, double kick_dt, hipStream_t st);
 // M2L of order p with the truncation code q (expansion.h: m2l_deg(q) = p or
 // p + 1; q | M2L_ALL keeps every term of degree <= p + 1, q = p + 1 only
@@ -241,7 +272,7 @@ void launch_vjp_gather(const double* w_in, const uint32_t* id, float4* pw, uint3
 void launch_adj_kick(double* xb, double* vb, double* w, size_t m, double dt, double c, bool update, hipStream_t st);
 void launch_adj_accum(const double* g, const uint32_t* id, uint32_t n, double* xb, double* mb, hipStream_t st);
 void launch_fill_f64(double* p, size_t m, double v, hipStream_t st);
-void launch_vjp_near(int p, const FmmParams& F, const float4* pw, uint32_t n, uint32_t num_leaves, double* g,
+void launch_vjp_near(int p, const FmmParams& F, const float4* pw, uint32_t n, uint32_t grid_items, double* g,
                      hipStream_t st);
 void launch_vjp_chain(int p, int q, const M2LPlan& plan, const FmmParams& F, const FmmParams& Fw, const float4* pw,
                       uint32_t num_leaves, const uint32_t* level_count, const uint32_t* level_off, int depth,

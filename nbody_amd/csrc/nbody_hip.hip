@@ -84,6 +84,7 @@ struct GraphShape {
     uint32_t node_cap = 0;       // node arrays
     uint32_t node_items = 0;     // grid sizing: nodes, leaves
     uint32_t leaf_items = 0;
+    unsigned long long p2p_items = 0;  // P2P entries
     uint32_t depth_cap = 0;      // levels 0..depth_cap are processed
     uint32_t level_items[MAX_LEVELS + 1] = {};
     uint32_t walk_grid[MAX_LEVELS + 1] = {};
@@ -120,7 +121,7 @@ struct nbh_handle {
     int cur = 0;
     DevBuf sys_off, keys, keys_alt, perm, perm_alt, sort_tmp, tree_tmp, scan_tmp;
     DevBuf box, inv, unit, bbox_part;
-    DevBuf geo, link, nsys_of, node_begin, leaf_ids, M, L, Lx, pf, pleaf, dtab, xtab, far_src, far_tgt;
+    DevBuf geo, link, nsys_of, node_begin, leaf_ids, M, L, Lx, pf, pleaf, dtab, xtab, far_src, far_tgt, near_items, near_k, near_first, near_part;
     DevBuf row_node, row_first, row_next, row_sl_start, row_sl_cnt, sl, row_m_start, row_m_cnt, row_mx_cnt,
         row_p_start, row_p_cnt, m2l_pool, p2p_pool;
     unsigned long long m2l_pool_cap = 0, p2p_pool_cap = 0;
@@ -286,6 +287,18 @@ int validate_config(const nbh_config* c, std::string& why) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
+// partial-sum slots of a handle (1 KiB each): NEAR_SLOTS, fewer for a small
+// system, whose lists have fewer batches
+static uint32_t near_slot_cap(const nbh_handle* h) {
+    return (uint32_t)std::min<size_t>(NEAR_SLOTS, std::max<size_t>(4 * h->n, 1024));
+}
+// at least the near-field items of an evaluation with this many leaves and
+// P2P entries (for grids; the kernels stride)
+static uint32_t near_grid_items(const nbh_handle* h, uint64_t leaves, uint64_t entries) {
+    const uint64_t cut = std::min<uint64_t>(near_slot_cap(h), 2 * (entries / 64 + leaves));
+    return (uint32_t)std::min<uint64_t>(leaves + h->n / 64 + cut, 1u << 24);
+}
+
 static int alloc_nodes(nbh_handle* h, uint32_t need) {
     if (need <= h->node_cap) return NBH_OK;
     uint32_t cap = std::max<uint32_t>(need + need / 4, 1024);
@@ -298,6 +311,11 @@ static int alloc_nodes(nbh_handle* h, uint32_t need) {
     HIPCHK(h, h->L.ensure((size_t)cap * ncp * 4));
     HIPCHK(h, h->Lx.ensure((size_t)cap * ncp * 4));
     HIPCHK(h, h->row_first.ensure((size_t)cap * 4));
+    HIPCHK(h, h->near_k.ensure((size_t)cap * 4));
+    HIPCHK(h, h->near_first.ensure((size_t)cap * 4));
+    // items: every leaf's target chunks, and the slots of the leaves that are cut
+    HIPCHK(h, h->near_items.ensure((std::min<size_t>(cap, h->n) + h->n / 64 + near_slot_cap(h)) * sizeof(NearItem)));
+    HIPCHK(h, h->near_part.ensure((size_t)near_slot_cap(h) * 1024));
     HIPCHK(h, h->scan_tmp.ensure(scan_tmp_bytes(cap + 1) + 256));
     h->node_cap = cap;
     return NBH_OK;
@@ -306,6 +324,15 @@ static int alloc_nodes(nbh_handle* h, uint32_t need) {
 static int read_counters(nbh_handle* h) {
     HIPCHK(h, hipMemcpyAsync(h->hc, h->counters.p, sizeof(Counters), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    Counters& c = *h->hc;
+    c.m2l_total = c.p2p_total = c.p2p_inter = c.split_total = c.m2lx_total = 0;
+    for (const LineTotals& t : c.tot) {
+        c.m2l_total += t.m2l;
+        c.p2p_total += t.p2p;
+        c.p2p_inter += t.p2p_inter;
+        c.split_total += t.split;
+        c.m2lx_total += t.m2lx;
+    }
     return NBH_OK;
 }
 
@@ -384,6 +411,14 @@ static int build_tree(nbh_handle* h, const GraphShape* gs = nullptr) {
     return NBH_OK;
 }
 
+static void set_near(nbh_handle* h, FmmParams& F) {
+    F.near_items = h->near_items.as<NearItem>();
+    F.near_k = h->near_k.as<uint32_t>();
+    F.near_first = h->near_first.as<uint32_t>();
+    F.near_part = h->near_part.as<float4>();
+    F.near_slot_cap = near_slot_cap(h);
+}
+
 static FmmParams fmm_params(nbh_handle* h) {
     FmmParams F{};
     F.nodes = node_view(h);
@@ -407,8 +442,9 @@ static FmmParams fmm_params(nbh_handle* h) {
     F.lists.p_cnt = h->row_p_cnt.as<uint32_t>();
     F.lists.m_pool = h->m2l_pool.as<int>();
     F.lists.p_pool = h->p2p_pool.as<int>();
-    F.p2p_inter = &h->counters.as<Counters>()->p2p_inter;
+    F.tot = h->counters.as<Counters>()->tot;
     F.pleaf = h->pleaf.as<uint32_t>();
+    if (h->cfg.p2p == NBH_P2P_LANE) set_near(h, F);
     F.dtab = nullptr;
     F.Lx = nullptr;
     F.eps2_64 = h->cfg.eps * h->cfg.eps;
@@ -587,7 +623,7 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
         }
         if (ovf & OVF_SL) {
             h->sl_cap = (uint32_t)std::min<unsigned long long>(
-                std::max<unsigned long long>(2ull * h->sl_cap, h->hc->sl_used + h->hc->sl_used / 4 + waste_s),
+                std::max<unsigned long long>(2ull * h->sl_cap, h->hc->sl_used.v + h->hc->sl_used.v / 4 + waste_s),
                 0xffff0000ull);
             HIPCHK(h, h->sl.ensure((size_t)h->sl_cap * 4));
         }
@@ -598,12 +634,12 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
         }
         if (ovf & OVF_M2L) {
             h->m2l_pool_cap = std::min<unsigned long long>(
-                std::max<unsigned long long>(h->m2l_pool_cap * 2, h->hc->m2l_pool_used + waste_m), 0xffff0000ull);
+                std::max<unsigned long long>(h->m2l_pool_cap * 2, h->hc->m2l_pool_used.v + waste_m), 0xffff0000ull);
             HIPCHK(h, h->m2l_pool.ensure((size_t)h->m2l_pool_cap * 4));
         }
         if (ovf & OVF_P2P) {
             h->p2p_pool_cap = std::min<unsigned long long>(
-                std::max<unsigned long long>(h->p2p_pool_cap * 2, h->hc->p2p_pool_used + waste_p), 0xffff0000ull);
+                std::max<unsigned long long>(h->p2p_pool_cap * 2, h->hc->p2p_pool_used.v + waste_p), 0xffff0000ull);
             HIPCHK(h, h->p2p_pool.ensure((size_t)h->p2p_pool_cap * 4));
         }
         if (ovf & walk_bits) {
@@ -773,16 +809,23 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
         F.far_src = h->far_src.as<int>();
         F.far_tgt = h->far_tgt.as<int>();
         F.far_cap = (uint32_t)std::min<unsigned long long>(nx, 0xffffffffull);
-        F.far_cnt = &h->counters.as<Counters>()->far_blocks;
+        F.far_cnt = &h->counters.as<Counters>()->far_pairs.v;
     }
     // side stream, overlapping M2L and L2L: the near field (raw sums)
     if (!for_vjp) {
         HIPCHK(h, hipEventRecord(h->ev_walk, h->stream));
         HIPCHK(h, hipStreamWaitEvent(h->stream2, h->ev_walk, 0));
         record_side(h, 2);
-        if (gs) launch_p2p_staged(p, p2p_chunk(h), F, S, DEV_COUNT, h->stream2, gs->leaf_items);
-        else if (h->cfg.p2p == NBH_P2P_LANE) launch_p2p_staged(p, p2p_chunk(h), F, S, h->num_leaves, h->stream2);
-        else launch_p2p(p, F, S, h->num_leaves, h->stream2);
+        if (gs) {
+            launch_near_plan(F, DEV_COUNT, h->stream2, gs->leaf_items);
+            launch_p2p_staged(p, p2p_chunk(h), F, S, h->stream2, near_grid_items(h, gs->leaf_items, gs->p2p_items));
+        } else if (F.near_items) {
+            launch_near_plan(F, h->num_leaves, h->stream2);
+            launch_p2p_staged(p, p2p_chunk(h), F, S, h->stream2,
+                              near_grid_items(h, h->num_leaves, h->hc->p2p_total));
+        } else {
+            launch_p2p(p, F, S, h->num_leaves, h->stream2);
+        }
         record_side(h, 3);
         HIPCHK(h, hipEventRecord(h->ev_near, h->stream2));
     }
@@ -907,6 +950,7 @@ static void graph_shape_update(nbh_handle* h) {
     g.node_cap = nn + nn / 4 + 1024;
     g.node_items = nn + nn / 8 + 64;
     g.leaf_items = nl + nl / 8 + 64;
+    g.p2p_items = c.p2p_total + c.p2p_total / 8;
     g.depth_cap = std::min<uint32_t>(h->cfg.max_depth, c.depth + 2);
     unsigned long long blocks = 0;
     for (uint32_t l = 0; l <= g.depth_cap; ++l) {
@@ -921,12 +965,12 @@ static void graph_shape_update(nbh_handle* h) {
     // every workgroup may leave one unused chunk tail per depth
     const unsigned long long cap32 = 0xffff0000ull;
     g.m2l_cap = std::min(std::max<unsigned long long>(h->m2l_pool_cap,
-                                                      c.m2l_pool_used + c.m2l_pool_used / 4 + blocks * POOL_CHUNK_M),
+                                                      c.m2l_pool_used.v + c.m2l_pool_used.v / 4 + blocks * POOL_CHUNK_M),
                          cap32);
     g.p2p_cap = std::min(std::max<unsigned long long>(h->p2p_pool_cap,
-                                                      c.p2p_pool_used + c.p2p_pool_used / 4 + blocks * POOL_CHUNK_P),
+                                                      c.p2p_pool_used.v + c.p2p_pool_used.v / 4 + blocks * POOL_CHUNK_P),
                          cap32);
-    g.sl_cap = (uint32_t)std::min(std::max<unsigned long long>(h->sl_cap, c.sl_used + c.sl_used / 4 +
+    g.sl_cap = (uint32_t)std::min(std::max<unsigned long long>(h->sl_cap, c.sl_used.v + c.sl_used.v / 4 +
                                                                               blocks * POOL_CHUNK_S),
                                   cap32);
     g.row_cap = std::max<uint32_t>(h->row_cap, 2 * g.node_cap + 1024);
@@ -1403,7 +1447,8 @@ void nbh_destroy(nbh_handle* h) {
     h->st[1].release();
     DevBuf* all[] = {&h->sys_off, &h->keys, &h->keys_alt, &h->perm, &h->perm_alt, &h->sort_tmp, &h->tree_tmp,
                      &h->scan_tmp, &h->box, &h->inv, &h->unit, &h->bbox_part, &h->geo, &h->link, &h->nsys_of,
-                     &h->node_begin, &h->leaf_ids, &h->M, &h->L, &h->Lx, &h->pf, &h->pleaf, &h->dtab, &h->xtab, &h->far_src, &h->far_tgt, &h->row_node, &h->row_first,
+                     &h->node_begin, &h->leaf_ids, &h->M, &h->L, &h->Lx, &h->pf, &h->pleaf, &h->dtab, &h->xtab, &h->far_src, &h->far_tgt, &h->near_items, &h->near_k, &h->near_first,
+                     &h->near_part, &h->row_node, &h->row_first,
                      &h->row_next, &h->row_sl_start, &h->row_sl_cnt, &h->row_m_start, &h->row_m_cnt,
                      &h->row_mx_cnt, &h->row_p_start, &h->row_p_cnt, &h->m2l_pool, &h->p2p_pool, &h->sl, &h->counters, &h->diag,
                      &h->tmp_small, &h->Mw, &h->Lw, &h->pw, &h->wbuf, &h->gbuf, &h->mb, &h->mbw, &h->d2tab,
@@ -1760,6 +1805,7 @@ static int vjp_device(nbh_handle* h, const double* w_dev) {
     HIPCHK(h, h->pw.ensure(n * 16));
     HIPCHK(h, h->gbuf.ensure(n * 32));
     FmmParams F = h->lastF;
+    set_near(h, F);
     FmmParams Fw = F;
     Fw.M = h->Mw.as<float>();
     Fw.L = h->Lw.as<float>();
@@ -1770,7 +1816,9 @@ static int vjp_device(nbh_handle* h, const double* w_dev) {
     // the near field on the side stream, beside the transposed far-field chain
     HIPCHK(h, hipEventRecord(h->ev_fork, h->stream));
     HIPCHK(h, hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
-    launch_vjp_near(p, F, pw, (uint32_t)n, h->num_leaves, gdev, h->stream2);
+    // (with NBH_P2P_LEAF too: the kernel takes items, whichever P2P the forward pass runs)
+    launch_near_plan(F, h->num_leaves, h->stream2);
+    launch_vjp_near(p, F, pw, (uint32_t)n, near_grid_items(h, h->num_leaves, h->hc->p2p_total), gdev, h->stream2);
     HIPCHK(h, hipEventRecord(h->ev_near, h->stream2));
     M2LPlan plan = m2l_plan(h);
     if (plan.mfma) {
@@ -1989,7 +2037,7 @@ int nbh_debug_lists(nbh_handle* h, int64_t* m2l_off, int32_t* m2l_src, int64_t* 
         rows += h->hc->level_count[s] + h->hc->carried[s];
     rows = std::min<size_t>(rows, h->row_cap);
     std::vector<uint32_t> first(nn), next(rows), ms(rows), mc(rows), ps(rows), pc(rows);
-    std::vector<int32_t> mpool(h->hc->m2l_pool_used), ppool(h->hc->p2p_pool_used);
+    std::vector<int32_t> mpool(h->hc->m2l_pool_used.v), ppool(h->hc->p2p_pool_used.v);
     struct { void* dst; const void* src; size_t bytes; } cp[] = {
         {first.data(), h->row_first.p, nn * 4},     {next.data(), h->row_next.p, rows * 4},
         {ms.data(), h->row_m_start.p, rows * 4},    {mc.data(), h->row_m_cnt.p, rows * 4},

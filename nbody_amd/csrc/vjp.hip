@@ -18,6 +18,7 @@
 #include "common.h"
 #include "expansion.h"
 #include "launch.h"
+#include "near.h"
 
 namespace nbh {
 
@@ -59,8 +60,8 @@ __global__ __launch_bounds__(256) void dipole_p2m_kernel(FmmParams F, const floa
 
 // near field (pair VJP over the P2P lists) + far field (Hessian of the mass
 // local expansion, gradient and value of the dipole local expansion).  One
-// wavefront per target leaf, organised like the forward P2P kernel: the
-// leaf's P2P sources are flattened over its row segments, 64 at a time
+// wavefront per near-field item, organised like the forward P2P kernel: the
+// item's P2P sources are flattened over its batches, 64 at a time
 // staged in LDS (offset in the target leaf's frame, mass, cotangent), lanes
 // = (target particle) x (source stride), partial sums combined by shuffles.
 // As there, every lane runs the chunk's ceil(nchunk / splits) iterations and
@@ -69,7 +70,7 @@ constexpr int VJP_WAVES = 4;
 constexpr int VJP_STAGE = 96;  // splits * ceil(nchunk / splits) <= 84
 
 template <int P>
-__global__ __launch_bounds__(WAVE * VJP_WAVES) void vjp_staged_kernel(FmmParams F, const float4* pw, uint32_t num_leaves,
+__global__ __launch_bounds__(WAVE * VJP_WAVES) void vjp_staged_kernel(FmmParams F, const float4* pw,
                                                                       double* gx, double* gy, double* gz, double* gm) {
     __shared__ float4 stage_p[VJP_WAVES][VJP_STAGE];
     __shared__ float4 stage_w[VJP_WAVES][VJP_STAGE];
@@ -91,12 +92,16 @@ __global__ __launch_bounds__(WAVE * VJP_WAVES) void vjp_staged_kernel(FmmParams 
     }
     const uint32_t nw = gridDim.x * VJP_WAVES;
     const float eps2 = F.eps2;
-    for (uint32_t w = blockIdx.x * VJP_WAVES + wslot; w < num_leaves; w += nw) {
-        const int A = (int)F.leaf_ids[w];
+    const NearCount items = near_count(F);
+    for (uint32_t w = blockIdx.x * VJP_WAVES + wslot; w < items.cut + items.uncut; w += nw) {
+        const NearItem item = near_item(F, items, w);
+        if (item.b1 == 0) continue;
+        const int A = item.node;
+        const int t0 = (int)item.t0;
         const int4 ga = F.nodes.geo[A];
         const int4 la = F.nodes.link[A];
         const float unit = F.unit[F.nodes.sys[A]];
-        for (int t0 = 0; t0 < la.y; t0 += WAVE) {
+        {
             const int nt = min(WAVE, la.y - t0);
             const int splits = WAVE / nt;
             // ceil(x / splits) = umulhi(x + splits - 1, magic) for x <= 64
@@ -108,8 +113,7 @@ __global__ __launch_bounds__(WAVE * VJP_WAVES) void vjp_staged_kernel(FmmParams 
             const float4 wi = pw[i];
             const float mi = me.w;
             float g0 = 0.f, g1 = 0.f, g2 = 0.f, gmm = 0.f;
-            for (uint32_t r = F.lists.first[A]; r != NO_ROW; r = F.lists.next[r])
-            for (uint32_t eb = F.lists.p_start[r], e_end = eb + F.lists.p_cnt[r]; eb < e_end; eb += WAVE) {
+            near_batches(F.lists, A, item.b0, item.b1, [&](uint32_t eb, uint32_t e_end) {
                 const int ne = (int)min((uint32_t)WAVE, e_end - eb);
                 int cnt = 0, beg = 0;
                 float dx = 0.f, dy = 0.f, dz = 0.f;
@@ -188,7 +192,7 @@ __global__ __launch_bounds__(WAVE * VJP_WAVES) void vjp_staged_kernel(FmmParams 
                     }
                     wave_lds_sync();
                 }
-            }
+            });
             {
                 const float a0 = g0, a1 = g1, a2 = g2, a3 = gmm;
                 for (int q = 1; q < splits; ++q) {
@@ -201,10 +205,14 @@ __global__ __launch_bounds__(WAVE * VJP_WAVES) void vjp_staged_kernel(FmmParams 
             }
             if (sp == 0) {
                 // raw near-field sums (FP32 values); vjp_far_kernel adds the far field
-                gx[i] = g0;
-                gy[i] = g1;
-                gz[i] = g2;
-                gm[i] = gmm;
+                if (item.slot != NO_SLOT) {
+                    F.near_part[(size_t)item.slot * WAVE + ti] = make_float4(g0, g1, g2, gmm);
+                } else {
+                    gx[i] = g0;
+                    gy[i] = g1;
+                    gz[i] = g2;
+                    gm[i] = gmm;
+                }
             }
         }
     }
@@ -239,7 +247,9 @@ __global__ __launch_bounds__(256) void vjp_far_kernel(FmmParams F, const float4*
         for (int k = 0; k < NC; ++k) L[k] = Ls[k];
         l2p_eval<P>(me.x, me.y, me.z, L, psi, px, py, pz);
     }
-    float g0 = (float)gx[i], g1 = (float)gy[i], g2 = (float)gz[i], gmm = (float)gm[i];
+    float4 nr;
+    if (!near_partial_sum(F, A, i, nr)) nr = make_float4((float)gx[i], (float)gy[i], (float)gz[i], (float)gm[i]);
+    float g0 = nr.x, g1 = nr.y, g2 = nr.z, gmm = nr.w;
     g0 += mi * px + H[0] * wi.x + H[3] * wi.y + H[4] * wi.z;
     g1 += mi * py + H[3] * wi.x + H[1] * wi.y + H[5] * wi.z;
     g2 += mi * pz + H[4] * wi.x + H[5] * wi.y + H[2] * wi.z;
@@ -252,10 +262,10 @@ __global__ __launch_bounds__(256) void vjp_far_kernel(FmmParams F, const float4*
 }
 
 template <int P>
-static void launch_vjp_near_t(const FmmParams& F, const float4* pw, uint32_t n, uint32_t num_leaves, double* g,
+static void launch_vjp_near_t(const FmmParams& F, const float4* pw, uint32_t n, uint32_t grid_items, double* g,
                               hipStream_t st) {
-    const unsigned grid = std::min<unsigned>(ceil_div(num_leaves, VJP_WAVES), 65536u);
-    hipLaunchKernelGGL((vjp_staged_kernel<P>), dim3(grid), dim3(WAVE * VJP_WAVES), 0, st, F, pw, num_leaves, g, g + n,
+    const unsigned grid = std::max(1u, std::min<unsigned>(ceil_div(grid_items, VJP_WAVES), 65536u));
+    hipLaunchKernelGGL((vjp_staged_kernel<P>), dim3(grid), dim3(WAVE * VJP_WAVES), 0, st, F, pw, g, g + n,
                        g + 2 * (size_t)n, g + 3 * (size_t)n);
 }
 
@@ -327,9 +337,9 @@ void launch_fill_f64(double* p, size_t m, double v, hipStream_t st) {
 void launch_vjp_gather(const double* w_in, const uint32_t* id, float4* pw, uint32_t n, hipStream_t st) {
     hipLaunchKernelGGL(vjp_gather_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, st, w_in, id, pw, n);
 }
-void launch_vjp_near(int p, const FmmParams& F, const float4* pw, uint32_t n, uint32_t num_leaves, double* g,
+void launch_vjp_near(int p, const FmmParams& F, const float4* pw, uint32_t n, uint32_t grid_items, double* g,
                      hipStream_t st) {
-    NBH_VJP_DISPATCH(p, launch_vjp_near_t<PP>(F, pw, n, num_leaves, g, st));
+    NBH_VJP_DISPATCH(p, launch_vjp_near_t<PP>(F, pw, n, grid_items, g, st));
 }
 void launch_vjp_chain(int p, int q, const M2LPlan& plan, const FmmParams& F, const FmmParams& Fw, const float4* pw,
                       uint32_t num_leaves, const uint32_t* level_count, const uint32_t* level_off, int depth,

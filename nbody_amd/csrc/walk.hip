@@ -221,21 +221,21 @@ __global__ __launch_bounds__(64) void walk_root_kernel(WalkParams W) {
         W.row_mx_cnt[r] = 0;
         uint32_t pc = 0, ps = 0, sc = 0, ss = 0;
         if (leaf) {
-            ps = atomicAdd(&C->p2p_pool_used, 1u);
+            ps = atomicAdd(&C->p2p_pool_used.v, 1u);
             if (ps < W.p2p_pool_cap) {
                 W.p2p_pool[ps] = A;
                 pc = 1;
-                atomicAdd(&C->p2p_total, 1ull);
+                atomicAdd(&C->tot[0].p2p, 1ull);
             } else {
                 atomicOr(&C->overflow, (uint32_t)OVF_P2P);
                 ps = 0;
             }
         } else {
-            ss = atomicAdd(&C->sl_used, 1u);
+            ss = atomicAdd(&C->sl_used.v, 1u);
             if (ss < W.sl_cap) {
                 W.sl[ss] = A;
                 sc = 1;
-                atomicAdd(&C->split_total, 1ull);
+                atomicAdd(&C->tot[0].split, 1ull);
             } else {
                 atomicOr(&C->overflow, (uint32_t)OVF_SL);
                 ss = 0;
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
     __shared__ int cnode[SL_CACHE];
     __shared__ int cfc[SL_CACHE];
     __shared__ uint32_t cnt_s[WALK_WAVES][2][4][MAXT];  // [wave][phase][same-level, other-level, P2P, split][target]
-    __shared__ uint32_t bcast[8];                       // carried row, pool starts, failure
+    __shared__ uint32_t bcast[8];                       // pool starts, carried row, failure
     // pass 1's categories of a cached group, 3 bits per target, per call and lane
     __shared__ uint32_t cat_s[WALK_WAVES][CAT_CALLS][WAVE];
     Counters* C = W.C;
@@ -288,7 +288,13 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
     const int bits = W.bits;
     const uint64_t num4 = W.num4, den3 = W.den3;
     const uint32_t nblk = gridDim.x;
-    uint2 mchunk = make_uint2(0, 0), pchunk = make_uint2(0, 0), schunk = make_uint2(0, 0);  // thread 0 only
+    // lanes 0..2 of the first wavefront: the M2L, P2P and split pools
+    uint2 chunk = make_uint2(0, 0);
+    const uint32_t pool_chunk = lane == 0 ? POOL_CHUNK_M : lane == 1 ? POOL_CHUNK_P : POOL_CHUNK_S;
+    uint32_t* const pool_used = lane == 0   ? &C->m2l_pool_used.v
+                                : lane == 1 ? &C->p2p_pool_used.v
+                                            : &C->sl_used.v;
+    const unsigned long long pool_cap = lane == 0 ? W.m2l_pool_cap : lane == 1 ? W.p2p_pool_cap : W.sl_cap;
     unsigned long long acc_m = 0, acc_p = 0, acc_s = 0, acc_x = 0;                           // thread 0 only
     for (uint64_t j0 = 0; (uint64_t)blockIdx.x + j0 * nblk < n_groups; j0 += WAVE) {
         // headers of the next 64 rows of this workgroup (identical in every wavefront)
@@ -316,18 +322,15 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
             const uint32_t sl_n = __builtin_amdgcn_readlane(sn_l, jl);
             const int nch = gpw >> 8;
             __syncthreads();  // the previous group is done with the cache, counts and broadcasts
-            if (nch == 0 && threadIdx.x == 0) bcast[0] = atomicAdd(&C->carried[s], 1u);
-            __syncthreads();
             int nt, A0;
-            uint32_t row0;
+            uint32_t row0 = 0;
             if (nch > 0) {  // the cell's children: level-s rows in id order
                 nt = nch;
                 A0 = W.nodes.link[P].z;
                 row0 = base + (uint32_t)(A0 - (int)loff);
-            } else {  // a leaf with sources left to split: carried to depth s
+            } else {  // a leaf with sources left to split: carried to depth s (its row is taken below)
                 nt = 1;
                 A0 = P;
-                row0 = base + n_level + bcast[0];
             }
             if ((unsigned long long)row0 + nt > W.row_cap) {
                 // the host retries with more rows; rows that fit are left empty so
@@ -443,25 +446,32 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
                     }
             }
             const uint32_t tm = wave_sum(Tm + Tx), tp = wave_sum(Tp), ts = wave_sum(Ts), tx = wave_sum(Tx);
-            // reserve one block per pool for all targets of the group
-            if (threadIdx.x == 0) {
-                uint32_t ms0 = 0, ps0 = 0, ss0 = 0, fail = 0;
-                if (tm) {
-                    ms0 = pool_take(mchunk, tm, POOL_CHUNK_M, &C->m2l_pool_used, W.m2l_pool_cap);
-                    if (ms0 == 0xffffffffu) { atomicOr(&C->overflow, (uint32_t)OVF_M2L); fail = 1; }
+            // reserve one block per pool for all targets of the group (lanes
+            // 0..2 of the first wavefront, a pool each) and a carried leaf's row
+            // (lane 3): the atomics go out together
+            if (wv == 0) {
+                const uint32_t need = lane == 0 ? tm : lane == 1 ? tp : lane == 2 ? ts : 0u;
+                const uint32_t ovf = lane == 0 ? OVF_M2L : lane == 1 ? OVF_P2P : OVF_SL;
+                uint32_t at = 0;
+                if (need) {
+                    at = pool_take(chunk, need, pool_chunk, pool_used, pool_cap);
+                    if (at == 0xffffffffu) atomicOr(&C->overflow, ovf);
                 }
-                if (tp) {
-                    ps0 = pool_take(pchunk, tp, POOL_CHUNK_P, &C->p2p_pool_used, W.p2p_pool_cap);
-                    if (ps0 == 0xffffffffu) { atomicOr(&C->overflow, (uint32_t)OVF_P2P); fail = 1; }
+                if (lane == 3 && nch == 0) {
+                    at = base + n_level + atomicAdd(&C->carried[s], 1u);
+                    if (at >= W.row_cap) {  // (no row to leave empty)
+                        atomicOr(&C->overflow, (uint32_t)OVF_ROWS);
+                        at = 0xffffffffu;
+                    }
                 }
-                if (ts) {
-                    ss0 = pool_take(schunk, ts, POOL_CHUNK_S, &C->sl_used, W.sl_cap);
-                    if (ss0 == 0xffffffffu) { atomicOr(&C->overflow, (uint32_t)OVF_SL); fail = 1; }
-                }
-                if (!fail) { acc_m += tm; acc_p += tp; acc_s += ts; acc_x += tx; }
-                bcast[1] = ms0; bcast[2] = ps0; bcast[3] = ss0; bcast[4] = fail;
+                const bool fail = __ballot(lane < 4 && at == 0xffffffffu) != 0;
+                if (lane == 0 && !fail) { acc_m += tm; acc_p += tp; acc_s += ts; acc_x += tx; }
+                if (lane < 4) bcast[lane] = at;
+                if (lane == 4) bcast[4] = fail;
             }
             __syncthreads();
+            if (nch == 0) row0 = bcast[3];
+            if (row0 == 0xffffffffu) continue;  // uniform: no row left for the carried leaf
             const uint32_t fail = bcast[4];
             // segment starts of lane t's target: exclusive prefix over lanes
             // 0..7; a row's M2L segment holds its same-level sources, then the others
@@ -472,7 +482,7 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
                 const uint32_t ym = __shfl_up(em, o, WAVE), yp = __shfl_up(ep, o, WAVE), ys = __shfl_up(es, o, WAVE);
                 if (lane >= o) { em += ym; ep += yp; es += ys; }
             }
-            const uint32_t m0 = bcast[1] + em - nm_l, p0 = bcast[2] + ep - np_l, s0 = bcast[3] + es - ns_l;
+            const uint32_t m0 = bcast[0] + em - nm_l, p0 = bcast[1] + ep - np_l, s0 = bcast[2] + es - ns_l;
             if (wv == 0 && lane < nt) {
                 const uint32_t r = row0 + lane;
                 W.row_node[r] = A0 + lane;
@@ -529,10 +539,11 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
         }
     }
     if (threadIdx.x == 0) {
-        if (acc_m) atomicAdd(&C->m2l_total, acc_m);
-        if (acc_p) atomicAdd(&C->p2p_total, acc_p);
-        if (acc_s) atomicAdd(&C->split_total, acc_s);
-        if (acc_x) atomicAdd(&C->m2lx_total, acc_x);
+        LineTotals& tot = C->tot[blockIdx.x % CNT_COPIES];
+        if (acc_m) atomicAdd(&tot.m2l, acc_m);
+        if (acc_p) atomicAdd(&tot.p2p, acc_p);
+        if (acc_s) atomicAdd(&tot.split, acc_s);
+        if (acc_x) atomicAdd(&tot.m2lx, acc_x);
     }
 }
 
