@@ -1,0 +1,328 @@
+// direct.hip -- O(N^2) sums: the FP32 direct solver, the reference's naive
+// force law, and the FP64 sums that the force error is measured against.
+#include <algorithm>
+
+#include "common.h"
+#include "launch.h"
+
+namespace nbh {
+
+// ---------------------------------------------------------------------------
+// Direct sum on the GPU (replaces NaiveSimulation::step's O(N^2) loop,
+// naive_simulation.cpp:8-35), softened law: FP32 positions relative to the
+// system's box centre, packed once: x, y, z and charge in arrays of n + DS_PAD
+// (zeros past the particles).
+__global__ void direct_pack_kernel(State S, uint32_t n, const uint32_t* sys_off, int nsys, const double4* box,
+                                   float* pk) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t m = (size_t)n + DS_PAD;
+    if (i >= m) return;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < n) {
+        int lo = 0, hi = nsys - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (sys_off[mid] <= i) lo = mid; else hi = mid - 1;
+        }
+        const double4 bx = box[lo];
+        const double h = 0.5 * bx.w;
+        v = make_float4((float)(S.x[i] - (bx.x + h)), (float)(S.y[i] - (bx.y + h)), (float)(S.z[i] - (bx.z + h)),
+                        (float)S.charge[i]);
+    }
+    pk[i] = v.x;
+    pk[m + i] = v.y;
+    pk[2 * m + i] = v.z;
+    pk[3 * m + i] = v.w;
+}
+
+// One workgroup per 64 targets (one per lane).  Each target's force is one
+// FP32 sum over the sources in order, a serial chain: with a thread per target
+// doing all of a pair's work, N / 64 wavefronts share the GPU (256 on 1024
+// SIMDs at N = 16,384: 842 us a sum).  Here the chain holds only what has to
+// be in order: 13 producer wavefronts compute q / r^3 for 8 sources each of a
+// chunk of 104 into LDS while three consumers, one per component, add the
+// chunk before it: a subtraction and an FMA per source.  The sums are bit for
+// bit those of the one-thread chain.  Per source and 64 targets the producers
+// issue 14 slots (the rsq takes four) and the consumers 6: 150 us at N =
+// 16,384 if the four SIMDs of a CU never wait; measured 190 us.  (The sum cut
+// into 16 slices takes 129 us, but rounds differently.)  Sources are the same for every lane of
+// a wavefront and come through scalar loads.  The potential has no such order:
+// each producer keeps a partial sum.  NORMAL: eps^2 is a normal float, so that
+// v_rsq_f32 needs no denormal scaling (rsqrtf's).
+constexpr int DS_PROD = 13, DS_PER = 8, DS_CH = DS_PROD * DS_PER, DS_WAVES = DS_PROD + 3;
+static_assert(DS_PAD >= DS_CH, "a chunk past the particles reads the padding");
+template <bool NORMAL>
+__global__ __launch_bounds__(WAVE * DS_WAVES) void direct_f32_kernel(State S, const float* __restrict__ pk, uint32_t n,
+                                                                     const uint32_t* __restrict__ sys_off, float G,
+                                                                     float eps2, double kick_dt) {
+    __shared__ float4 w3s[2][DS_CH / 4][WAVE];  // q / r^3 of four sources
+    __shared__ float part[DS_PROD + 3][WAVE];
+    const uint32_t b = sys_off[blockIdx.y], e = sys_off[blockIdx.y + 1];
+    const uint32_t i0 = b + blockIdx.x * WAVE;
+    if (i0 >= e) return;
+    const int lane = lane_id();
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t i = i0 + lane, it = min(i, e - 1);
+    const size_t m = (size_t)n + DS_PAD;
+    const uint32_t nch = (e - b + DS_CH - 1) / DS_CH;
+    if (wv < 3) {  // consumers: component wv
+        const float* src = pk + wv * m + b;
+        const float me = pk[wv * m + it];
+        float acc = 0.f;
+        for (uint32_t c = 0; c <= nch; ++c) {
+            if (c > 0) {
+                const float* q = src + (size_t)(c - 1) * DS_CH;
+#pragma unroll 2
+                for (int g = 0; g < DS_CH / 4; ++g) {
+                    const float4 w = w3s[(c - 1) & 1][g][lane];
+                    acc = fmaf(q[4 * g] - me, w.x, acc);
+                    acc = fmaf(q[4 * g + 1] - me, w.y, acc);
+                    acc = fmaf(q[4 * g + 2] - me, w.z, acc);
+                    acc = fmaf(q[4 * g + 3] - me, w.w, acc);
+                }
+            }
+            __syncthreads();
+        }
+        part[DS_PROD + wv][lane] = acc;
+    } else {
+        const int pw = wv - 3;
+        const float px = pk[it], py = pk[m + it], pz = pk[2 * m + it];
+        float ph = 0.f;
+        for (uint32_t c = 0; c <= nch; ++c) {
+            if (c < nch) {
+                const uint32_t j0 = b + c * DS_CH + pw * DS_PER;  // uniform
+                const float *sx = pk + j0, *sy = sx + m, *sz = sy + m, *sq = sz + m;
+                float w3[DS_PER];
+                auto pairs = [&](auto&& skip) {
+#pragma unroll
+                    for (int k = 0; k < DS_PER; ++k) {
+                        const float rx = sx[k] - px, ry = sy[k] - py, rz = sz[k] - pz;
+                        const float r2 = fmaf(rx, rx, fmaf(ry, ry, fmaf(rz, rz, eps2)));
+                        const float inv = skip(k) ? 0.f : NORMAL ? __builtin_amdgcn_rsqf(r2) : rsqrtf(r2);
+                        const float w = sq[k] * inv;
+                        w3[k] = w * inv * inv;
+                        ph += w;
+                    }
+                };
+                // the self pair and the slots past the system's end contribute nothing
+                if (j0 + DS_PER <= e && (j0 + DS_PER <= i0 || j0 >= i0 + WAVE)) pairs([](int) { return false; });
+                else pairs([&](int k) { return j0 + k == i || j0 + k >= e; });
+#pragma unroll
+                for (int g = 0; g < DS_PER / 4; ++g)
+                    w3s[c & 1][pw * (DS_PER / 4) + g][lane] =
+                        make_float4(w3[4 * g], w3[4 * g + 1], w3[4 * g + 2], w3[4 * g + 3]);
+            }
+            __syncthreads();
+        }
+        part[pw][lane] = ph;
+    }
+    __syncthreads();
+    if (wv != 0 || i >= e) return;
+    float ph = 0.f;
+    for (int w = 0; w < DS_PROD; ++w) ph += part[w][lane];
+    const float fac = (float)(S.charge[i] / S.mass[i]) * G;
+    const float ax = fac * part[DS_PROD][lane], ay = fac * part[DS_PROD + 1][lane], az = fac * part[DS_PROD + 2][lane];
+    S.ax[i] = ax; S.ay[i] = ay; S.az[i] = az;
+    S.pot[i] = -G * ph;
+    if (kick_dt != 0.0) {
+        S.vx[i] += (double)ax * kick_dt;
+        S.vy[i] += (double)ay * kick_dt;
+        S.vz[i] += (double)az * kick_dt;
+    }
+}
+
+// The reference's naive force law (compat): separation (dx, dx, dx), no
+// softening (naive_simulation.cpp:10-17), with each pair's term formed as the
+// reference forms it in FP32 (uncentred x difference, r = sqrt(d d + d d +
+// d d), force = (k q_i q_j) d / (r r r), divided by m_i; no contraction into
+// FMAs) and summed in FP64, so one evaluation differs from the reference only
+// by its FP32 summation order.  One thread per target, source tiles in LDS.
+constexpr int DC_THREADS = 256;
+__global__ __launch_bounds__(DC_THREADS) void direct_compat_kernel(State S, const uint32_t* sys_off, float G,
+                                                                   double kick_dt) {
+    __shared__ float2 tile[DC_THREADS];  // x, charge
+    const int s = blockIdx.y;
+    const uint32_t b = sys_off[s], e = sys_off[s + 1];
+    const uint32_t i = b + blockIdx.x * DC_THREADS + threadIdx.x;
+    if (b + blockIdx.x * DC_THREADS >= e) return;
+    const bool valid = i < e;
+    const float px = valid ? (float)S.x[i] : 0.f;
+    float ph = 0;
+    double acd = 0.0;  // sum of the reference's per-pair kicks / dt
+    const float qi = valid ? (float)S.charge[i] : 0.f, mi = valid ? (float)S.mass[i] : 1.f;
+    for (uint32_t j0 = b; j0 < e; j0 += DC_THREADS) {
+        const uint32_t j = j0 + threadIdx.x;
+        __syncthreads();
+        tile[threadIdx.x] = j < e ? make_float2((float)S.x[j], (float)S.charge[j]) : make_float2(0, 0);
+        __syncthreads();
+        const uint32_t jn = min((uint32_t)DC_THREADS, e - j0);
+        if (!valid) continue;
+        for (uint32_t k = 0; k < jn; ++k) {
+            // IEEE single operations in the reference's order: no FMA
+            // contraction; sqrtf and '/' are correctly rounded in HIP
+#pragma clang fp contract(off)
+            if (j0 + k == i) continue;
+            const float2 q = tile[k];
+            const float d = q.x - px;
+            const float r = sqrtf(d * d + d * d + d * d);
+            const float f = G * (qi * q.y) * d / (r * r * r);
+            acd += (double)(f / mi);
+            ph += q.y / r;
+        }
+    }
+    if (!valid) return;
+    const float a = (float)acd;
+    S.ax[i] = a; S.ay[i] = a; S.az[i] = a;
+    S.pot[i] = -G * ph;
+    if (kick_dt != 0.0) {
+        S.vx[i] += (double)a * kick_dt;
+        S.vy[i] += (double)a * kick_dt;
+        S.vz[i] += (double)a * kick_dt;
+    }
+}
+
+void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uint32_t* sys_off, int nsys,
+                       const double4* box, float G, float eps2, int compat_law, double kick_dt, float* pk,
+                       hipStream_t st) {
+    if (compat_law) {
+        hipLaunchKernelGGL(direct_compat_kernel, dim3(ceil_div(max_sys_n, DC_THREADS), nsys), dim3(DC_THREADS), 0, st,
+                           S, sys_off, G, kick_dt);
+        return;
+    }
+    hipLaunchKernelGGL(direct_pack_kernel, dim3(ceil_div(n + DS_PAD, 256)), dim3(256), 0, st, S, n, sys_off, nsys, box,
+                       pk);
+    const dim3 grid(ceil_div(max_sys_n, WAVE), nsys), block(WAVE * DS_WAVES);
+    if (eps2 >= 1.17549435e-38f)
+        hipLaunchKernelGGL(direct_f32_kernel<true>, grid, block, 0, st, S, pk, n, sys_off, G, eps2, kick_dt);
+    else
+        hipLaunchKernelGGL(direct_f32_kernel<false>, grid, block, 0, st, S, pk, n, sys_off, G, eps2, kick_dt);
+}
+
+// ---------------------------------------------------------------------------
+// FP64 direct sum for selected targets (sorted slots).  A workgroup takes T
+// targets; its 8 wavefronts stride over the sources with one source per lane,
+// so each source is loaded once for T targets (one target per wavefront read
+// 32 bytes per pair from L2, 12 TB/s at 262,144 sources x 4096 targets, which
+// bound it).  1/r is v_rsq_f64 (relative error e/2 ~ 2^-27) and one third-order
+// step y (1 + e/2 + 3/8 e^2), e = 1 - r^2 y^2, whose remainder ~e^3 is below
+// the rounding; 1/sqrt took ~50 instructions of the pair's ~70.  262,144 x
+// 4096: 2.7 -> 1.0 ms, of 0.68 ms that the pairs' FP64 instructions take.
+constexpr int DD_WAVES = 8;
+template <int T>
+__global__ __launch_bounds__(WAVE * DD_WAVES) void direct_fp64_kernel(State S, const uint32_t* __restrict__ sys_off,
+                                                                      int nsys, const uint32_t* __restrict__ targets,
+                                                                      uint32_t nt, double G, double eps2, double* acc,
+                                                                      double* pot) {
+    __shared__ double part[DD_WAVES][T][4];
+    const uint32_t w0 = blockIdx.x * T;
+    const uint32_t n = sys_off[nsys];
+    const uint32_t wv = threadIdx.x / WAVE;
+    const int lane = lane_id();
+    uint32_t id[T];
+    double px[T], py[T], pz[T], a[T][4];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        // (no such particle, or past the last target: the sums are dropped)
+        const uint32_t i = targets[min(w0 + t, nt - 1)];
+        id[t] = i;
+        const uint32_t k = i < n ? i : 0u;
+        px[t] = S.x[k]; py[t] = S.y[k]; pz[t] = S.z[k];
+        a[t][0] = a[t][1] = a[t][2] = a[t][3] = 0.0;
+    }
+    // T > 1: one system (the launcher's rule)
+    uint32_t b = 0, e = n;
+    if (T == 1 && nsys > 1) {
+        int lo = 0, hi = nsys - 1;
+        while (lo < hi) { int mid = (lo + hi + 1) >> 1; if (sys_off[mid] <= id[0]) lo = mid; else hi = mid - 1; }
+        b = sys_off[lo];
+        e = sys_off[lo + 1];
+    }
+    for (uint32_t j = b + wv * WAVE + lane; j < e; j += WAVE * DD_WAVES) {
+        const double sx = S.x[j], sy = S.y[j], sz = S.z[j], q = S.charge[j];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const double rx = sx - px[t], ry = sy - py[t], rz = sz - pz[t];
+            const double r2 = rx * rx + ry * ry + rz * rz + eps2;
+            const double y = __builtin_amdgcn_rsq(r2);
+            const double err = fma(-r2 * y, y, 1.0);
+            const double yn = fma(y * err, fma(0.375, err, 0.5), y);
+            // (r2 = 0 or infinite: err is NaN, and y is the limit)
+            const double inv = fabs(err) < 1.0 ? yn : y;
+            const double w = j == id[t] ? 0.0 : q * inv;
+            const double w3 = j == id[t] ? 0.0 : w * inv * inv;
+            a[t][0] = fma(rx, w3, a[t][0]);
+            a[t][1] = fma(ry, w3, a[t][1]);
+            a[t][2] = fma(rz, w3, a[t][2]);
+            a[t][3] += w;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double v = wave_sum(a[t][k]);
+            if (lane == 0) part[wv][t][k] = v;
+        }
+    __syncthreads();
+    if (threadIdx.x < 4 * T) {
+        const int t = threadIdx.x / 4, k = threadIdx.x % 4;
+        const uint32_t w = w0 + t;
+        if (w >= nt) return;
+        const uint32_t i = targets[w];
+        double v = 0.0;
+        for (int q = 0; q < DD_WAVES; ++q) v += part[q][t][k];
+        // no such particle: report NaN
+        if (k < 3) acc[3 * (size_t)w + k] = i < n ? S.charge[i] / S.mass[i] * G * v : NAN;
+        else pot[w] = i < n ? -G * v : NAN;
+    }
+}
+
+void launch_direct_fp64(const State& S, const uint32_t* sys_off, int nsys, const uint32_t* targets, uint32_t nt,
+                        double G, double eps2, double* acc, double* pot, hipStream_t st) {
+    if (!nt) return;
+    // eight targets a workgroup where that still leaves two workgroups per
+    // CU; of several systems each target has its own sources
+    if (nsys == 1 && nt >= 4096)
+        hipLaunchKernelGGL(direct_fp64_kernel<8>, dim3(ceil_div(nt, 8)), dim3(WAVE * DD_WAVES), 0, st, S, sys_off,
+                           nsys, targets, nt, G, eps2, acc, pot);
+    else if (nsys == 1 && nt >= 1024)
+        hipLaunchKernelGGL(direct_fp64_kernel<4>, dim3(ceil_div(nt, 4)), dim3(WAVE * DD_WAVES), 0, st, S, sys_off,
+                           nsys, targets, nt, G, eps2, acc, pot);
+    else
+        hipLaunchKernelGGL(direct_fp64_kernel<1>, dim3(nt), dim3(WAVE * DD_WAVES), 0, st, S, sys_off, nsys, targets,
+                           nt, G, eps2, acc, pot);
+}
+
+// slots[k] = slot_of[targets[k]] (targets checked by the host)
+__global__ void map_slots_kernel(const uint32_t* slot_of, const int64_t* targets, uint32_t nt, uint32_t* slots) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nt) slots[k] = slot_of[targets[k]];
+}
+void launch_map_slots(const uint32_t* slot_of, const int64_t* targets, uint32_t nt, uint32_t* slots, hipStream_t st) {
+    hipLaunchKernelGGL(map_slots_kernel, dim3(ceil_div(nt, 256)), dim3(256), 0, st, slot_of, targets, nt, slots);
+}
+
+// Sorted slot of each target given in input order, by a scan of the id array
+// (one wavefront per target; an id array is a permutation, so every index in
+// [0, n) is found once; anything else gets 0xffffffff).  Costs a read of the
+// ids per target, an eighth of what the FP64 sum then reads per target.
+__global__ __launch_bounds__(256) void find_slots_kernel(const uint32_t* __restrict__ id, uint32_t n,
+                                                         const int64_t* __restrict__ targets, uint32_t nt,
+                                                         uint32_t* slots) {
+    const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+    if (w >= nt) return;
+    const int64_t t = targets[w];
+    uint32_t found = 0xffffffffu;
+    for (uint32_t j0 = 0; j0 < n && found == 0xffffffffu; j0 += WAVE) {
+        const uint32_t j = j0 + lane_id();
+        const uint64_t hit = __ballot(j < n && (int64_t)id[j] == t);
+        if (hit) found = j0 + (uint32_t)__ffsll((unsigned long long)hit) - 1;
+    }
+    if (lane_id() == 0) slots[w] = found;
+}
+void launch_find_slots(const uint32_t* id, uint32_t n, const int64_t* targets, uint32_t nt, uint32_t* slots,
+                       hipStream_t st) {
+    hipLaunchKernelGGL(find_slots_kernel, dim3(ceil_div(nt, 4)), dim3(256), 0, st, id, n, targets, nt, slots);
+}
+
+}  // namespace nbh

@@ -1349,170 +1349,6 @@ void launch_integrate(const State& S, uint32_t n, int mode, double dt_k, double 
 }
 
 // ---------------------------------------------------------------------------
-// Direct sum on the GPU (replaces NaiveSimulation::step's O(N^2) loop,
-// naive_simulation.cpp:8-35).  Source tiles staged in LDS; FP32 positions
-// relative to the system's box centre.  compat_law reproduces the reference
-// naive force law: separation (dx, dx, dx), no softening (:10-17), with each
-// pair's term formed as the reference forms it in FP32 (uncentred x
-// difference, r = sqrt(d d + d d + d d), force = (k q_i q_j) d / (r r r),
-// divided by m_i; no contraction into FMAs) and summed in FP64, so one
-// evaluation differs from the reference only by its FP32 summation order.
-constexpr int DS_THREADS = 256;
-
-__global__ __launch_bounds__(DS_THREADS) void direct_f32_kernel(State S, uint32_t n, const uint32_t* sys_off,
-                                                                int nsys, const double4* box, float G, float eps2,
-                                                                int compat, double kick_dt) {
-    __shared__ float4 tile[DS_THREADS];
-    const int s = blockIdx.y;
-    const uint32_t b = sys_off[s], e = sys_off[s + 1];
-    const uint32_t i = b + blockIdx.x * DS_THREADS + threadIdx.x;
-    if (b + blockIdx.x * DS_THREADS >= e) return;
-    const double4 bx = box[s];
-    const double h = 0.5 * bx.w;
-    // compat: absolute FP32 coordinates, as the reference holds them
-    const double cx = compat ? 0.0 : bx.x + h, cy = compat ? 0.0 : bx.y + h, cz = compat ? 0.0 : bx.z + h;
-    const bool valid = i < e;
-    float px = 0, py = 0, pz = 0;
-    if (valid) { px = (float)(S.x[i] - cx); py = (float)(S.y[i] - cy); pz = (float)(S.z[i] - cz); }
-    float ax = 0, ay = 0, az = 0, ph = 0;
-    double acd = 0.0;  // compat: sum of the reference's per-pair kicks / dt
-    const float qi = valid ? (float)S.charge[i] : 0.f, mi = valid ? (float)S.mass[i] : 1.f;
-    for (uint32_t j0 = b; j0 < e; j0 += DS_THREADS) {
-        const uint32_t j = j0 + threadIdx.x;
-        __syncthreads();
-        tile[threadIdx.x] = j < e ? make_float4((float)(S.x[j] - cx), (float)(S.y[j] - cy), (float)(S.z[j] - cz),
-                                                (float)S.charge[j])
-                                  : make_float4(0, 0, 0, 0);
-        __syncthreads();
-        const uint32_t jn = min((uint32_t)DS_THREADS, e - j0);
-        if (!valid) continue;
-        if (!compat) {
-            for (uint32_t k = 0; k < jn; ++k) {
-                const float4 q = tile[k];
-                const float rx = q.x - px, ry = q.y - py, rz = q.z - pz;
-                const float r2 = fmaf(rx, rx, fmaf(ry, ry, fmaf(rz, rz, eps2)));
-                // the self pair contributes nothing (r2 = 0 when unsoftened)
-                const float inv = (j0 + k == i) ? 0.f : rsqrtf(r2);
-                const float w = q.w * inv;
-                const float w3 = w * inv * inv;
-                ax = fmaf(rx, w3, ax); ay = fmaf(ry, w3, ay); az = fmaf(rz, w3, az);
-                ph += w;
-            }
-        } else {
-            for (uint32_t k = 0; k < jn; ++k) {
-                // IEEE single operations in the reference's order: no FMA
-                // contraction; sqrtf and '/' are correctly rounded in HIP
-#pragma clang fp contract(off)
-                if (j0 + k == i) continue;
-                const float4 q = tile[k];
-                const float d = q.x - px;
-                const float r = sqrtf(d * d + d * d + d * d);
-                const float f = G * (qi * q.w) * d / (r * r * r);
-                acd += (double)(f / mi);
-                ph += q.w / r;
-            }
-        }
-    }
-    if (!valid) return;
-    if (compat) {
-        const float a = (float)acd;
-        S.ax[i] = a; S.ay[i] = a; S.az[i] = a;
-        S.pot[i] = -G * ph;
-        if (kick_dt != 0.0) {
-            S.vx[i] += (double)a * kick_dt;
-            S.vy[i] += (double)a * kick_dt;
-            S.vz[i] += (double)a * kick_dt;
-        }
-        return;
-    }
-    const float fac = (float)(S.charge[i] / S.mass[i]) * G;
-    S.ax[i] = fac * ax; S.ay[i] = fac * ay; S.az[i] = fac * az;
-    S.pot[i] = -G * ph;
-    if (kick_dt != 0.0) {
-        S.vx[i] += (double)(fac * ax) * kick_dt;
-        S.vy[i] += (double)(fac * ay) * kick_dt;
-        S.vz[i] += (double)(fac * az) * kick_dt;
-    }
-}
-
-void launch_direct_f32(const State& S, uint32_t n, const uint32_t* sys_off, int nsys, const double4* box, float G,
-                       float eps2, int compat_law, double kick_dt, hipStream_t st) {
-    // grid.x sized for the largest system: callers pass n = max system size
-    hipLaunchKernelGGL(direct_f32_kernel, dim3(ceil_div(n, DS_THREADS), nsys), dim3(DS_THREADS), 0, st, S, n, sys_off,
-                       nsys, box, G, eps2, compat_law, kick_dt);
-}
-
-// FP64 direct sum for selected targets (sorted slots): one wavefront per target.
-__global__ __launch_bounds__(256) void direct_fp64_kernel(State S, const uint32_t* sys_off, int nsys,
-                                                          const uint32_t* targets, uint32_t nt, double G,
-                                                          double eps2, double* acc, double* pot) {
-    const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    if (w >= nt) return;
-    const uint32_t i = targets[w];
-    if (i >= sys_off[nsys]) {  // no such particle: report NaN rather than read out of bounds
-        if (lane_id() == 0) {
-            acc[3 * w] = acc[3 * w + 1] = acc[3 * w + 2] = NAN;
-            pot[w] = NAN;
-        }
-        return;
-    }
-    int s = 0;
-    {
-        int lo = 0, hi = nsys - 1;
-        while (lo < hi) { int mid = (lo + hi + 1) >> 1; if (sys_off[mid] <= i) lo = mid; else hi = mid - 1; }
-        s = lo;
-    }
-    const uint32_t b = sys_off[s], e = sys_off[s + 1];
-    const double px = S.x[i], py = S.y[i], pz = S.z[i];
-    double ax = 0, ay = 0, az = 0, ph = 0;
-    for (uint32_t j = b + lane_id(); j < e; j += WAVE) {
-        if (j == i) continue;
-        const double rx = S.x[j] - px, ry = S.y[j] - py, rz = S.z[j] - pz;
-        const double r2 = rx * rx + ry * ry + rz * rz + eps2;
-        const double inv = 1.0 / sqrt(r2);
-        const double q = S.charge[j] * inv;
-        const double q3 = q * inv * inv;
-        ax += rx * q3; ay += ry * q3; az += rz * q3;
-        ph += q;
-    }
-    ax = wave_sum(ax); ay = wave_sum(ay); az = wave_sum(az); ph = wave_sum(ph);
-    if (lane_id() == 0) {
-        const double fac = S.charge[i] / S.mass[i] * G;
-        acc[3 * w] = fac * ax; acc[3 * w + 1] = fac * ay; acc[3 * w + 2] = fac * az;
-        pot[w] = -G * ph;
-    }
-}
-
-void launch_direct_fp64(const State& S, const uint32_t* sys_off, int nsys, const uint32_t* targets, uint32_t nt,
-                        double G, double eps2, double* acc, double* pot, hipStream_t st) {
-    hipLaunchKernelGGL(direct_fp64_kernel, dim3(ceil_div(nt, 4)), dim3(256), 0, st, S, sys_off, nsys, targets, nt, G,
-                       eps2, acc, pot);
-}
-
-// Sorted slot of each target given in input order, by a scan of the id array
-// (one wavefront per target; an id array is a permutation, so every index in
-// [0, n) is found once; anything else gets 0xffffffff).  Costs a read of the
-// ids per target, an eighth of what the FP64 sum then reads per target.
-__global__ __launch_bounds__(256) void find_slots_kernel(const uint32_t* __restrict__ id, uint32_t n,
-                                                         const int64_t* __restrict__ targets, uint32_t nt,
-                                                         uint32_t* slots) {
-    const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    if (w >= nt) return;
-    const int64_t t = targets[w];
-    uint32_t found = 0xffffffffu;
-    for (uint32_t j0 = 0; j0 < n && found == 0xffffffffu; j0 += WAVE) {
-        const uint32_t j = j0 + lane_id();
-        const uint64_t hit = __ballot(j < n && (int64_t)id[j] == t);
-        if (hit) found = j0 + (uint32_t)__ffsll((unsigned long long)hit) - 1;
-    }
-    if (lane_id() == 0) slots[w] = found;
-}
-void launch_find_slots(const uint32_t* id, uint32_t n, const int64_t* targets, uint32_t nt, uint32_t* slots,
-                       hipStream_t st) {
-    hipLaunchKernelGGL(find_slots_kernel, dim3(ceil_div(nt, 4)), dim3(256), 0, st, id, n, targets, nt, slots);
-}
-
-// ---------------------------------------------------------------------------
 // Diagnostics partials per block: KE, PE, P[3], Lang[3]
 constexpr int DG_THREADS = 256;
 uint32_t diagnostics_blocks(uint32_t n) { return min(1024u, ceil_div(n, DG_THREADS)); }

@@ -132,6 +132,7 @@ struct nbh_handle {
     // (forward and adjoint), dense tensor tables, candidate offsets
     DevBuf mb, mbw, d2tab, cand, hank, opar;
     DevBuf sl_offs, sl_map;  // same-level table: offsets that occur (rows), offset -> row map
+    DevBuf slot_of, direct_buf;  // nbh_direct_fp64
     DevBuf acc_save;         // nbh_diagnostics: the accelerations kept across its evaluation
     int sl_rows = 0;         // rows of the same-level table per level, its zero row included
     // trajectory adjoint: checkpoints of the full state (every adj_k steps),
@@ -913,8 +914,8 @@ static int force_direct(nbh_handle* h, double kick_dt) {
     launch_bbox(S.x, S.y, S.z, h->sys_off.as<uint32_t>(), h->nsys, h->max_sys_n, h->bits, (int)h->cfg.fixed_root,
                 h->cfg.root_lo, h->cfg.root_size, h->bbox_part.as<double>(), h->box.as<double4>(),
                 h->inv.as<double>(), h->unit.as<float>(), &dC->nonfinite, h->stream);
-    launch_direct_f32(S, h->max_sys_n, h->sys_off.as<uint32_t>(), h->nsys, h->box.as<double4>(), (float)h->cfg.G,
-                      (float)(h->cfg.eps * h->cfg.eps), (int)h->cfg.force_law, kick_dt, h->stream);
+    launch_direct_f32(S, (uint32_t)h->n, h->max_sys_n, h->sys_off.as<uint32_t>(), h->nsys, h->box.as<double4>(), (float)h->cfg.G,
+                      (float)(h->cfg.eps * h->cfg.eps), (int)h->cfg.force_law, kick_dt, h->pf.as<float>(), h->stream);
     HIPCHK(h, hipGetLastError());
     CHK(read_counters(h));
     if (h->hc->nonfinite) return h->fail(NBH_E_NONFINITE, "non-finite particle position");
@@ -1292,7 +1293,7 @@ static int create_impl(const nbh_config* cfg, size_t nsys, const uint32_t* sys_o
     CCHK(h->unit.ensure(nsys * 4));
     CCHK(h->bbox_part.ensure(nsys * (size_t)ceil_div(h->max_sys_n, 4096) * 6 * 8 + 64));
     CCHK(h->leaf_ids.ensure(n * 4));
-    CCHK(h->pf.ensure(n * 16));
+    CCHK(h->pf.ensure((n + DS_PAD) * 16));
     CCHK(h->pleaf.ensure(n * 4));
     CCHK(h->counters.ensure(sizeof(Counters)));
     CCHK(h->diag.ensure(1024 * 8 * 8));
@@ -1452,7 +1453,7 @@ void nbh_destroy(nbh_handle* h) {
                      &h->row_next, &h->row_sl_start, &h->row_sl_cnt, &h->row_m_start, &h->row_m_cnt,
                      &h->row_mx_cnt, &h->row_p_start, &h->row_p_cnt, &h->m2l_pool, &h->p2p_pool, &h->sl, &h->counters, &h->diag,
                      &h->tmp_small, &h->Mw, &h->Lw, &h->pw, &h->wbuf, &h->gbuf, &h->mb, &h->mbw, &h->d2tab,
-                     &h->cand, &h->hank, &h->opar, &h->sl_offs, &h->sl_map, &h->acc_save};
+                     &h->cand, &h->hank, &h->opar, &h->sl_offs, &h->sl_map, &h->acc_save, &h->slot_of, &h->direct_buf};
     for (DevBuf* b : all) b->release();
     for (DevBuf& b : h->adj_ckpt) b.release();
     for (DevBuf& b : h->adj_seg) b.release();
@@ -1636,27 +1637,24 @@ int nbh_direct_fp64(nbh_handle* h, size_t nt, const int64_t* targets, double* ac
     const size_t n = h->n;
     if (!nt) return NBH_OK;
     State S = h->st[h->cur].view();
-    std::vector<uint32_t> ids(n), slot(n), tg(nt);
-    HIPCHK(h, hipMemcpyAsync(ids.data(), S.id, n * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (size_t i = 0; i < n; ++i) slot[ids[i]] = (uint32_t)i;
-    for (size_t k = 0; k < nt; ++k) {
+    for (size_t k = 0; k < nt; ++k)
         if (targets[k] < 0 || (size_t)targets[k] >= n) return h->fail(NBH_E_INVALID, "target index out of range");
-        tg[k] = slot[targets[k]];
-    }
-    // the box is needed only by direct_f32; fp64 uses raw positions
-    DevBuf dt, da, dp;
-    HIPCHK(h, dt.ensure(nt * 4));
-    HIPCHK(h, da.ensure(nt * 24));
-    HIPCHK(h, dp.ensure(nt * 8));
-    HIPCHK(h, hipMemcpyAsync(dt.p, tg.data(), nt * 4, hipMemcpyHostToDevice, h->stream));
-    launch_direct_fp64(S, h->sys_off.as<uint32_t>(), h->nsys, dt.as<uint32_t>(), (uint32_t)nt, h->cfg.G,
-                       h->cfg.eps * h->cfg.eps, da.as<double>(), dp.as<double>(), h->stream);
+    // targets, their sorted slots and the results: scratch kept by the handle
+    HIPCHK(h, h->slot_of.ensure(n * 4));
+    HIPCHK(h, h->direct_buf.ensure(nt * (8 + 24 + 8 + 4)));
+    int64_t* dtg = h->direct_buf.as<int64_t>();
+    double* dacc = (double*)(dtg + nt);
+    double* dpot = dacc + 3 * nt;
+    uint32_t* dslot = (uint32_t*)(dpot + nt);
+    HIPCHK(h, hipMemcpyAsync(dtg, targets, nt * 8, hipMemcpyHostToDevice, h->stream));
+    launch_inverse_perm(S.id, h->slot_of.as<uint32_t>(), (uint32_t)n, h->stream);
+    launch_map_slots(h->slot_of.as<uint32_t>(), dtg, (uint32_t)nt, dslot, h->stream);
+    launch_direct_fp64(S, h->sys_off.as<uint32_t>(), h->nsys, dslot, (uint32_t)nt, h->cfg.G,
+                       h->cfg.eps * h->cfg.eps, dacc, dpot, h->stream);
     HIPCHK(h, hipGetLastError());
-    HIPCHK(h, hipMemcpyAsync(acc, da.p, nt * 24, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(pot, dp.p, nt * 8, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipMemcpyAsync(acc, dacc, nt * 24, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipMemcpyAsync(pot, dpot, nt * 8, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    dt.release(); da.release(); dp.release();
     return NBH_OK;
 }
 

@@ -1,0 +1,85 @@
+"""The direct sums (FP32 solver, FP64 check) against numpy in 64 bits, at the
+edges of their 64-target workgroups, source slices and targets per workgroup."""
+import numpy as np
+import pytest
+
+import nbody_amd as nb
+
+pytestmark = pytest.mark.gpu
+
+
+def _sum64(x, m, eps, targets):
+    acc, pot = np.zeros((len(targets), 3)), np.zeros(len(targets))
+    for k, i in enumerate(targets):
+        d = x - x[i]
+        r2 = (d * d).sum(1) + eps * eps
+        r2[i] = 1.0
+        w = m / np.sqrt(r2)
+        w[i] = 0.0
+        acc[k] = ((w / r2)[:, None] * d).sum(0)
+        pot[k] = -w.sum()
+    return acc, pot
+
+
+def _packed(x):
+    """The positions that the FP32 solver sums over: FP32 offsets from the
+    centre of the system's bounding cube."""
+    lo = x.min(0)
+    size = (x.max(0) - lo).max()
+    return (x - (lo + 0.5 * (size if size > 0 else 1.0))).astype(np.float32).astype(np.float64)
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 63, 64, 65, 129, 1000, 4097])
+@pytest.mark.parametrize("eps", [1e-2, 0.0])
+def test_direct_solver(n, eps):
+    x, v, m = nb.ics.plummer(n, 3)
+    cfg = nb.default_config(solver=nb.SOLVER_DIRECT, eps=eps)
+    with nb.HipSimulation.from_arrays(x, v, m, m, config=cfg) as sim:
+        acc, pot = sim.forces()
+    t = np.arange(0, n, max(1, n // 97))
+    ar, pr = _sum64(_packed(x), m, eps, t)
+    # FP32 terms and sums of up to n of them
+    tol = 2e-5
+    scale = np.sqrt((ar * ar).sum(1).mean()) + 1e-30
+    assert np.max(np.abs(acc[t] - ar)) <= tol * max(scale, np.abs(ar).max()) + 1e-30
+    assert np.max(np.abs(pot[t] - pr)) <= tol * np.abs(pr).max() + 1e-30
+
+
+def test_direct_solver_ensemble():
+    x, v, m, off = nb.ics.ensemble(5, nmin=30, nmax=700)
+    cfg = nb.default_config(solver=nb.SOLVER_DIRECT, eps=1e-2)
+    with nb.HipSimulation.from_arrays(x, v, m, m, config=cfg, sys_off=off) as sim:
+        acc, _ = sim.forces()
+    for a, b in zip(off[:-1], off[1:]):
+        t = np.arange(a, b, 11)
+        ar, _ = _sum64(_packed(x[a:b]), m[a:b], 1e-2, t - a)
+        assert np.max(np.abs(acc[t] - ar)) <= 2e-5 * np.abs(ar).max()
+
+
+@pytest.mark.parametrize("n,nt", [(1, 1), (2, 2), (500, 3), (511, 511), (1500, 1031), (5003, 4096), (5003, 4099)])
+@pytest.mark.parametrize("eps", [1e-3, 0.0])
+def test_fp64_sums(n, nt, eps):
+    x, v, m = nb.ics.plummer(n, 5)
+    t = np.random.default_rng(n).permutation(n)[:nt]
+    with nb.HipSimulation.from_arrays(x, v, m, m, config=nb.default_config(eps=eps)) as sim:
+        sim.step(1)
+        x = sim.positions()
+        acc, pot = sim.direct_fp64(t)
+        acc2, pot2 = sim.direct_fp64_noalloc(t)
+    assert np.array_equal(acc, acc2) and np.array_equal(pot, pot2)
+    s = np.arange(0, nt, max(1, nt // 97))
+    ar, pr = _sum64(x, m, eps, t[s])
+    # 64-bit sums of up to n terms, each to a few ulps
+    assert np.max(np.abs(acc[s] - ar)) <= 1e-13 * np.abs(ar).max() + 1e-300
+    assert np.max(np.abs(pot[s] - pr)) <= 1e-13 * np.abs(pr).max() + 1e-300
+
+
+def test_fp64_sums_of_coincident_particles():
+    # distinct particles at one point, unsoftened: no finite potential; far away ones: no force
+    x = np.array([[0.0, 0, 0], [0, 0, 0], [1, 0, 0], [1e160, 0, 0]])
+    m = np.ones(4)
+    with nb.HipSimulation.from_arrays(x, np.zeros_like(x), m, m, config=nb.default_config(eps=0.0)) as sim:
+        acc, pot = sim.direct_fp64([0, 2, 3])
+    assert pot[0] == -np.inf and np.isnan(acc[0]).any()
+    assert acc[1][0] == -2.0 and pot[1] == -2.0
+    assert np.all(acc[2] == 0.0) and pot[2] == 0.0
