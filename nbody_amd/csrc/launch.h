@@ -284,6 +284,16 @@ void launch_vjp_chain(int p, int q, const M2LPlan& plan, const FmmParams& F, con
 void launch_vjp_far(int p, const FmmParams& F, const FmmParams& Fw, const float4* pw, uint32_t n, double* g,
                     hipStream_t st);
 
+// sorted state <-> the caller's input order (io.hip)
+void launch_pack_state(const State& S, uint32_t n, double* pos, double* vel, double* mass, double* charge,
+                       hipStream_t st);
+void launch_pack_forces(const State& S, uint32_t n, float* acc, float* pot, hipStream_t st);
+void launch_pack_gradient(const double* g, const uint32_t* id, uint32_t n, double* gx, double* gm, hipStream_t st);
+void launch_init_state(const State& dst, uint32_t n, const double* pos, const double* vel, const double* mass,
+                       const double* charge, hipStream_t st);
+void launch_unpack_state(const State& src, const State& dst, uint32_t n, const double* pos, const double* vel,
+                         uint32_t* bad, hipStream_t st);
+
 void launch_inverse_perm(const uint32_t* id, uint32_t* slot_of, uint32_t n, hipStream_t st);
 
 }  // namespace nbh

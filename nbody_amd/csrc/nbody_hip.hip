@@ -22,6 +22,7 @@
 #include "common.h"
 #include "expansion.h"
 #include "launch.h"
+#include "staging.h"
 
 using namespace nbh;
 
@@ -127,6 +128,9 @@ struct nbh_handle {
     unsigned long long m2l_pool_cap = 0, p2p_pool_cap = 0;
     DevBuf counters, diag, tmp_small;
     Counters* hc = nullptr;  // pinned host copy
+    uint32_t* bad = nullptr;  // pinned: nbh_set_state's values were not finite
+    DevBuf io;               // the caller's arrays on the device, in their layout
+    Staging staging;         // pinned chunks between io and the caller's memory
     DevBuf Mw, Lw, pw, wbuf, gbuf;   // adjoint
     // same-level M2L by translation offset (matrix cores): split moments
     // (forward and adjoint), dense tensor tables, candidate offsets
@@ -1298,8 +1302,9 @@ static int create_impl(const nbh_config* cfg, size_t nsys, const uint32_t* sys_o
     CCHK(h->counters.ensure(sizeof(Counters)));
     CCHK(h->diag.ensure(1024 * 8 * 8));
     CCHK(h->tmp_small.ensure(64));
-    CCHK(hipHostMalloc((void**)&h->hc, sizeof(Counters), hipHostMallocDefault));
-    std::memset(h->hc, 0, sizeof(Counters));
+    CCHK(hipHostMalloc((void**)&h->hc, sizeof(Counters) + 64, hipHostMallocDefault));
+    std::memset((void*)h->hc, 0, sizeof(Counters) + 64);
+    h->bad = (uint32_t*)(h->hc + 1);
     if (cfg->solver == NBH_SOLVER_FMM) {
         int r = alloc_nodes(h, (uint32_t)std::min<size_t>(n / 2 + 64, 0x7fffffff));
         if (r) return bail(r);
@@ -1393,24 +1398,16 @@ static int create_impl(const nbh_config* cfg, size_t nsys, const uint32_t* sys_o
                                                   : (cfg->m2l_order ? cfg->m2l_order : cfg->order + 1);
     CCHK(hipMemcpy(h->sys_off.p, sys_off, (nsys + 1) * 4, hipMemcpyHostToDevice));
     {
-        std::vector<double> buf(n);
-        State S = h->st[0].view();
-        double* dst[6] = {S.x, S.y, S.z, S.vx, S.vy, S.vz};
-        for (int k = 0; k < 6; ++k) {
-            const double* srcp = k < 3 ? pos : vel;
-            for (size_t i = 0; i < n; ++i) buf[i] = srcp[3 * i + (k % 3)];
-            CCHK(hipMemcpy(dst[k], buf.data(), n * 8, hipMemcpyHostToDevice));
-        }
-        CCHK(hipMemcpy(S.mass, mass, n * 8, hipMemcpyHostToDevice));
-        if (charge) CCHK(hipMemcpy(S.charge, charge, n * 8, hipMemcpyHostToDevice));
-        else CCHK(hipMemcpy(S.charge, mass, n * 8, hipMemcpyHostToDevice));
-        std::vector<uint32_t> ids(n);
-        for (size_t i = 0; i < n; ++i) ids[i] = (uint32_t)i;
-        CCHK(hipMemcpy(S.id, ids.data(), n * 4, hipMemcpyHostToDevice));
-        CCHK(hipMemset(S.ax, 0, n * 4));
-        CCHK(hipMemset(S.ay, 0, n * 4));
-        CCHK(hipMemset(S.az, 0, n * 4));
-        CCHK(hipMemset(S.pot, 0, n * 4));
+        const Staging::Part part[4] = {{const_cast<double*>(pos), n * 24},
+                                       {const_cast<double*>(vel), n * 24},
+                                       {const_cast<double*>(mass), n * 8},
+                                       {const_cast<double*>(charge ? charge : mass), n * 8}};
+        CCHK(h->io.ensure(n * 64));
+        CCHK(h->staging.to_device(part, 4, h->io.p, h->stream));
+        const double* d = h->io.as<double>();
+        launch_init_state(h->st[0].view(), (uint32_t)n, d, d + 3 * n, d + 6 * n, d + 7 * n, h->stream);
+        CCHK(hipGetLastError());
+        CCHK(hipStreamSynchronize(h->stream));
     }
 #undef CCHK
     *out = h;
@@ -1453,12 +1450,13 @@ void nbh_destroy(nbh_handle* h) {
                      &h->row_next, &h->row_sl_start, &h->row_sl_cnt, &h->row_m_start, &h->row_m_cnt,
                      &h->row_mx_cnt, &h->row_p_start, &h->row_p_cnt, &h->m2l_pool, &h->p2p_pool, &h->sl, &h->counters, &h->diag,
                      &h->tmp_small, &h->Mw, &h->Lw, &h->pw, &h->wbuf, &h->gbuf, &h->mb, &h->mbw, &h->d2tab,
-                     &h->cand, &h->hank, &h->opar, &h->sl_offs, &h->sl_map, &h->acc_save, &h->slot_of, &h->direct_buf};
+                     &h->cand, &h->hank, &h->opar, &h->sl_offs, &h->sl_map, &h->acc_save, &h->slot_of, &h->direct_buf, &h->io};
     for (DevBuf* b : all) b->release();
     for (DevBuf& b : h->adj_ckpt) b.release();
     for (DevBuf& b : h->adj_seg) b.release();
     DevBuf* adj[] = {&h->adj_final, &h->adj_xb, &h->adj_vb, &h->adj_mb, &h->adj_w};
     for (DevBuf* b : adj) b->release();
+    h->staging.release();
     if (h->hc) (void)hipHostFree(h->hc);
     for (auto& e : h->ev)
         if (e) (void)hipEventDestroy(e);
@@ -1491,23 +1489,26 @@ int nbh_get_state(nbh_handle* h, double* pos, double* vel, double* mass, double*
     if (!h) return NBH_E_INVALID;
     HIPCHK(h, hipSetDevice(h->device));
     const size_t n = h->n;
-    State S = h->st[h->cur].view();
-    std::vector<uint32_t> ids(n);
-    std::vector<double> buf(8 * n);
-    HIPCHK(h, hipMemcpyAsync(ids.data(), S.id, n * 4, hipMemcpyDeviceToHost, h->stream));
-    const double* src[8] = {S.x, S.y, S.z, S.vx, S.vy, S.vz, S.mass, S.charge};
-    double* dsts[8] = {pos, pos, pos, vel, vel, vel, mass, charge};
-    for (int k = 0; k < 8; ++k)
-        if (dsts[k]) HIPCHK(h, hipMemcpyAsync(&buf[k * n], src[k], n * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (int k = 0; k < 8; ++k) {
-        double* dst = dsts[k];
-        if (!dst) continue;
-        const double* b = &buf[k * n];
-        if (k < 6)
-            for (size_t i = 0; i < n; ++i) dst[3 * (size_t)ids[i] + (k % 3)] = b[i];
-        else
-            for (size_t i = 0; i < n; ++i) dst[ids[i]] = b[i];
+    double* const dst[4] = {pos, vel, mass, charge};
+    const size_t width[4] = {3, 3, 1, 1};
+    Staging::Part part[4];
+    int np = 0;
+    size_t doubles = 0;
+    for (int k = 0; k < 4; ++k)
+        if (dst[k]) {
+            part[np++] = {dst[k], width[k] * n * 8};
+            doubles += width[k] * n;
+        }
+    if (np) {
+        HIPCHK(h, h->io.ensure(doubles * 8));
+        double *d[4], *o = h->io.as<double>();
+        for (int k = 0; k < 4; ++k) {
+            d[k] = dst[k] ? o : nullptr;
+            if (dst[k]) o += width[k] * n;
+        }
+        launch_pack_state(h->st[h->cur].view(), (uint32_t)n, d[0], d[1], d[2], d[3], h->stream);
+        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, h->staging.to_host(part, np, h->io.p, h->stream));
     }
     if (t) *t = h->time;
     return NBH_OK;
@@ -1517,30 +1518,17 @@ int nbh_set_state(nbh_handle* h, const double* pos, const double* vel, double t)
     if (!h || !pos || !vel) return h ? h->fail(NBH_E_INVALID, "pos and vel are required") : NBH_E_INVALID;
     HIPCHK(h, hipSetDevice(h->device));
     const size_t n = h->n;
-    for (size_t i = 0; i < 3 * n; ++i)
-        if (!std::isfinite(pos[i]) || !std::isfinite(vel[i])) return h->fail(NBH_E_NONFINITE, "non-finite state");
-    State S = h->st[h->cur].view();
-    // masses/charges keep their current (sorted) slots: bring them to input order first
-    std::vector<uint32_t> ids(n);
-    std::vector<double> m(n), q(n), mi(n), qi(n), buf(n);
-    HIPCHK(h, hipMemcpyAsync(ids.data(), S.id, n * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(m.data(), S.mass, n * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(q.data(), S.charge, n * 8, hipMemcpyDeviceToHost, h->stream));
+    // into the other state buffer, which takes over if every value is finite
+    HIPCHK(h, h->io.ensure(n * 48));
+    const Staging::Part part[2] = {{const_cast<double*>(pos), n * 24}, {const_cast<double*>(vel), n * 24}};
+    HIPCHK(h, h->staging.to_device(part, 2, h->io.p, h->stream));
+    *h->bad = 0;
+    launch_unpack_state(h->st[h->cur].view(), h->st[1 - h->cur].view(), (uint32_t)n, h->io.as<double>(),
+                        h->io.as<double>() + 3 * n, h->bad, h->stream);
+    HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (size_t i = 0; i < n; ++i) { mi[ids[i]] = m[i]; qi[ids[i]] = q[i]; }
-    double* dst[6] = {S.x, S.y, S.z, S.vx, S.vy, S.vz};
-    buf.resize(6 * n);
-    for (int k = 0; k < 6; ++k) {
-        const double* srcp = k < 3 ? pos : vel;
-        double* b = &buf[k * n];
-        for (size_t i = 0; i < n; ++i) b[i] = srcp[3 * i + (k % 3)];
-        HIPCHK(h, hipMemcpyAsync(dst[k], b, n * 8, hipMemcpyHostToDevice, h->stream));
-    }
-    HIPCHK(h, hipMemcpyAsync(S.mass, mi.data(), n * 8, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipMemcpyAsync(S.charge, qi.data(), n * 8, hipMemcpyHostToDevice, h->stream));
-    for (size_t i = 0; i < n; ++i) ids[i] = (uint32_t)i;
-    HIPCHK(h, hipMemcpyAsync(S.id, ids.data(), n * 4, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (*h->bad) return h->fail(NBH_E_NONFINITE, "non-finite state");
+    h->cur = 1 - h->cur;
     h->time = t;
     h->acc_valid = false;
     h->pot_valid = false;
@@ -1553,24 +1541,17 @@ int nbh_compute_forces(nbh_handle* h, float* acc, float* pot) {
     CHK(force_eval(h, 0.0));
     h->acc_valid = true;
     const size_t n = h->n;
-    State S = h->st[h->cur].view();
-    std::vector<uint32_t> ids(n);
-    std::vector<float> a(n);
-    HIPCHK(h, hipMemcpyAsync(ids.data(), S.id, n * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    if (acc) {
-        float* src[3] = {S.ax, S.ay, S.az};
-        for (int k = 0; k < 3; ++k) {
-            HIPCHK(h, hipMemcpyAsync(a.data(), src[k], n * 4, hipMemcpyDeviceToHost, h->stream));
-            HIPCHK(h, hipStreamSynchronize(h->stream));
-            for (size_t i = 0; i < n; ++i) acc[3 * (size_t)ids[i] + k] = a[i];
-        }
-    }
-    if (pot) {
-        HIPCHK(h, hipMemcpyAsync(a.data(), S.pot, n * 4, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
-        for (size_t i = 0; i < n; ++i) pot[ids[i]] = a[i];
-    }
+    Staging::Part part[2];
+    int np = 0;
+    if (acc) part[np++] = {acc, n * 12};
+    if (pot) part[np++] = {pot, n * 4};
+    if (!np) return NBH_OK;
+    HIPCHK(h, h->io.ensure(n * 16));
+    float* d = h->io.as<float>();
+    launch_pack_forces(h->st[h->cur].view(), (uint32_t)n, acc ? d : nullptr, pot ? d + (acc ? 3 * n : 0) : nullptr,
+                       h->stream);
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, h->staging.to_host(part, np, h->io.p, h->stream));
     return NBH_OK;
 }
 
@@ -1646,15 +1627,15 @@ int nbh_direct_fp64(nbh_handle* h, size_t nt, const int64_t* targets, double* ac
     double* dacc = (double*)(dtg + nt);
     double* dpot = dacc + 3 * nt;
     uint32_t* dslot = (uint32_t*)(dpot + nt);
-    HIPCHK(h, hipMemcpyAsync(dtg, targets, nt * 8, hipMemcpyHostToDevice, h->stream));
+    const Staging::Part in{const_cast<int64_t*>(targets), nt * 8};
+    HIPCHK(h, h->staging.to_device(&in, 1, dtg, h->stream));
     launch_inverse_perm(S.id, h->slot_of.as<uint32_t>(), (uint32_t)n, h->stream);
     launch_map_slots(h->slot_of.as<uint32_t>(), dtg, (uint32_t)nt, dslot, h->stream);
     launch_direct_fp64(S, h->sys_off.as<uint32_t>(), h->nsys, dslot, (uint32_t)nt, h->cfg.G,
                        h->cfg.eps * h->cfg.eps, dacc, dpot, h->stream);
     HIPCHK(h, hipGetLastError());
-    HIPCHK(h, hipMemcpyAsync(acc, dacc, nt * 24, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(pot, dpot, nt * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const Staging::Part out[2] = {{acc, nt * 24}, {pot, nt * 8}};
+    HIPCHK(h, h->staging.to_host(out, 2, dacc, h->stream));
     return NBH_OK;
 }
 
@@ -1877,21 +1858,15 @@ int nbh_force_vjp(nbh_handle* h, const double* w, double* gx, double* gm) {
     HIPCHK(h, hipSetDevice(h->device));
     const size_t n = h->n;
     HIPCHK(h, h->wbuf.ensure(n * 24));
-    HIPCHK(h, hipMemcpyAsync(h->wbuf.p, w, n * 24, hipMemcpyHostToDevice, h->stream));
+    const Staging::Part in{const_cast<double*>(w), n * 24};
+    HIPCHK(h, h->staging.to_device(&in, 1, h->wbuf.p, h->stream));
     CHK(vjp_device(h, h->wbuf.as<double>()));
-    State S = h->st[h->cur].view();
-    std::vector<double> g(4 * n);
-    std::vector<uint32_t> ids(n);
-    HIPCHK(h, hipMemcpyAsync(g.data(), h->gbuf.p, 4 * n * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(ids.data(), S.id, n * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (size_t i = 0; i < n; ++i) {
-        const size_t j = ids[i];
-        gx[3 * j] = g[i];
-        gx[3 * j + 1] = g[n + i];
-        gx[3 * j + 2] = g[2 * n + i];
-        gm[j] = g[3 * n + i];
-    }
+    HIPCHK(h, h->io.ensure(n * 32));
+    double* d = h->io.as<double>();
+    launch_pack_gradient(h->gbuf.as<double>(), h->st[h->cur].view().id, (uint32_t)n, d, d + 3 * n, h->stream);
+    HIPCHK(h, hipGetLastError());
+    const Staging::Part out[2] = {{gx, n * 24}, {gm, n * 8}};
+    HIPCHK(h, h->staging.to_host(out, 2, d, h->stream));
     return NBH_OK;
 }
 
@@ -1937,8 +1912,9 @@ int nbh_adjoint_backward(nbh_handle* h, const double* xbar, const double* vbar, 
     double* vb = h->adj_vb.as<double>();
     double* mbar = h->adj_mb.as<double>();
     double* w = h->adj_w.as<double>();
-    HIPCHK(h, hipMemcpyAsync(xb, xbar, n * 24, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(h, hipMemcpyAsync(vb, vbar, n * 24, hipMemcpyHostToDevice, h->stream));
+    const Staging::Part in_x{const_cast<double*>(xbar), n * 24}, in_v{const_cast<double*>(vbar), n * 24};
+    HIPCHK(h, h->staging.to_device(&in_x, 1, xb, h->stream));
+    HIPCHK(h, h->staging.to_device(&in_v, 1, vb, h->stream));
     launch_fill_f64(mbar, n, 0.0, h->stream);
     // the last state: second half kick of the last step, cotangent dt/2 vbar
     CHK(snapshot_restore(h, h->adj_final, h->adj_final_t));
@@ -1968,9 +1944,10 @@ int nbh_adjoint_backward(nbh_handle* h, const double* xbar, const double* vbar, 
         }
     }
     HIPCHK(h, hipGetLastError());
-    HIPCHK(h, hipMemcpyAsync(gx, xb, n * 24, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(gv, vb, n * 24, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(gm, mbar, n * 8, hipMemcpyDeviceToHost, h->stream));
+    const Staging::Part out_x{gx, n * 24}, out_v{gv, n * 24}, out_m{gm, n * 8};
+    HIPCHK(h, h->staging.to_host(&out_x, 1, xb, h->stream));
+    HIPCHK(h, h->staging.to_host(&out_v, 1, vb, h->stream));
+    HIPCHK(h, h->staging.to_host(&out_m, 1, mbar, h->stream));
     // the handle ends at the trajectory's last state
     CHK(snapshot_restore(h, h->adj_final, h->adj_final_t));
     HIPCHK(h, hipStreamSynchronize(h->stream));
