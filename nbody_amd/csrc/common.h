@@ -21,16 +21,17 @@ struct NodeView {
 __device__ __forceinline__ int geo_level(int4 g) { return g.w & 0xff; }
 __device__ __forceinline__ int geo_nchild(int4 g) { return g.w >> 8; }
 
-// Counters that many wavefronts add to.  Atomics on one 128-byte line are
-// served one after the other, ~12 ns each however many XCDs they come from
-// (16,384 wavefronts adding once: 200 us on one line, 42 us on 8, 7 us on 64,
-// the time of the empty launch): every such counter has a line of its own, and
-// the sums that are only read later are kept in CNT_COPIES copies.
+// Counters that many wavefronts add to.  Atomics on one memory channel (256
+// bytes) are served one after the other, ~12 ns each however many XCDs they
+// come from (16,384 wavefronts adding once: 200 us on one word, 42 us on 8
+// words 128 bytes apart, 7 us on 64, the time of the empty launch), and loads
+// from it wait among them: every such counter has a channel's width of its
+// own, and the sums that are only read later are kept in CNT_COPIES copies.
 constexpr int CNT_COPIES = 64;
-struct alignas(128) LineU32 {
+struct alignas(256) LineU32 {
     uint32_t v;
 };
-struct alignas(128) LineTotals {
+struct alignas(256) LineTotals {
     unsigned long long m2l, p2p, split;
     unsigned long long m2lx;       // M2L entries between different levels
     unsigned long long p2p_inter;  // particle pairs of the P2P kernels
@@ -46,12 +47,12 @@ struct Counters {
     uint32_t level_count[MAX_LEVELS + 1];
     uint32_t level_off[MAX_LEVELS + 2];
     // (from here to far_pairs: cleared before each walk)
-    alignas(128) uint32_t carried[MAX_LEVELS + 2];  // walk: carried leaf rows per depth
+    alignas(256) uint32_t carried[MAX_LEVELS + 2];  // walk: carried leaf rows per depth
     LineU32 sl_used;                   // walk: split-list entries used
     LineU32 m2l_pool_used;             // walk: phase-1 segment pools used
     LineU32 p2p_pool_used;
     LineTotals tot[CNT_COPIES];
-    alignas(128) unsigned long long near_used;  // near field: work items (low half), slots asked for (high half)
+    alignas(256) unsigned long long near_used;  // near field: work items (low half), slots asked for (high half)
     LineU32 far_pairs;                 // M2L: deferred pairs (level gap >= 2)
     uint32_t nonfinite;
     uint32_t outside;                  // fixed root box: a particle lies outside it

@@ -38,10 +38,11 @@ void launch_tree_link(const uint64_t* keys, uint32_t n, const uint32_t* sys_off,
                       NodeView nodes, hipStream_t st);
 
 // ---- walk (walk.hip)
-// Per-wave chunk sizes of the walk's segment pools (entries).  A wave reserves
-// a chunk with one atomic and carves row segments from it; the host sizes the
-// pools for one unused tail per wave per depth.
-constexpr uint32_t POOL_CHUNK_M = 2048, POOL_CHUNK_P = 512, POOL_CHUNK_S = 512;
+// Chunk sizes of the walk's segment pools (entries).  A workgroup starts with
+// a chunk of its own, reserves more with one atomic each and carves row
+// segments from them; the host sizes the pools for one unused tail per
+// workgroup and depth.
+constexpr uint32_t POOL_CHUNK_M = 4096, POOL_CHUNK_P = 1024, POOL_CHUNK_S = 1024;
 constexpr uint32_t WALK_WAVES = 4;
 
 // A node's interaction lists are the segments of its rows, one row per walk
@@ -55,6 +56,9 @@ struct WalkParams {
     int bits;
     uint32_t num4;  // 4 num^2
     uint32_t den3;  // 3 den^2
+    uint32_t thr[MAX_LEVELS];  // walk_thresholds
+    uint32_t blocks;           // workgroups of all depths, and of the depths before
+    uint32_t first_block;      // the launch's (first chunks of the pools)
     uint32_t row_cap;
     int* row_node;
     uint32_t* row_first;  // [nodes]
@@ -72,6 +76,7 @@ struct WalkParams {
     int* p2p_pool;
     unsigned long long m2l_pool_cap, p2p_pool_cap;
 };
+void walk_thresholds(uint32_t num4, uint32_t den3, uint32_t* thr);
 void launch_walk_root(const WalkParams& W, hipStream_t st);
 void launch_walk_group(const WalkParams& W, int s, uint32_t grid, hipStream_t st);
 // workgroups of the group kernel resident at once on a device with num_cu CUs

@@ -514,7 +514,7 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
     for (uint32_t s = 1; s <= depth; ++s) {
         const uint32_t groups = gs ? 0 : h->hc->level_count[s - 1];
         grid[s] = gs ? gs->walk_grid[s] : std::max<uint32_t>(std::min<uint32_t>(groups + 16, h->walk_grid), 64);
-        blocks += std::min<unsigned long long>(grid[s], nn);
+        blocks += grid[s];
     }
     const unsigned long long waste_m = blocks * POOL_CHUNK_M, waste_p = blocks * POOL_CHUNK_P;
     const unsigned long long waste_s = blocks * POOL_CHUNK_S;
@@ -539,6 +539,7 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
     W.bits = h->bits;
     W.num4 = 4u * h->theta_num * h->theta_num;
     W.den3 = 3u * h->theta_den * h->theta_den;
+    walk_thresholds(W.num4, W.den3, W.thr);
     bool side_done = false;
     // the first walk depths are queued before the side stream's launches
     const uint32_t side_after = std::min<uint32_t>(depth, 2);
@@ -565,6 +566,8 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
         W.p2p_pool = h->p2p_pool.as<int>();
         W.m2l_pool_cap = h->m2l_pool_cap;
         W.p2p_pool_cap = h->p2p_pool_cap;
+        W.blocks = (uint32_t)blocks;
+        W.first_block = 0;
         const bool early = em && em->on;
         FmmParams Fe{};
         M2LPlan plan{};
@@ -596,6 +599,7 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
         }
         for (uint32_t s = 1; s <= depth; ++s) {
             launch_walk_group(W, (int)s, grid[s], h->stream);
+            W.first_block += grid[s];
             if (!side_done && s == side_after) {
                 CHK(run_side());
                 CHK(fork_same());

@@ -37,6 +37,8 @@
 //
 // The MAC is evaluated exactly in integers (units of half the finest cell):
 //   3 den^2 (d_A + d_B)^2 < 4 num^2 |c_B - c_A|^2,  theta = num/den.
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 
@@ -52,73 +54,19 @@ __device__ __forceinline__ uint32_t depth_base(const Counters* C, int s) {
 // Per-wave LDS cache of one split list (SL_CACHE entries at a time): the
 // entry's node id, geometry and first child.  Loading it once, coalesced,
 // leaves one global round trip (the children's geometry) per candidate chunk.
-constexpr int SL_CACHE = 256;
+constexpr int SL_CACHE = 512;
+constexpr int SL_FLY = 4;
 struct SLCache {
     int4* geo;
     int* node;
     int* fc;
 };
 
-__device__ __forceinline__ void sl_cache_fill(const WalkParams& W, const SLCache& c, uint32_t st, uint32_t e0,
-                                              uint32_t n) {
-    const int lane = lane_id();
-    for (uint32_t k = lane; k < n; k += WAVE) {
-        const int B = W.sl[st + e0 + k];
-        c.node[k] = B;
-        c.geo[k] = W.nodes.geo[B];
-        c.fc[k] = W.nodes.link[B].z;
-    }
-    wave_lds_sync();
-}
-
-// Enumerate expand(SL) for the split list at sl[st, st+cnt), one wavefront
-// with the cache to itself; f(phase, valid, B, geo) is called once per chunk
-// of 64 lanes (uniformly), in ascending candidate order: phase 0 the entries
-// without children (kept as themselves), then phase 1 the children of the
-// others, entry by entry.  The cache is refilled SL_CACHE entries at a time.
-template <typename F>
-__device__ __forceinline__ void enumerate_sl(const WalkParams& W, const SLCache& cache, uint32_t st, uint32_t cnt,
-                                             F&& f) {
-    const int lane = lane_id();
-    for (uint32_t p0 = 0; p0 < cnt; p0 += SL_CACHE) {
-        const uint32_t pn = min((uint32_t)SL_CACHE, cnt - p0);
-        sl_cache_fill(W, cache, st, p0, pn);
-        for (uint32_t e0 = 0; e0 < pn; e0 += WAVE) {
-            const uint32_t e = e0 + lane;
-            int B = -1;
-            int4 gb = make_int4(0, 0, 0, 0);
-            if (e < pn) {
-                B = cache.node[e];
-                gb = cache.geo[e];
-            }
-            const bool valid = B >= 0 && (gb.w >> 8) == 0;
-            if (__ballot(valid) == 0) continue;
-            f(0, valid, B, gb);
-        }
-        wave_lds_sync();
-    }
-    for (uint32_t p0 = 0; p0 < cnt; p0 += SL_CACHE) {
-        const uint32_t pn = min((uint32_t)SL_CACHE, cnt - p0);
-        sl_cache_fill(W, cache, st, p0, pn);
-        const int c = lane & 7;
-        for (uint32_t e0 = 0; e0 < pn; e0 += 16) {
-            bool v0 = false, v1 = false;
-            int C0 = -1, C1 = -1;
-            int4 g0 = make_int4(0, 0, 0, 0), g1 = make_int4(0, 0, 0, 0);
-            const uint32_t ea = e0 + (lane >> 3), eb = ea + 8;
-            if (ea < pn && c < (cache.geo[ea].w >> 8)) { C0 = cache.fc[ea] + c; v0 = true; }
-            if (eb < pn && c < (cache.geo[eb].w >> 8)) { C1 = cache.fc[eb] + c; v1 = true; }
-            if (v0) g0 = W.nodes.geo[C0];
-            if (v1) g1 = W.nodes.geo[C1];
-            if (__ballot(v0)) f(1, v0, C0, g0);
-            if (__ballot(v1)) f(1, v1, C1, g1);
-        }
-        wave_lds_sync();
-    }
-}
-
-// The same for the cached entries [lo, hi) of a list that the cache holds
-// whole (one wavefront's slice of a workgroup-shared cache).
+// Enumerate expand(SL) for the cached entries [lo, hi) of a split list (one
+// wavefront's slice of a workgroup-shared cache); f(phase, valid, B, geo) is
+// called once per chunk of 64 lanes (uniformly), in ascending candidate order:
+// phase 0 the entries without children (kept as themselves), then phase 1 the
+// children of the others, entry by entry.
 template <typename F>
 __device__ __forceinline__ void enumerate_slice(const WalkParams& W, const SLCache& cache, uint32_t lo, uint32_t hi,
                                                 F&& f) {
@@ -135,19 +83,25 @@ __device__ __forceinline__ void enumerate_slice(const WalkParams& W, const SLCac
         if (__ballot(valid) == 0) continue;
         f(0, valid, B, gb);
     }
-    // children: 8 entries x 8 slots per chunk, two chunks in flight
+    // children: 8 entries x 8 slots per chunk, SL_FLY chunks' cells loaded
+    // before the first is classified (every lane loads, a lane without a child
+    // node 0: a load under a branch is waited for at the branch's end, and each
+    // chunk then pays a memory round trip of its own)
     const int c = lane & 7;
-    for (uint32_t e0 = lo; e0 < hi; e0 += 16) {
-        bool v0 = false, v1 = false;
-        int C0 = -1, C1 = -1;
-        int4 g0 = make_int4(0, 0, 0, 0), g1 = make_int4(0, 0, 0, 0);
-        const uint32_t ea = e0 + (lane >> 3), eb = ea + 8;
-        if (ea < hi && c < (cache.geo[ea].w >> 8)) { C0 = cache.fc[ea] + c; v0 = true; }
-        if (eb < hi && c < (cache.geo[eb].w >> 8)) { C1 = cache.fc[eb] + c; v1 = true; }
-        if (v0) g0 = W.nodes.geo[C0];
-        if (v1) g1 = W.nodes.geo[C1];
-        if (__ballot(v0)) f(1, v0, C0, g0);
-        if (__ballot(v1)) f(1, v1, C1, g1);
+    for (uint32_t e0 = lo; e0 < hi; e0 += 8 * SL_FLY) {
+        int C[SL_FLY];
+        int4 g[SL_FLY];
+#pragma unroll
+        for (int k = 0; k < SL_FLY; ++k) {
+            const uint32_t e = e0 + 8 * k + (lane >> 3);
+            C[k] = -1;
+            if (e < hi && c < (cache.geo[e].w >> 8)) C[k] = cache.fc[e] + c;
+        }
+#pragma unroll
+        for (int k = 0; k < SL_FLY; ++k) g[k] = W.nodes.geo[max(C[k], 0)];
+#pragma unroll
+        for (int k = 0; k < SL_FLY; ++k)
+            if (__ballot(C[k] >= 0)) f(1, C[k] >= 0, C[k], g[k]);
     }
 }
 
@@ -169,14 +123,11 @@ __device__ __forceinline__ void enumerate_slice_ids(const SLCache& cache, uint32
         f(0, valid, B);
     }
     const int c = lane & 7;
-    for (uint32_t e0 = lo; e0 < hi; e0 += 16) {
-        bool v0 = false, v1 = false;
-        int C0 = -1, C1 = -1;
-        const uint32_t ea = e0 + (lane >> 3), eb = ea + 8;
-        if (ea < hi && c < (cache.geo[ea].w >> 8)) { C0 = cache.fc[ea] + c; v0 = true; }
-        if (eb < hi && c < (cache.geo[eb].w >> 8)) { C1 = cache.fc[eb] + c; v1 = true; }
-        if (__ballot(v0)) f(1, v0, C0);
-        if (__ballot(v1)) f(1, v1, C1);
+    for (uint32_t e0 = lo; e0 < hi; e0 += 8) {
+        const uint32_t e = e0 + (lane >> 3);
+        int C = -1;
+        if (e < hi && c < (cache.geo[e].w >> 8)) C = cache.fc[e] + c;
+        if (__ballot(C >= 0)) f(1, C >= 0, C);
     }
 }
 
@@ -206,6 +157,13 @@ __global__ __launch_bounds__(64) void walk_root_kernel(WalkParams W) {
     Counters* C = W.C;
     if (C->overflow & OVF_NODES) return;  // a captured step's tree outgrew its node arrays
     const uint32_t n_roots = C->level_count[0];
+    // (one workgroup) the pools start behind every workgroup's first chunks
+    if (threadIdx.x == 0) {
+        C->m2l_pool_used.v = W.blocks * POOL_CHUNK_M;
+        C->p2p_pool_used.v = W.blocks * POOL_CHUNK_P;
+        C->sl_used.v = W.blocks * POOL_CHUNK_S;
+    }
+    __syncthreads();
     for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n_roots; r += gridDim.x * blockDim.x) {
         if (r >= W.row_cap) {
             atomicOr(&C->overflow, (uint32_t)OVF_ROWS);
@@ -248,31 +206,75 @@ __global__ __launch_bounds__(64) void walk_root_kernel(WalkParams W) {
     }
 }
 
-constexpr int MAXT = 8;  // targets per group: the children of one cell
+constexpr int MAXT = 8;  // targets per group: the children of one cell, by octant
 // Calls of enumerate_slice per wavefront and group: a slice of at most
-// SL_CACHE / WALK_WAVES = 64 entries gives one chunk of kept entries and at
-// most 4 x 2 chunks of children.
-constexpr int CAT_CALLS = 1 + 2 * (SL_CACHE / WALK_WAVES / 16);
+// SL_CACHE / WALK_WAVES = 128 entries gives two chunks of kept entries and
+// sixteen of children.
+constexpr int SLICE = SL_CACHE / WALK_WAVES;
+constexpr int CAT_CALLS = SLICE / WAVE + SLICE / 8;
+
+__device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+
+// Per lane o < 8 (an octant): running entry counts of one phase by category.
+struct CatCount {
+    uint32_t m, x, p, s;  // M2L same level, M2L other level, P2P, split
+};
+// adds a chunk's entries: a the candidates that the lane's target accepts, of
+// the valid ones v, with lb those that are leaves and sl those of the
+// target's level
+__device__ __forceinline__ void cat_add(CatCount& c, uint64_t a, uint64_t v, uint64_t lb, uint64_t sl, bool leaf) {
+    const uint64_t near = v & ~a;
+    const uint32_t m = __popcll(a & sl), pp = leaf ? __popcll(near & lb) : 0;
+    c.m += m;
+    c.x += __popcll(a) - m;
+    c.p += pp;
+    c.s += __popcll(near) - pp;
+}
 
 // Depth s >= 1: one workgroup of WALK_WAVES wavefronts per group (row of
 // depth s-1).  The group's split list is cached once for the workgroup and
 // each wavefront classifies the candidates of a contiguous slice of it
 // against all targets.  Pass 1 counts per (wavefront, phase, target,
-// category); thread 0 reserves one block per pool for the group; every
+// category); one reservation per pool is made for the group; every
 // wavefront then writes its entries at offsets ordered phase-major,
 // wavefront-minor, which is the order of one wavefront walking the whole
-// list.  Lists longer than the cache are walked by wavefront 0 alone.  Rows
-// are taken with a fixed stride over the workgroups; their headers are read
-// 64 at a time so rows without work (leaves with nothing left to split) cost
-// one batched read.
+// list.  Lists longer than the cache (a coarse leaf beside a dense region
+// keeps thousands of entries) are taken a cache at a time: pass 1 counts,
+// pass 2 classifies each section again, the wavefronts' counts of the section
+// giving their offsets.  Rows are taken with a fixed stride over the
+// workgroups; their headers are read 64 at a time so rows without work (leaves
+// with nothing left to split) cost one batched read.
+//
+// The criterion for the 8 targets of a cell: in units of half the finer cell
+// of the pair the centre offset is (dx, dy, dz) for octant 0 and one or more
+// of them less 2 for the others, so a candidate takes six squares, eight sums
+// and eight compares with a threshold that depends on the level gap alone
+// (floor of 3 den^2 (d_A + d_B)^2 / 4 num^2, exact).  Squares are 24-bit
+// products in 32 bits where every offset of the chunk is below 32,000 (all but
+// level gaps of ten and more, which take the 64-bit form).  A chunk's
+// accepted candidates are one 64-bit mask per target; the categories follow
+// from it and three masks of the candidates (valid, leaf, target's level) by
+// scalar logic, and pass 2 replays the masks from LDS.
+//
+// Measured, a depth's kernel on average, against 64-bit offsets and a category
+// per lane, candidate and target, 256 cached entries with longer lists walked
+// by one wavefront, and every reservation an atomic: pair of 150,001 (theta =
+// 0.4) 281 -> 129 us, Plummer 1,048,576 151 -> 120 us (beside the M2L), 5003
+// 30 -> 20 us.  What is left of a heavy group (200 entries, 8 targets) at N =
+// 30,011 is 2 us of loads, 5 of counts, 12 of writes alone on its CU, and up
+// to 60 us where the CU's other groups are heavy too: the 4-byte list stores
+// bound it (one store per target with the list chosen per lane took the same).
 __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParams W, int s) {
     __shared__ int4 cgeo[SL_CACHE];
     __shared__ int cnode[SL_CACHE];
     __shared__ int cfc[SL_CACHE];
-    __shared__ uint32_t cnt_s[WALK_WAVES][2][4][MAXT];  // [wave][phase][same-level, other-level, P2P, split][target]
-    __shared__ uint32_t bcast[8];                       // pool starts, carried row, failure
-    // pass 1's categories of a cached group, 3 bits per target, per call and lane
-    __shared__ uint32_t cat_s[WALK_WAVES][CAT_CALLS][WAVE];
+    __shared__ CatCount cnt_s[WALK_WAVES][2][MAXT];       // [wave][phase][octant]
+    __shared__ uint32_t bcast[8];                         // pool starts, carried row, failure
+    __shared__ uint64_t mask_s[WALK_WAVES][CAT_CALLS][MAXT + 3];  // accepted by octant; valid, leaf, level
+    __shared__ uint32_t thr_s[MAX_LEVELS];
     Counters* C = W.C;
     if (C->overflow & OVF_NODES) return;  // a captured step's tree outgrew its node arrays
     const uint32_t n_prev_level = C->level_count[s - 1];
@@ -282,20 +284,26 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
     const uint32_t n_level = C->level_count[s];
     const uint32_t loff = C->level_off[s], loff_prev = C->level_off[s - 1];
     const int lane = lane_id();
-    const int wv = threadIdx.x / WAVE;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const SLCache cache{cgeo, cnode, cfc};
-    const uint64_t lt = lanemask_lt();
-    const int bits = W.bits;
-    const uint64_t num4 = W.num4, den3 = W.den3;
     const uint32_t nblk = gridDim.x;
+    if (threadIdx.x < MAX_LEVELS) thr_s[threadIdx.x] = W.thr[threadIdx.x];
     // lanes 0..2 of the first wavefront: the M2L, P2P and split pools
-    uint2 chunk = make_uint2(0, 0);
     const uint32_t pool_chunk = lane == 0 ? POOL_CHUNK_M : lane == 1 ? POOL_CHUNK_P : POOL_CHUNK_S;
     uint32_t* const pool_used = lane == 0   ? &C->m2l_pool_used.v
                                 : lane == 1 ? &C->p2p_pool_used.v
                                             : &C->sl_used.v;
     const unsigned long long pool_cap = lane == 0 ? W.m2l_pool_cap : lane == 1 ? W.p2p_pool_cap : W.sl_cap;
-    unsigned long long acc_m = 0, acc_p = 0, acc_s = 0, acc_x = 0;                           // thread 0 only
+    // the workgroup's first chunk of each pool is its own without asking: the
+    // pools begin with one for every workgroup of every depth, and the
+    // counters start behind them (walk_root_kernel).  At small sizes a
+    // workgroup has one group, and a thousand of them reserving at once
+    // waited up to 40 us for the counters.
+    uint2 chunk;
+    chunk.x = (W.first_block + blockIdx.x) * pool_chunk;
+    chunk.y = chunk.x + pool_chunk;
+    if (chunk.y > pool_cap) chunk = make_uint2(0, 0);
+    unsigned long long acc = 0;  // totals, lanes 0..3 of the first wavefront: M2L, P2P, split, M2L of other levels
     for (uint64_t j0 = 0; (uint64_t)blockIdx.x + j0 * nblk < n_groups; j0 += WAVE) {
         // headers of the next 64 rows of this workgroup (identical in every wavefront)
         const uint64_t gl = (uint64_t)blockIdx.x + (j0 + lane) * nblk;
@@ -317,11 +325,11 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
             const uint32_t g = (uint32_t)(blockIdx.x + (j0 + jl) * nblk);
             const uint32_t rg = base_prev + g;
             const int P = __builtin_amdgcn_readlane(P_l, jl);
-            const int gpw = __builtin_amdgcn_readlane(gp_l.w, jl);
+            const int gpx = __builtin_amdgcn_readlane(gp_l.x, jl), gpy = __builtin_amdgcn_readlane(gp_l.y, jl);
+            const int gpz = __builtin_amdgcn_readlane(gp_l.z, jl), gpw = __builtin_amdgcn_readlane(gp_l.w, jl);
             const uint32_t sl_st = __builtin_amdgcn_readlane(st_l, jl);
             const uint32_t sl_n = __builtin_amdgcn_readlane(sn_l, jl);
             const int nch = gpw >> 8;
-            __syncthreads();  // the previous group is done with the cache, counts and broadcasts
             int nt, A0;
             uint32_t row0 = 0;
             if (nch > 0) {  // the cell's children: level-s rows in id order
@@ -332,6 +340,7 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
                 nt = 1;
                 A0 = P;
             }
+            __syncthreads();  // the previous group is done with the cache, counts and broadcasts
             if ((unsigned long long)row0 + nt > W.row_cap) {
                 // the host retries with more rows; rows that fit are left empty so
                 // that the next depth reads only rows of this evaluation
@@ -346,204 +355,244 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
                 }
                 continue;
             }
-            // targets (all of one level): lane t < nt holds target t; per-target
-            // state lives in lane t and is read with readlane where the loop
-            // over targets needs it
-            int4 gt_l = make_int4(0, 0, 0, 0);
-            if (lane < nt) gt_l = W.nodes.geo[A0 + lane];
-            const int la = gpw & 0xff;
-            const int lt_level = nch > 0 ? la + 1 : la;
-            const int sa = bits - lt_level;
-            const int side_a = 1 << (sa + 1);
-            const int cax_l = (2 * gt_l.x + 1) << sa, cay_l = (2 * gt_l.y + 1) << sa, caz_l = (2 * gt_l.z + 1) << sa;
-            const int leaf_l = (gt_l.w >> 8) == 0;
-            // the split list: cached for the workgroup and sliced over the
-            // wavefronts, or (longer than the cache) walked by wavefront 0
-            const bool solo = sl_n > (uint32_t)SL_CACHE;
-            if (!solo) {
-                for (uint32_t k = threadIdx.x; k < sl_n; k += blockDim.x) {
-                    const int B = W.sl[sl_st + k];
+            // the split list, cached for the workgroup (a section of it at a
+            // time if it is longer than the cache) and sliced over the wavefronts
+            const bool whole = sl_n <= (uint32_t)SL_CACHE;
+            auto section = [&](uint32_t p0) -> uint32_t {  // entries cached
+                const uint32_t pn = min((uint32_t)SL_CACHE, sl_n - p0);
+                for (uint32_t k = threadIdx.x; k < pn; k += blockDim.x) {
+                    const int B = W.sl[sl_st + p0 + k];
                     cache.node[k] = B;
                     cache.geo[k] = W.nodes.geo[B];
                     cache.fc[k] = W.nodes.link[B].z;
                 }
-            }
-            __syncthreads();
-            const uint32_t lo = solo ? 0u : (uint32_t)(((uint64_t)sl_n * wv) / WALK_WAVES);
-            const uint32_t hi = solo ? (wv == 0 ? sl_n : 0u) : (uint32_t)(((uint64_t)sl_n * (wv + 1)) / WALK_WAVES);
-            auto each = [&](auto&& f) {
-                if (solo) {
-                    if (wv == 0 && sl_n) enumerate_sl(W, cache, sl_st, sl_n, f);
-                } else if (lo < hi) {
-                    enumerate_slice(W, cache, lo, hi, f);
-                }
+                return pn;
             };
-            // per-candidate part of the MAC, then the per-target categories
-            // (0 = M2L same level, 4 = M2L other level, 1 = P2P, 2 = split, 3 = none)
-            auto classify_all = [&](bool valid, int B, int4 gb, auto&& per_target) {
+            // targets: lane o < 8 holds the child of octant o (of a carried leaf,
+            // lane 0 the leaf): its index among the children, which are in
+            // octant order, and whether it is a leaf
+            int tgt = 0;  // index | leaf << 3 | present << 4
+            if (nch > 0) {
+                int4 gt = make_int4(0, 0, 0, 0);
+                if (lane < nt) gt = W.nodes.geo[A0 + lane];
+                const int oct = (gt.x & 1) << 2 | (gt.y & 1) << 1 | (gt.z & 1);
+                // (lanes without a child push past the octants)
+                tgt = __builtin_amdgcn_ds_permute((lane < nt ? oct : 8 + (lane & 31)) << 2,
+                                                  lane | ((gt.w >> 8) == 0) << 3 | 1 << 4);
+            } else {
+                tgt = 1 << 3 | 1 << 4;
+            }
+            const bool pres_l = lane < (nch > 0 ? MAXT : 1) && (tgt >> 4 & 1);
+            const bool leaf_l = tgt >> 3 & 1;
+            const int t_l = tgt & 7;
+            const uint32_t omask = __builtin_amdgcn_readfirstlane((uint32_t)__ballot(pres_l));
+            const uint32_t leaves = omask & __builtin_amdgcn_readfirstlane((uint32_t)__ballot(leaf_l));
+            const int lt_level = (gpw & 0xff) + (nch > 0 ? 1 : 0);
+            // octant 0's centre, in half cells of the targets' level
+            const int tx = nch > 0 ? 4 * gpx + 1 : 2 * gpx + 1, ty = nch > 0 ? 4 * gpy + 1 : 2 * gpy + 1;
+            const int tz = nch > 0 ? 4 * gpz + 1 : 2 * gpz + 1;
+            // the candidates that each octant's target accepts (lane o: octant o)
+            auto accept = [&](uint64_t v, int4 gb) -> uint64_t {
                 const int lb = gb.w & 0xff;
-                const int sb = bits - lb;
-                const int cbx = (2 * gb.x + 1) << sb, cby = (2 * gb.y + 1) << sb, cbz = (2 * gb.z + 1) << sb;
-                const uint64_t side = (uint64_t)side_a + (1ull << (sb + 1));
-                const uint64_t lhs = den3 * side * side;
-                const bool b_leaf = (gb.w >> 8) == 0;
+                const int sa = max(lb - lt_level, 0), sb = max(lt_level - lb, 0);
+                const int dx = ((2 * gb.x + 1) << sb) - (tx << sa), dy = ((2 * gb.y + 1) << sb) - (ty << sa);
+                const int dz = ((2 * gb.z + 1) << sb) - (tz << sa);
+                const uint32_t thr = thr_s[sa + sb];
+                const bool big = (uint32_t)(dx + 32000) > 64000u || (uint32_t)(dy + 32000) > 64000u ||
+                                 (uint32_t)(dz + 32000) > 64000u || thr == 0xffffffffu;
+                uint64_t a = 0;
+                if (!(__ballot(big) & v)) {
+                    const uint32_t x[2] = {(uint32_t)__mul24(dx, dx), (uint32_t)__mul24(dx - 2, dx - 2)};
+                    const uint32_t y[2] = {(uint32_t)__mul24(dy, dy), (uint32_t)__mul24(dy - 2, dy - 2)};
+                    const uint32_t z[2] = {(uint32_t)__mul24(dz, dz), (uint32_t)__mul24(dz - 2, dz - 2)};
 #pragma unroll
-                for (int t = 0; t < MAXT; ++t) {
-                    if (t < nt) {
-                        const int64_t dx = cbx - __builtin_amdgcn_readlane(cax_l, t);
-                        const int64_t dy = cby - __builtin_amdgcn_readlane(cay_l, t);
-                        const int64_t dz = cbz - __builtin_amdgcn_readlane(caz_l, t);
-                        const uint64_t dsq = (uint64_t)(dx * dx + dy * dy + dz * dz);
-                        // evaluated without short cuts: selects, not branches
-                        const bool approx = (B != A0 + t) & (lhs < num4 * dsq);
-                        const bool both_leaf = (__builtin_amdgcn_readlane(leaf_l, t) != 0) & b_leaf;
-                        const int near = both_leaf ? 1 : 2;
-                        const int far = lb == lt_level ? 0 : 4;
-                        const int cat = valid ? (approx ? far : near) : 3;
-                        per_target(t, cat);
+                    for (int o = 0; o < MAXT; ++o) {
+                        const uint64_t k = __ballot(x[o >> 2] + y[o >> 1 & 1] + z[o & 1] > thr) & v;
+                        a = lane == o ? k : a;
+                    }
+                } else {
+                    const uint64_t side = 2ull + (2ull << (sa + sb));
+                    const uint64_t lhs = (uint64_t)W.den3 * side * side;
+#pragma nounroll
+                    for (int o = 0; o < MAXT; ++o) {
+                        const int64_t ex = dx - (o >> 2) * 2, ey = dy - (o >> 1 & 1) * 2, ez = dz - (o & 1) * 2;
+                        const uint64_t k = __ballot(lhs < (uint64_t)W.num4 * (uint64_t)(ex * ex + ey * ey + ez * ez)) & v;
+                        a = lane == o ? k : a;
                     }
                 }
+                return a;
             };
-            // pass 1: counts of this wavefront's slice per phase, category, target
-            // (lane t); a cached group also keeps every call's categories for pass 2
-            uint32_t k0m = 0, k0x = 0, k0p = 0, k0s = 0, k1m = 0, k1x = 0, k1p = 0, k1s = 0;
-            int ncall = 0;  // uniform
-            each([&](int ph, bool valid, int B, int4 gb) {
-                uint32_t word = 0;
-                classify_all(valid, B, gb, [&](int t, int cat) {
-                    word |= (uint32_t)cat << (3 * t);
-                    const uint32_t cm = __popcll(__ballot(cat == 0)), cx = __popcll(__ballot(cat == 4));
-                    const uint32_t cp = __popcll(__ballot(cat == 1)), cs = __popcll(__ballot(cat == 2));
-                    if (lane == t) {
-                        if (ph == 0) { k0m += cm; k0x += cx; k0p += cp; k0s += cs; }
-                        else { k1m += cm; k1x += cx; k1p += cp; k1s += cs; }
-                    }
-                });
-                if (!solo && ncall < CAT_CALLS) cat_s[wv][ncall][lane] = word;
-                ++ncall;
-            });
-            if (lane < MAXT) {
-                cnt_s[wv][0][0][lane] = k0m; cnt_s[wv][0][1][lane] = k0x;
-                cnt_s[wv][0][2][lane] = k0p; cnt_s[wv][0][3][lane] = k0s;
-                cnt_s[wv][1][0][lane] = k1m; cnt_s[wv][1][1][lane] = k1x;
-                cnt_s[wv][1][2][lane] = k1p; cnt_s[wv][1][3][lane] = k1s;
-            }
-            __syncthreads();
-            // per target (lane t): totals, and this wavefront's start inside the
-            // target's segments per phase (counts of earlier (phase, wavefront))
-            uint32_t Tm = 0, Tx = 0, Tp = 0, Ts = 0;
-            uint32_t o0m = 0, o0x = 0, o0p = 0, o0s = 0, o1m = 0, o1x = 0, o1p = 0, o1s = 0;
-            if (lane < nt) {
-#pragma unroll
-                for (int ph = 0; ph < 2; ++ph)
-#pragma unroll
-                    for (int w = 0; w < (int)WALK_WAVES; ++w) {
-                        const uint32_t m = cnt_s[w][ph][0][lane], x = cnt_s[w][ph][1][lane];
-                        const uint32_t pp = cnt_s[w][ph][2][lane], ss = cnt_s[w][ph][3][lane];
-                        if (ph == 0 && w == wv) { o0m = Tm; o0x = Tx; o0p = Tp; o0s = Ts; }
-                        if (ph == 1 && w == wv) { o1m = Tm; o1x = Tx; o1p = Tp; o1s = Ts; }
-                        Tm += m; Tx += x; Tp += pp; Ts += ss;
-                    }
-            }
-            const uint32_t tm = wave_sum(Tm + Tx), tp = wave_sum(Tp), ts = wave_sum(Ts), tx = wave_sum(Tx);
-            // reserve one block per pool for all targets of the group (lanes
-            // 0..2 of the first wavefront, a pool each) and a carried leaf's row
-            // (lane 3): the atomics go out together
-            if (wv == 0) {
-                const uint32_t need = lane == 0 ? tm : lane == 1 ? tp : lane == 2 ? ts : 0u;
-                const uint32_t ovf = lane == 0 ? OVF_M2L : lane == 1 ? OVF_P2P : OVF_SL;
-                uint32_t at = 0;
-                if (need) {
-                    at = pool_take(chunk, need, pool_chunk, pool_used, pool_cap);
-                    if (at == 0xffffffffu) atomicOr(&C->overflow, ovf);
-                }
-                if (lane == 3 && nch == 0) {
-                    at = base + n_level + atomicAdd(&C->carried[s], 1u);
-                    if (at >= W.row_cap) {  // (no row to leave empty)
-                        atomicOr(&C->overflow, (uint32_t)OVF_ROWS);
-                        at = 0xffffffffu;
-                    }
-                }
-                const bool fail = __ballot(lane < 4 && at == 0xffffffffu) != 0;
-                if (lane == 0 && !fail) { acc_m += tm; acc_p += tp; acc_s += ts; acc_x += tx; }
-                if (lane < 4) bcast[lane] = at;
-                if (lane == 4) bcast[4] = fail;
-            }
-            __syncthreads();
-            if (nch == 0) row0 = bcast[3];
-            if (row0 == 0xffffffffu) continue;  // uniform: no row left for the carried leaf
-            const uint32_t fail = bcast[4];
-            // segment starts of lane t's target: exclusive prefix over lanes
-            // 0..7; a row's M2L segment holds its same-level sources, then the others
-            uint32_t em = fail ? 0u : Tm + Tx, ep = fail ? 0u : Tp, es = fail ? 0u : Ts;
-            const uint32_t nm_l = em, np_l = ep, ns_l = es;
-#pragma unroll
-            for (int o = 1; o < MAXT; o <<= 1) {
-                const uint32_t ym = __shfl_up(em, o, WAVE), yp = __shfl_up(ep, o, WAVE), ys = __shfl_up(es, o, WAVE);
-                if (lane >= o) { em += ym; ep += yp; es += ys; }
-            }
-            const uint32_t m0 = bcast[0] + em - nm_l, p0 = bcast[1] + ep - np_l, s0 = bcast[2] + es - ns_l;
-            if (wv == 0 && lane < nt) {
-                const uint32_t r = row0 + lane;
-                W.row_node[r] = A0 + lane;
-                W.row_next[r] = NO_ROW;
-                W.row_m_start[r] = m0;
-                W.row_m_cnt[r] = nm_l;
-                W.row_mx_cnt[r] = fail ? 0u : Tx;
-                W.row_p_start[r] = p0;
-                W.row_p_cnt[r] = np_l;
-                W.row_sl_start[r] = s0;
-                W.row_sl_cnt[r] = ns_l;
-                if (nch > 0) W.row_first[A0 + lane] = r;
-            }
-            if (nch == 0 && threadIdx.x == 0) W.row_next[rg] = row0;
-            if (fail || !(tm | tp | ts)) continue;  // uniform; the host retries after a failure
-            // pass 2: write this wavefront's entries
-            uint32_t c0m = m0 + o0m, c0x = m0 + Tm + o0x, c0p = p0 + o0p, c0s = s0 + o0s;
-            uint32_t c1m = m0 + o1m, c1x = m0 + Tm + o1x, c1p = p0 + o1p, c1s = s0 + o1s;
-            auto write_entries = [&](int ph, int B, int t, int cat) {
-                    const uint64_t bm = __ballot(cat == 0), bp = __ballot(cat == 1), bs = __ballot(cat == 2);
-                    const uint64_t bx = __ballot(cat == 4);
-                    const uint32_t cm = __builtin_amdgcn_readlane(ph == 0 ? c0m : c1m, t);
-                    const uint32_t cx = __builtin_amdgcn_readlane(ph == 0 ? c0x : c1x, t);
-                    const uint32_t cp = __builtin_amdgcn_readlane(ph == 0 ? c0p : c1p, t);
-                    const uint32_t cs = __builtin_amdgcn_readlane(ph == 0 ? c0s : c1s, t);
-                    if (cat == 0) W.m2l_pool[cm + __popcll(bm & lt)] = B;
-                    if (cat == 4) W.m2l_pool[cx + __popcll(bx & lt)] = B;
-                    if (cat == 1) W.p2p_pool[cp + __popcll(bp & lt)] = B;
-                    if (cat == 2) W.sl[cs + __popcll(bs & lt)] = B;
-                    if (lane == t) {
-                        if (ph == 0) {
-                            c0m += __popcll(bm); c0x += __popcll(bx); c0p += __popcll(bp); c0s += __popcll(bs);
-                        } else {
-                            c1m += __popcll(bm); c1x += __popcll(bx); c1p += __popcll(bp); c1s += __popcll(bs);
-                        }
-                    }
+            uint32_t pn = 0, lo = 0, hi = 0;
+            auto slice = [&] {
+                lo = (pn * wv) / WALK_WAVES;
+                hi = (pn * (wv + 1)) / WALK_WAVES;
             };
-            if (!solo && ncall <= CAT_CALLS) {
-                // the categories of pass 1, without the children's geometry or the MAC
+            // counts of this wavefront's slice per phase (lane o: octant o), and
+            // every call's masks, kept for the writes
+            CatCount k0, k1;
+            auto count_slice = [&] {
+                int ncall = 0;  // uniform
+                if (lo < hi)
+                    enumerate_slice(W, cache, lo, hi, [&](int ph, bool valid, int B, int4 gb) {
+                        const uint64_t v = __ballot(valid), lb = __ballot((gb.w >> 8) == 0);
+                        const uint64_t sl = __ballot((gb.w & 0xff) == lt_level);
+                        const uint64_t a = accept(v, gb);
+                        if (ph == 0) cat_add(k0, a, v, lb, sl, leaf_l);
+                        else cat_add(k1, a, v, lb, sl, leaf_l);
+                        if (lane < MAXT + 3)
+                            mask_s[wv][ncall][lane] = lane < MAXT ? a : lane == MAXT ? v : lane == MAXT + 1 ? lb : sl;
+                        ++ncall;
+                    });
+            };
+            auto write_slice = [&](CatCount& c0, CatCount& c1) {
                 int k = 0;
                 if (lo < hi)
-                    enumerate_slice_ids(cache, lo, hi, [&](int ph, bool valid, int B) {
-                        const uint32_t word = cat_s[wv][k][lane];
+                    enumerate_slice_ids(cache, lo, hi, [&](int ph, bool, int B) {
+                        const uint64_t w = mask_s[wv][k][min(lane, MAXT + 2)];
                         ++k;
-#pragma unroll
-                        for (int t = 0; t < MAXT; ++t)
-                            if (t < nt) write_entries(ph, B, t, valid ? (int)((word >> (3 * t)) & 7u) : 3);
+                        const uint64_t v = readlane64(w, MAXT), lb = readlane64(w, MAXT + 1), sl = readlane64(w, MAXT + 2);
+                        CatCount c = ph == 0 ? c0 : c1;
+#pragma nounroll
+                        for (uint32_t om = omask; om; om &= om - 1) {
+                            const int o = __ffs((int)om) - 1;  // uniform
+                            const uint64_t a = readlane64(w, o), near = v & ~a;
+                            const uint64_t bm = a & sl, bx = a & ~sl;
+                            const uint64_t bp = (leaves >> o & 1) ? near & lb : 0ull, bs = near & ~bp;
+                            auto put = [&](int* pool, uint32_t first, uint64_t b) {
+                                if (__builtin_amdgcn_inverse_ballot_w64(b))
+                                    pool[first + __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = B;
+                            };
+                            if (bm) put(W.m2l_pool, __builtin_amdgcn_readlane(c.m, o), bm);
+                            if (bx) put(W.m2l_pool, __builtin_amdgcn_readlane(c.x, o), bx);
+                            if (bp) put(W.p2p_pool, __builtin_amdgcn_readlane(c.p, o), bp);
+                            if (bs) put(W.sl, __builtin_amdgcn_readlane(c.s, o), bs);
+                        }
+                        cat_add(c, w, v, lb, sl, leaf_l);
+                        (ph == 0 ? c0 : c1) = c;
                     });
-            } else {
-                each([&](int ph, bool valid, int B, int4 gb) {
-                    classify_all(valid, B, gb, [&](int t, int cat) { write_entries(ph, B, t, cat); });
-                });
+            };
+            // one section: counted, reserved for, written.  More: all of them
+            // counted (their sums in k0, k1), reserved for, then each counted
+            // again and written.  b0, b1: where the section's entries of each
+            // phase start in lane o's segments (phase 1 after all of phase 0)
+            const uint32_t ns = max(1u, (sl_n + SL_CACHE - 1) / SL_CACHE), steps = ns == 1 ? 1 : 2 * ns;
+            CatCount b0{0, 0, 0, 0}, b1{0, 0, 0, 0};
+            k0 = k1 = CatCount{0, 0, 0, 0};
+            for (uint32_t step = 0; step < steps; ++step) {
+                if (step) __syncthreads();  // the cache and the counts are free
+                pn = section((step < ns ? step : step - ns) * SL_CACHE);
+                __syncthreads();
+                slice();
+                if (step >= ns) k0 = k1 = CatCount{0, 0, 0, 0};
+                count_slice();
+                if (step + 1 < ns) continue;
+                if (lane < MAXT) {
+                    cnt_s[wv][0][lane] = k0;
+                    cnt_s[wv][1][lane] = k1;
+                }
+                __syncthreads();
+                if (step + 1 == ns) {
+                    // per octant (lane o): totals, of phase 0 and of both
+                    CatCount T{0, 0, 0, 0}, Z{0, 0, 0, 0};
+                    if (pres_l) {
+#pragma unroll
+                        for (int ph = 0; ph < 2; ++ph) {
+#pragma unroll
+                            for (int w = 0; w < (int)WALK_WAVES; ++w) {
+                                const CatCount k = cnt_s[w][ph][lane];
+                                T.m += k.m; T.x += k.x; T.p += k.p; T.s += k.s;
+                            }
+                            if (ph == 0) Z = T;
+                        }
+                    }
+                    // totals of the group and segment starts of lane o's target:
+                    // inclusive prefixes over lanes 0..7; a row's M2L segment holds
+                    // its same-level sources, then the others
+                    uint32_t em = T.m + T.x, ep = T.p, es = T.s, ex = T.x;
+#pragma unroll
+                    for (int o = 1; o < MAXT; o <<= 1) {
+                        const uint32_t ym = __shfl_up(em, o, WAVE), yp = __shfl_up(ep, o, WAVE);
+                        const uint32_t ys = __shfl_up(es, o, WAVE), yx = __shfl_up(ex, o, WAVE);
+                        if (lane >= o) { em += ym; ep += yp; es += ys; ex += yx; }
+                    }
+                    const uint32_t tm = __builtin_amdgcn_readlane(em, MAXT - 1);
+                    const uint32_t tp = __builtin_amdgcn_readlane(ep, MAXT - 1);
+                    const uint32_t ts = __builtin_amdgcn_readlane(es, MAXT - 1);
+                    // reserve one block per pool for all targets of the group (lanes
+                    // 0..2 of the first wavefront, a pool each) and a carried leaf's
+                    // row (lane 3): the atomics go out together
+                    if (wv == 0) {
+                        const uint32_t need = lane == 0 ? tm : lane == 1 ? tp : lane == 2 ? ts : 0u;
+                        const uint32_t ovf = lane == 0 ? OVF_M2L : lane == 1 ? OVF_P2P : OVF_SL;
+                        uint32_t at = 0;
+                        if (need) {
+                            at = pool_take(chunk, need, pool_chunk, pool_used, pool_cap);
+                            if (at == 0xffffffffu) atomicOr(&C->overflow, ovf);
+                        }
+                        if (lane == 3 && nch == 0) {
+                            at = base + n_level + atomicAdd(&C->carried[s], 1u);
+                            if (at >= W.row_cap) {  // (no row to leave empty)
+                                atomicOr(&C->overflow, (uint32_t)OVF_ROWS);
+                                at = 0xffffffffu;
+                            }
+                        }
+                        const bool fail = __ballot(lane < 4 && at == 0xffffffffu) != 0;
+                        if (!fail) acc += lane == 3 ? __builtin_amdgcn_readlane(ex, MAXT - 1) : need;
+                        if (lane < 4) bcast[lane] = at;
+                        if (lane == 4) bcast[4] = fail;
+                    }
+                    __syncthreads();
+                    if (nch == 0) row0 = bcast[3];
+                    if (row0 == 0xffffffffu) break;  // uniform: no row left for the carried leaf
+                    const bool fail = bcast[4] != 0;
+                    const uint32_t m0 = bcast[0] + em - (T.m + T.x), p0 = bcast[1] + ep - T.p, s0 = bcast[2] + es - T.s;
+                    if (wv == 0 && pres_l) {
+                        const uint32_t r = row0 + t_l;
+                        W.row_node[r] = A0 + t_l;
+                        W.row_next[r] = NO_ROW;
+                        W.row_m_start[r] = fail ? 0u : m0;
+                        W.row_m_cnt[r] = fail ? 0u : T.m + T.x;
+                        W.row_mx_cnt[r] = fail ? 0u : T.x;
+                        W.row_p_start[r] = fail ? 0u : p0;
+                        W.row_p_cnt[r] = fail ? 0u : T.p;
+                        W.row_sl_start[r] = fail ? 0u : s0;
+                        W.row_sl_cnt[r] = fail ? 0u : T.s;
+                        if (nch > 0) W.row_first[A0 + t_l] = r;
+                    }
+                    if (nch == 0 && threadIdx.x == 0) W.row_next[rg] = row0;
+                    if (fail || !(tm | tp | ts)) break;  // uniform; the host retries after a failure
+                    b0 = CatCount{m0, m0 + T.m, p0, s0};
+                    b1 = CatCount{m0 + Z.m, m0 + T.m + Z.x, p0 + Z.p, s0 + Z.s};
+                    if (ns > 1) continue;
+                }
+                CatCount c0{0, 0, 0, 0}, c1{0, 0, 0, 0};  // this wavefront's next positions
+                if (pres_l) {
+#pragma unroll
+                    for (int w = 0; w < (int)WALK_WAVES; ++w) {
+                        if (w == wv) { c0 = b0; c1 = b1; }
+                        const CatCount u0 = cnt_s[w][0][lane], u1 = cnt_s[w][1][lane];
+                        b0.m += u0.m; b0.x += u0.x; b0.p += u0.p; b0.s += u0.s;
+                        b1.m += u1.m; b1.x += u1.x; b1.p += u1.p; b1.s += u1.s;
+                    }
+                }
+                write_slice(c0, c1);
             }
         }
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 4 && acc) {
         LineTotals& tot = C->tot[blockIdx.x % CNT_COPIES];
-        if (acc_m) atomicAdd(&tot.m2l, acc_m);
-        if (acc_p) atomicAdd(&tot.p2p, acc_p);
-        if (acc_s) atomicAdd(&tot.split, acc_s);
-        if (acc_x) atomicAdd(&tot.m2lx, acc_x);
+        atomicAdd(lane == 0 ? &tot.m2l : lane == 1 ? &tot.p2p : lane == 2 ? &tot.split : &tot.m2lx, acc);
+    }
+}
+
+// thr[gap]: the largest squared centre offset, in half cells of the finer of
+// two cells `gap` levels apart, that the criterion does not accept (2^32 - 1:
+// not below 2^32 - 1)
+void walk_thresholds(uint32_t num4, uint32_t den3, uint32_t* thr) {
+    for (int g = 0; g < MAX_LEVELS; ++g) {
+        const uint64_t side = 2ull + (2ull << g);
+        thr[g] = (uint32_t)std::min<uint64_t>((uint64_t)den3 * side * side / num4, 0xffffffffu);
     }
 }
 
