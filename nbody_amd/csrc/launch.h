@@ -18,14 +18,24 @@ size_t scan_tmp_bytes(uint32_t n_max);
 size_t radix_tmp_bytes(uint32_t n);
 void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, uint32_t n,
                       int nbits, void* tmp, hipStream_t st);
+// Systems of at most RANK_MAX particles: sorted keys and the state gathered
+// into their order in one launch
+constexpr uint32_t RANK_MAX = 40960;
+struct State;
+void launch_rank_sort(const uint64_t* keys, uint64_t* keys_out, const State& src, const State& dst, uint32_t n,
+                      hipStream_t st);
 
 // ---- tree (tree.hip)
 void launch_bbox(const double* x, const double* y, const double* z, const uint32_t* sys_off, int nsys,
                  uint32_t max_sys_n, int bits, int fixed, const double* flo, double fsize, double* part,
                  double4* box, double* inv, float* unit, uint32_t* nonfinite, hipStream_t st);
-void launch_keys(const double* x, const double* y, const double* z, uint32_t n, const uint32_t* sys_off,
-                 int nsys, int bits, const double4* box, const double* inv, uint64_t* keys, uint32_t* perm,
-                 uint32_t* fixed_flags, hipStream_t st);
+size_t bbox_part_bytes(uint32_t max_sys_n, int nsys);
+// the bounding cubes and the keys; perm = 0, 1, .., n - 1 (flags: non-finite,
+// outside a fixed root box)
+void launch_bbox_keys(const double* x, const double* y, const double* z, uint32_t n, const uint32_t* sys_off, int nsys,
+                      uint32_t max_sys_n, int bits, int fixed, const double* flo, double fsize, double* part,
+                      double4* box, double* inv, float* unit, uint32_t* flags, uint64_t* keys, uint32_t* perm,
+                      hipStream_t st);
 size_t tree_tmp_bytes(uint32_t n, int max_depth);
 void launch_tree_build(const uint64_t* keys, uint32_t n, const uint32_t* sys_off, int nsys, int bits, int cap,
                        int max_depth, NodeView nodes, uint32_t* node_begin, uint32_t* leaf_ids, uint32_t node_cap,

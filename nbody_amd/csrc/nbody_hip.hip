@@ -357,12 +357,17 @@ static int sort_particles(nbh_handle* h) {
     const uint32_t n = (uint32_t)h->n;
     State a = h->st[h->cur].view(), b = h->st[1 - h->cur].view();
     Counters* dC = h->counters.as<Counters>();
-    launch_bbox(a.x, a.y, a.z, h->sys_off.as<uint32_t>(), h->nsys, h->max_sys_n, h->bits, (int)h->cfg.fixed_root,
-                h->cfg.root_lo, h->cfg.root_size, h->bbox_part.as<double>(), h->box.as<double4>(),
-                h->inv.as<double>(), h->unit.as<float>(), &dC->nonfinite, h->stream);
-    launch_keys(a.x, a.y, a.z, n, h->sys_off.as<uint32_t>(), h->nsys, h->bits, h->box.as<double4>(),
-                h->inv.as<double>(), h->keys.as<uint64_t>(), h->perm.as<uint32_t>(),
-                h->cfg.fixed_root ? &dC->nonfinite : nullptr, h->stream);
+    // small systems: keys to one buffer, ranked into the other with the state
+    const bool rank = n <= RANK_MAX;
+    launch_bbox_keys(a.x, a.y, a.z, n, h->sys_off.as<uint32_t>(), h->nsys, h->max_sys_n, h->bits,
+                     (int)h->cfg.fixed_root, h->cfg.root_lo, h->cfg.root_size, h->bbox_part.as<double>(),
+                     h->box.as<double4>(), h->inv.as<double>(), h->unit.as<float>(), &dC->nonfinite,
+                     rank ? h->keys_alt.as<uint64_t>() : h->keys.as<uint64_t>(), h->perm.as<uint32_t>(), h->stream);
+    if (rank) {
+        launch_rank_sort(h->keys_alt.as<uint64_t>(), h->keys.as<uint64_t>(), a, b, n, h->stream);
+        h->cur = 1 - h->cur;
+        return NBH_OK;
+    }
     int keybits = 3 * h->bits;
     if (h->nsys > 1) {
         int sb = 0;
@@ -590,8 +595,8 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
         // ran 5.6 -> 6.1 ms per step at N=1M)
         if (gs && !side_done) CHK(run_side());
         if (side_done) CHK(fork_same());
-        // reset the walk part of the counters
-        zero_u32(&dC->carried[0], (offsetof(Counters, nonfinite) - offsetof(Counters, carried)) / 4, h->stream);
+        // reset the walk part of the counters (the tree build cleared all of them)
+        if (attempt) zero_u32(&dC->carried[0], (offsetof(Counters, nonfinite) - offsetof(Counters, carried)) / 4, h->stream);
         launch_walk_root(W, h->stream);
         if (!side_done && side_after == 0) {
             CHK(run_side());
@@ -1299,7 +1304,7 @@ static int create_impl(const nbh_config* cfg, size_t nsys, const uint32_t* sys_o
     CCHK(h->box.ensure(nsys * sizeof(double4)));
     CCHK(h->inv.ensure(nsys * 8));
     CCHK(h->unit.ensure(nsys * 4));
-    CCHK(h->bbox_part.ensure(nsys * (size_t)ceil_div(h->max_sys_n, 4096) * 6 * 8 + 64));
+    CCHK(h->bbox_part.ensure(bbox_part_bytes(h->max_sys_n, (int)nsys)));
     CCHK(h->leaf_ids.ensure(n * 4));
     CCHK(h->pf.ensure((n + DS_PAD) * 16));
     CCHK(h->pleaf.ensure(n * 4));

