@@ -52,7 +52,7 @@ void launch_tree_link(const uint64_t* keys, uint32_t n, const uint32_t* sys_off,
 // a chunk of its own, reserves more with one atomic each and carves row
 // segments from them; the host sizes the pools for one unused tail per
 // workgroup and depth.
-constexpr uint32_t POOL_CHUNK_M = 4096, POOL_CHUNK_P = 1024, POOL_CHUNK_S = 1024;
+constexpr uint32_t POOL_CHUNK_M = 2048, POOL_CHUNK_P = 512, POOL_CHUNK_S = 512;
 constexpr uint32_t WALK_WAVES = 4;
 
 // A node's interaction lists are the segments of its rows, one row per walk

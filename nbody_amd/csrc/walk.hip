@@ -162,6 +162,9 @@ __global__ __launch_bounds__(64) void walk_root_kernel(WalkParams W) {
         C->m2l_pool_used.v = W.blocks * POOL_CHUNK_M;
         C->p2p_pool_used.v = W.blocks * POOL_CHUNK_P;
         C->sl_used.v = W.blocks * POOL_CHUNK_S;
+        // the same-level M2L kernel's lanes past their lists load entry 0 and
+        // the node it names: it lies in a chunk that may stay empty
+        W.m2l_pool[0] = (int)C->level_off[0];
     }
     __syncthreads();
     for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n_roots; r += gridDim.x * blockDim.x) {
