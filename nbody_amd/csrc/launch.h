@@ -53,7 +53,9 @@ void launch_tree_link(const uint64_t* keys, uint32_t n, const uint32_t* sys_off,
 // segments from them; the host sizes the pools for one unused tail per
 // workgroup and depth.
 constexpr uint32_t POOL_CHUNK_M = 2048, POOL_CHUNK_P = 512, POOL_CHUNK_S = 512;
-constexpr uint32_t WALK_WAVES = 4;
+// A depth of at most this many workgroups (two a compute unit) is walked with
+// eight wavefronts a workgroup instead of four
+constexpr uint32_t WALK_WIDE = 512;
 
 // A node's interaction lists are the segments of its rows, one row per walk
 // depth that reached it: row_first[node] is its level row, row_next[row] the

@@ -211,10 +211,10 @@ __global__ __launch_bounds__(64) void walk_root_kernel(WalkParams W) {
 
 constexpr int MAXT = 8;  // targets per group: the children of one cell, by octant
 // Calls of enumerate_slice per wavefront and group: a slice of at most
-// SL_CACHE / WALK_WAVES = 128 entries gives two chunks of kept entries and
-// sixteen of children.
-constexpr int SLICE = SL_CACHE / WALK_WAVES;
-constexpr int CAT_CALLS = SLICE / WAVE + SLICE / 8;
+// SL_CACHE / NW entries (128 for four wavefronts) gives chunks of 64 kept
+// entries (two) and chunks of the children of 8 (sixteen).
+template <int NW>
+constexpr int cat_calls() { return (SL_CACHE / NW + WAVE - 1) / WAVE + SL_CACHE / NW / 8; }
 
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
     return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32 |
@@ -237,7 +237,7 @@ __device__ __forceinline__ void cat_add(CatCount& c, uint64_t a, uint64_t v, uin
     c.s += __popcll(near) - pp;
 }
 
-// Depth s >= 1: one workgroup of WALK_WAVES wavefronts per group (row of
+// Depth s >= 1: one workgroup of NW (4 or 8) wavefronts per group (row of
 // depth s-1).  The group's split list is cached once for the workgroup and
 // each wavefront classifies the candidates of a contiguous slice of it
 // against all targets.  Pass 1 counts per (wavefront, phase, target,
@@ -270,13 +270,14 @@ __device__ __forceinline__ void cat_add(CatCount& c, uint64_t a, uint64_t v, uin
 // 30,011 is 2 us of loads, 5 of counts, 12 of writes alone on its CU, and up
 // to 60 us where the CU's other groups are heavy too: the 4-byte list stores
 // bound it (one store per target with the list chosen per lane took the same).
-__global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParams W, int s) {
+template <int NW>
+__global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int s) {
     __shared__ int4 cgeo[SL_CACHE];
     __shared__ int cnode[SL_CACHE];
     __shared__ int cfc[SL_CACHE];
-    __shared__ CatCount cnt_s[WALK_WAVES][2][MAXT];       // [wave][phase][octant]
+    __shared__ CatCount cnt_s[NW][2][MAXT];       // [wave][phase][octant]
     __shared__ uint32_t bcast[8];                         // pool starts, carried row, failure
-    __shared__ uint64_t mask_s[WALK_WAVES][CAT_CALLS][MAXT + 3];  // accepted by octant; valid, leaf, level
+    __shared__ uint64_t mask_s[NW][cat_calls<NW>()][MAXT + 3];  // accepted by octant; valid, leaf, level
     __shared__ uint32_t thr_s[MAX_LEVELS];
     Counters* C = W.C;
     if (C->overflow & OVF_NODES) return;  // a captured step's tree outgrew its node arrays
@@ -427,8 +428,8 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
             };
             uint32_t pn = 0, lo = 0, hi = 0;
             auto slice = [&] {
-                lo = (pn * wv) / WALK_WAVES;
-                hi = (pn * (wv + 1)) / WALK_WAVES;
+                lo = (pn * wv) / NW;
+                hi = (pn * (wv + 1)) / NW;
             };
             // counts of this wavefront's slice per phase (lane o: octant o), and
             // every call's masks, kept for the writes
@@ -502,7 +503,7 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
 #pragma unroll
                         for (int ph = 0; ph < 2; ++ph) {
 #pragma unroll
-                            for (int w = 0; w < (int)WALK_WAVES; ++w) {
+                            for (int w = 0; w < (int)NW; ++w) {
                                 const CatCount k = cnt_s[w][ph][lane];
                                 T.m += k.m; T.x += k.x; T.p += k.p; T.s += k.s;
                             }
@@ -572,7 +573,7 @@ __global__ __launch_bounds__(WAVE * WALK_WAVES) void walk_group_kernel(WalkParam
                 CatCount c0{0, 0, 0, 0}, c1{0, 0, 0, 0};  // this wavefront's next positions
                 if (pres_l) {
 #pragma unroll
-                    for (int w = 0; w < (int)WALK_WAVES; ++w) {
+                    for (int w = 0; w < (int)NW; ++w) {
                         if (w == wv) { c0 = b0; c1 = b1; }
                         const CatCount u0 = cnt_s[w][0][lane], u1 = cnt_s[w][1][lane];
                         b0.m += u0.m; b0.x += u0.x; b0.p += u0.p; b0.s += u0.s;
@@ -604,14 +605,20 @@ void launch_walk_root(const WalkParams& W, hipStream_t st) {
 }
 uint32_t walk_group_resident_blocks(int num_cu) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&walk_group_kernel),
-                                                     WAVE * WALK_WAVES, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&walk_group_kernel<4>),
+                                                     WAVE * 4, 0) != hipSuccess ||
         per_cu < 1)
         per_cu = 1;
     return (uint32_t)per_cu * (uint32_t)(num_cu > 0 ? num_cu : 1);
 }
+// A depth with at most two groups a compute unit lasts as long as its heaviest
+// group, which eight wavefronts finish sooner than four (N = 5003, a depth's
+// kernel on average 19.1 -> 17.5 us, the two longest 34 -> 26 us).  With more
+// groups they only hold each other up: N = 30,011, all depths with four
+// wavefronts 26.4 us, with eight 29.8, by this rule 25.9.
 void launch_walk_group(const WalkParams& W, int s, uint32_t grid, hipStream_t st) {
-    hipLaunchKernelGGL(walk_group_kernel, dim3(grid), dim3(WAVE * WALK_WAVES), 0, st, W, s);
+    if (grid <= WALK_WIDE) hipLaunchKernelGGL(walk_group_kernel<8>, dim3(grid), dim3(WAVE * 8), 0, st, W, s);
+    else hipLaunchKernelGGL(walk_group_kernel<4>, dim3(grid), dim3(WAVE * 4), 0, st, W, s);
 }
 
 }  // namespace nbh
