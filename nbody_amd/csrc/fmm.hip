@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void l2p_kernel(FmmParams F, State S, uint32_t
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4 me = F.pf[i];
-    const float* Ls = F.L + (size_t)F.pleaf[i] * F.ncp;
+    const float* Ls = F.Lt + (size_t)F.pleaf[i] * F.ncp;
     float L[NC];
 #pragma unroll
     for (int k = 0; k < NC; ++k) L[k] = Ls[k];
@@ -173,8 +173,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     for (int k = 0; k < NC; ++k) out[k] = L[k];
 }
 
-// L2L: one thread per cell of the level (top-down), adds the parent's local
-// expansion shifted to this cell's centre.
+// A cell's own local expansion.
+template <int P>
+__device__ __forceinline__ void load_local(const FmmParams& F, int A, float* Lc) {
+    constexpr int NC = ncoef(P);
+    const float* sc = F.L + (size_t)A * F.ncp;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) Lc[k] = sc[k];
+    if (F.Lx) {  // the other-level and deferred pairs' part
+        const float* sx = F.Lx + (size_t)A * F.ncp;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) Lc[k] += sx[k];
+    }
+}
+// L2L of a level: one thread per cell (top-down), its expansion and the shifted
+// total of its parent, into Lt.
 template <int P>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void l2l_kernel(FmmParams F, uint32_t count,
                                                                                            uint32_t off) {
@@ -188,22 +201,63 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     const int A = (int)(off + t);
     const int4 g = F.nodes.geo[A];
     const int par = F.nodes.link[A].w;
-    if (par < 0) continue;
     const int4 gp = F.nodes.geo[par];
     const float3 d = centre_diff(gp, g, F.bits, F.unit[F.nodes.sys[A]]);  // c_child - c_parent
     float Lp[NC], Lc[NC];
-    const float* sp = F.L + (size_t)par * F.ncp;
-    float* sc = F.L + (size_t)A * F.ncp;
+    const float* sp = F.Lt + (size_t)par * F.ncp;
 #pragma unroll
-    for (int k = 0; k < NC; ++k) { Lp[k] = sp[k]; Lc[k] = sc[k]; }
-    if (F.Lx) {  // the other-level and deferred pairs' part
-        const float* sx = F.Lx + (size_t)A * F.ncp;
-#pragma unroll
-        for (int k = 0; k < NC; ++k) Lc[k] += sx[k];
-    }
+    for (int k = 0; k < NC; ++k) Lp[k] = sp[k];
+    load_local<P>(F, A, Lc);
     l2l_apply<P>(d.x, d.y, d.z, Lp, Lc);
+    float* out = F.Lt + (size_t)A * F.ncp;
 #pragma unroll
-    for (int k = 0; k < NC; ++k) sc[k] = Lc[k];
+    for (int k = 0; k < NC; ++k) out[k] = Lc[k];
+    }
+}
+
+// L2L of all levels from the root's down to `last` in one launch: a thread
+// notes the path from its cell up to the root and comes down it, every cell's
+// expansion added to the shifted sum so far, in the order of a launch per
+// level (the same sums).  The shifts are repeated for every cell below, which
+// costs nothing while the levels have no more cells than the GPU has lanes for
+// at one wavefront a SIMD; a launch per level then waits for launches
+// (3-5 us each) and memory.
+template <int P>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void l2l_path_kernel(FmmParams F,
+                                                                                                uint32_t count,
+                                                                                                uint32_t last) {
+    constexpr int NC = ncoef(P);
+    __shared__ int path_s[MAX_LEVELS][64];  // this lane's column: the cell, its parent, .., the root
+    if (count == DEV_COUNT) {
+        if (F.C->overflow & OVF_WALK) return;
+        count = last >= F.C->depth ? F.C->num_nodes : F.C->level_off[last + 1];
+    }
+    const int lane = threadIdx.x;
+    for (uint32_t A = blockIdx.x * 64u + lane; A < count; A += gridDim.x * 64u) {
+        int d = 0;
+        for (int a = (int)A; a >= 0 && d < MAX_LEVELS; a = F.nodes.link[a].w) path_s[d++][lane] = a;
+        const float unit = F.unit[F.nodes.sys[A]];
+        int4 gp = F.nodes.geo[path_s[d - 1][lane]];
+        float Lp[NC];
+        {
+            const float* sp = F.L + (size_t)path_s[d - 1][lane] * F.ncp;  // (a root has no other part)
+#pragma unroll
+            for (int k = 0; k < NC; ++k) Lp[k] = sp[k];
+        }
+        for (int j = d - 2; j >= 0; --j) {
+            const int c = path_s[j][lane];
+            const int4 g = F.nodes.geo[c];
+            float Lc[NC];
+            load_local<P>(F, c, Lc);
+            const float3 dx = centre_diff(gp, g, F.bits, unit);
+            l2l_apply<P>(dx.x, dx.y, dx.z, Lp, Lc);
+#pragma unroll
+            for (int k = 0; k < NC; ++k) Lp[k] = Lc[k];
+            gp = g;
+        }
+        float* out = F.Lt + (size_t)A * F.ncp;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) out[k] = Lp[k];
     }
 }
 
@@ -1217,6 +1271,10 @@ static void launch_l2l_t(const FmmParams& F, uint32_t count, uint32_t off, uint3
     hipLaunchKernelGGL((l2l_kernel<P>), dim3(ceil_div(items, 64)), dim3(64), 0, st, F, count, off);
 }
 template <int P>
+static void launch_l2l_path_t(const FmmParams& F, uint32_t count, uint32_t last, uint32_t items, hipStream_t st) {
+    hipLaunchKernelGGL((l2l_path_kernel<P>), dim3(ceil_div(items, 64)), dim3(64), 0, st, F, count, last);
+}
+template <int P>
 static void launch_p2p_t(const FmmParams& F, const State& S, uint32_t num_leaves, hipStream_t st) {
     if (F.pot) hipLaunchKernelGGL((p2p_kernel<P, true>), dim3(ceil_div(num_leaves, 4)), dim3(256), 0, st, F, S, num_leaves);
     else hipLaunchKernelGGL((p2p_kernel<P, false>), dim3(ceil_div(num_leaves, 4)), dim3(256), 0, st, F, S, num_leaves);
@@ -1263,12 +1321,17 @@ void launch_m2m_level(int p, const FmmParams& F, int level, uint32_t count, uint
     if (count == DEV_COUNT) off = (uint32_t)level;
     NBH_DISPATCH_P(p, launch_m2m_t<PP>(F, count, off, items, st));
 }
-void launch_l2l_level(int p, const FmmParams& F, int level, uint32_t count, uint32_t off, hipStream_t st,
-                      uint32_t grid_items) {
-    if (!count) return;
-    const uint32_t items = grid_items_of(count, grid_items);
-    if (count == DEV_COUNT) off = (uint32_t)level;
-    NBH_DISPATCH_P(p, launch_l2l_t<PP>(F, count, off, items, st));
+void launch_l2l(int p, const FmmParams& F, uint32_t depth, const uint32_t* level_count, const uint32_t* level_off,
+                hipStream_t st, const uint32_t* level_items) {
+    const uint32_t* items = level_items ? level_items : level_count;
+    uint32_t last = 0, sum = items[0];
+    while (last < depth && (uint64_t)sum + items[last + 1] <= L2L_PATH_NODES) sum += items[++last];
+    NBH_DISPATCH_P(p, launch_l2l_path_t<PP>(F, level_items ? DEV_COUNT : sum, last, sum, st));
+    for (uint32_t l = last + 1; l <= depth; ++l) {
+        if (!items[l]) continue;
+        const uint32_t count = level_items ? DEV_COUNT : level_count[l], off = level_items ? l : level_off[l];
+        NBH_DISPATCH_P(p, launch_l2l_t<PP>(F, count, off, items[l], st));
+    }
 }
 void launch_near_plan(const FmmParams& F, uint32_t num_leaves, hipStream_t st, uint32_t grid_items) {
     if (!num_leaves) return;

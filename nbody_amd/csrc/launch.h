@@ -149,6 +149,7 @@ struct FmmParams {
     // apart so that it can be computed beside the same-level kernels; L2L
     // adds it in (nullptr: those kernels add to L)
     float* Lx;
+    float* Lt;             // L2L's result: every cell's expansion and its ancestors' shifted to it
     int ncp;               // padded coefficient stride
     const uint32_t* leaf_ids;
     float4* pf;            // per particle: offset from its leaf centre, charge
@@ -194,8 +195,13 @@ void launch_p2m(int p, const FmmParams& F, const State& S, uint32_t num_leaves, 
                 uint32_t grid_items = 0);
 void launch_m2m_level(int p, const FmmParams& F, int level, uint32_t count, uint32_t off, hipStream_t st,
                       uint32_t grid_items = 0);
-void launch_l2l_level(int p, const FmmParams& F, int level, uint32_t count, uint32_t off, hipStream_t st,
-                      uint32_t grid_items = 0);
+// L2L down to `depth`; level_items: a captured step's grids, counts and offsets
+// read on the device.  The levels from the root's on that have at most
+// L2L_PATH_NODES cells together (one wavefront a SIMD: 256 x 4 x 64) take one
+// launch, those below one each
+constexpr uint32_t L2L_PATH_NODES = 65536;
+void launch_l2l(int p, const FmmParams& F, uint32_t depth, const uint32_t* level_count, const uint32_t* level_off,
+                hipStream_t st, const uint32_t* level_items = nullptr);
 // the P2P kernels leave the raw near-field sums of every particle in (ax, ay,
 // az, pot); launch_l2p adds the far field of the leaf's local expansion,
 // applies G q/m and the sign of the potential, and the kick v += a kick_dt

@@ -122,7 +122,7 @@ struct nbh_handle {
     int cur = 0;
     DevBuf sys_off, keys, keys_alt, perm, perm_alt, sort_tmp, tree_tmp, scan_tmp;
     DevBuf box, inv, unit, bbox_part;
-    DevBuf geo, link, nsys_of, node_begin, leaf_ids, M, L, Lx, pf, pleaf, dtab, xtab, far_src, far_tgt, near_items, near_k, near_first, near_part;
+    DevBuf geo, link, nsys_of, node_begin, leaf_ids, M, L, Lx, Lt, pf, pleaf, dtab, xtab, far_src, far_tgt, near_items, near_k, near_first, near_part;
     DevBuf row_node, row_first, row_next, row_sl_start, row_sl_cnt, sl, row_m_start, row_m_cnt, row_mx_cnt,
         row_p_start, row_p_cnt, m2l_pool, p2p_pool;
     unsigned long long m2l_pool_cap = 0, p2p_pool_cap = 0;
@@ -131,7 +131,7 @@ struct nbh_handle {
     uint32_t* bad = nullptr;  // pinned: nbh_set_state's values were not finite
     DevBuf io;               // the caller's arrays on the device, in their layout
     Staging staging;         // pinned chunks between io and the caller's memory
-    DevBuf Mw, Lw, pw, wbuf, gbuf;   // adjoint
+    DevBuf Mw, Lw, Lwt, pw, wbuf, gbuf;   // adjoint
     // same-level M2L by translation offset (matrix cores): split moments
     // (forward and adjoint), dense tensor tables, candidate offsets
     DevBuf mb, mbw, d2tab, cand, hank, opar;
@@ -315,6 +315,7 @@ static int alloc_nodes(nbh_handle* h, uint32_t need) {
     HIPCHK(h, h->M.ensure((size_t)cap * ncp * 4));
     HIPCHK(h, h->L.ensure((size_t)cap * ncp * 4));
     HIPCHK(h, h->Lx.ensure((size_t)cap * ncp * 4));
+    HIPCHK(h, h->Lt.ensure((size_t)cap * ncp * 4));
     HIPCHK(h, h->row_first.ensure((size_t)cap * 4));
     HIPCHK(h, h->near_k.ensure((size_t)cap * 4));
     HIPCHK(h, h->near_first.ensure((size_t)cap * 4));
@@ -440,6 +441,7 @@ static FmmParams fmm_params(nbh_handle* h) {
     F.G = (float)h->cfg.G;
     F.M = h->M.as<float>();
     F.L = h->L.as<float>();
+    F.Lt = h->Lt.as<float>();
     F.ncp = ncp_of((int)h->cfg.order);
     F.leaf_ids = h->leaf_ids.as<uint32_t>();
     F.pf = h->pf.as<float4>();
@@ -860,10 +862,7 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
         launch_m2l(p, q, F, gs ? graph_plan(h, *gs) : m2l_plan(h), h->stream);
     }
     record(h, 3);
-    for (uint32_t l = 1; l <= depth; ++l) {
-        if (gs) launch_l2l_level(p, F, (int)l, DEV_COUNT, 0, h->stream, gs->level_items[l]);
-        else launch_l2l_level(p, F, (int)l, h->hc->level_count[l], h->hc->level_off[l], h->stream);
-    }
+    launch_l2l(p, F, depth, h->hc->level_count, h->hc->level_off, h->stream, gs ? gs->level_items : nullptr);
     record(h, 4);
     h->lastF = F;
     if (for_vjp) {
@@ -1458,7 +1457,7 @@ void nbh_destroy(nbh_handle* h) {
     h->st[1].release();
     DevBuf* all[] = {&h->sys_off, &h->keys, &h->keys_alt, &h->perm, &h->perm_alt, &h->sort_tmp, &h->tree_tmp,
                      &h->scan_tmp, &h->box, &h->inv, &h->unit, &h->bbox_part, &h->geo, &h->link, &h->nsys_of,
-                     &h->node_begin, &h->leaf_ids, &h->M, &h->L, &h->Lx, &h->pf, &h->pleaf, &h->dtab, &h->xtab, &h->far_src, &h->far_tgt, &h->near_items, &h->near_k, &h->near_first,
+                     &h->node_begin, &h->leaf_ids, &h->M, &h->L, &h->Lx, &h->Lt, &h->Lwt, &h->pf, &h->pleaf, &h->dtab, &h->xtab, &h->far_src, &h->far_tgt, &h->near_items, &h->near_k, &h->near_first,
                      &h->near_part, &h->row_node, &h->row_first,
                      &h->row_next, &h->row_sl_start, &h->row_sl_cnt, &h->row_m_start, &h->row_m_cnt,
                      &h->row_mx_cnt, &h->row_p_start, &h->row_p_cnt, &h->m2l_pool, &h->p2p_pool, &h->sl, &h->counters, &h->diag,
@@ -1794,6 +1793,7 @@ static int vjp_device(nbh_handle* h, const double* w_dev) {
     const size_t ncp = (size_t)ncp_of(p);
     HIPCHK(h, h->Mw.ensure((size_t)h->num_nodes * ncp * 4));
     HIPCHK(h, h->Lw.ensure((size_t)h->num_nodes * ncp * 4));
+    HIPCHK(h, h->Lwt.ensure((size_t)h->num_nodes * ncp * 4));
     HIPCHK(h, h->pw.ensure(n * 16));
     HIPCHK(h, h->gbuf.ensure(n * 32));
     FmmParams F = h->lastF;
@@ -1801,6 +1801,7 @@ static int vjp_device(nbh_handle* h, const double* w_dev) {
     FmmParams Fw = F;
     Fw.M = h->Mw.as<float>();
     Fw.L = h->Lw.as<float>();
+    Fw.Lt = h->Lwt.as<float>();
     State S = h->st[h->cur].view();
     float4* pw = h->pw.as<float4>();
     double* gdev = h->gbuf.as<double>();
@@ -2064,7 +2065,7 @@ int nbh_debug_expansions(nbh_handle* h, float* M, float* L) {
     const int nc = ncoef((int)h->cfg.order), ncp = ncp_of((int)h->cfg.order);
     std::vector<float> buf(nn * ncp);
     float* outs[2] = {M, L};
-    DevBuf* srcs[2] = {&h->M, &h->L};
+    DevBuf* srcs[2] = {&h->M, &h->Lt};
     for (int k = 0; k < 2; ++k) {
         if (!outs[k]) continue;
         HIPCHK(h, hipMemcpyAsync(buf.data(), srcs[k]->p, buf.size() * 4, hipMemcpyDeviceToHost, h->stream));

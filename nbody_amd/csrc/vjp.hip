@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void vjp_far_kernel(FmmParams F, const float4*
     float L[NC];
     float H[6];
     {
-        const float* Ls = F.L + (size_t)A * F.ncp;
+        const float* Ls = F.Lt + (size_t)A * F.ncp;
 #pragma unroll
         for (int k = 0; k < NC; ++k) L[k] = Ls[k];
         l2p_hessian<P>(me.x, me.y, me.z, L, H);
@@ -280,7 +280,7 @@ static void launch_vjp_chain_t(int q, const M2LPlan& plan, const FmmParams& F, c
     if (plan.mfma)
         launch_off_moments(P, plan.mfma == 1, Fw.M, Fw.ncp, plan.num_nodes, Fw.nodes.geo, Fw.box, (void*)plan.off.mb, st);
     launch_m2l(P, q, Fw, plan, st);
-    for (int l = 1; l <= depth; ++l) launch_l2l_level(P, Fw, l, level_count[l], level_off[l], st);
+    launch_l2l(P, Fw, (uint32_t)depth, level_count, level_off, st);
 }
 
 #define NBH_VJP_DISPATCH(p, call)                      \
@@ -349,7 +349,7 @@ void launch_vjp_chain(int p, int q, const M2LPlan& plan, const FmmParams& F, con
 void launch_vjp_far(int p, const FmmParams& F, const FmmParams& Fw, const float4* pw, uint32_t n, double* g,
                     hipStream_t st) {
     NBH_VJP_DISPATCH(p, hipLaunchKernelGGL((vjp_far_kernel<PP>), dim3(ceil_div(n, 256)), dim3(256), 0, st, F, pw,
-                                           Fw.L, n, g, g + n, g + 2 * (size_t)n, g + 3 * (size_t)n));
+                                           Fw.Lt, n, g, g + n, g + 2 * (size_t)n, g + 3 * (size_t)n));
 }
 
 }  // namespace nbh
