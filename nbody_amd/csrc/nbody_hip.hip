@@ -501,6 +501,15 @@ static void copy_tables(FmmParams& F, const FmmParams& T) {
 
 static M2LPlan graph_plan(const nbh_handle* h, const GraphShape& gs);
 
+// Walk depths that are queued before the side stream's work (about 20 launches
+// at N = 5003, which take the host longer than two depths take the GPU: the
+// walk waited for its third).  With 4 against 2: five steps of N = 5003 2714 ->
+// 2221 us, forces at N = 4096 370 -> 326 us, gradient at N = 16,384 57.2 -> 51.5
+// ms, forces at N = 262,144 2605 -> 2553 us.  With 3: 2374, 337, 53.7, 2511; with
+// 6: 2100, 322, 54.0, 2519 (the moments and tables start too late for the
+// same-level kernels).
+constexpr uint32_t WALK_AHEAD = 4;
+
 // gs: a captured step: one attempt with the grids and buffers of gs, no
 // read-back (an overflow is flagged on the device and found after the step)
 // side: enqueues the side stream's work of the evaluation (moments and
@@ -553,7 +562,7 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
     walk_thresholds(W.num4, W.den3, W.thr);
     bool side_done = false;
     // the first walk depths are queued before the side stream's launches
-    const uint32_t side_after = std::min<uint32_t>(depth, 2);
+    const uint32_t side_after = std::min<uint32_t>(depth, WALK_AHEAD);
     auto run_side = [&]() -> int {
         if (side_done) return NBH_OK;
         side_done = true;
@@ -604,30 +613,37 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
         // reset the walk part of the counters (the tree build cleared all of them)
         if (attempt) zero_u32(&dC->carried[0], (offsetof(Counters, nonfinite) - offsetof(Counters, carried)) / 4, h->stream);
         launch_walk_root(W, h->stream);
-        if (!side_done && side_after == 0) {
-            CHK(run_side());
-            CHK(fork_same());
-        }
-        for (uint32_t s = 1; s <= depth; ++s) {
-            launch_walk_group(W, (int)s, grid[s], h->stream);
-            W.first_block += grid[s];
+        // the same-level kernel of a level, once its walk depth is queued
+        auto tabled = [&](uint32_t l) {
+            return early && (int)l >= Fe.dlevel0 && (int)l < Fe.dlevel0 + Fe.dnlev && (gs || h->hc->level_count[l]);
+        };
+        auto same_level = [&](uint32_t l) -> int {
+            if (!tabled(l)) return NBH_OK;
+            hipStream_t sl = (l & 1) ? h->stream4 : h->stream3;
+            HIPCHK(h, hipStreamWaitEvent(sl, h->ev_depth[l], 0));
+            if (!started && h->timing) (void)hipEventRecord(h->evc0, sl);
+            started = true;
+            if (h->timing) (void)hipEventRecord(h->ev_lvl[2 * l], sl);
+            launch_m2l_parts(em->p, em->q, Fe, plan, M2L_LEVELS, (int)l, sl);
+            if (h->timing) {
+                (void)hipEventRecord(h->ev_lvl[2 * l + 1], sl);
+                h->lvl_timed[l] = true;
+            }
+            return NBH_OK;
+        };
+        uint32_t queued = 1;  // levels below it are launched or not tabled
+        for (uint32_t s = 0; s <= depth; ++s) {
+            if (s) {
+                launch_walk_group(W, (int)s, grid[s], h->stream);
+                W.first_block += grid[s];
+                if (tabled(s)) HIPCHK(h, hipEventRecord(h->ev_depth[s], h->stream));
+            }
             if (!side_done && s == side_after) {
                 CHK(run_side());
                 CHK(fork_same());
             }
-            if (early && (int)s >= Fe.dlevel0 && (int)s < Fe.dlevel0 + Fe.dnlev && (gs || h->hc->level_count[s])) {
-                hipStream_t sl = (s & 1) ? h->stream4 : h->stream3;
-                HIPCHK(h, hipEventRecord(h->ev_depth[s], h->stream));
-                HIPCHK(h, hipStreamWaitEvent(sl, h->ev_depth[s], 0));
-                if (!started && h->timing) (void)hipEventRecord(h->evc0, sl);
-                started = true;
-                if (h->timing) (void)hipEventRecord(h->ev_lvl[2 * s], sl);
-                launch_m2l_parts(em->p, em->q, Fe, plan, M2L_LEVELS, (int)s, sl);
-                if (h->timing) {
-                    (void)hipEventRecord(h->ev_lvl[2 * s + 1], sl);
-                    h->lvl_timed[s] = true;
-                }
-            }
+            if (side_done)
+                for (; queued <= s; ++queued) CHK(same_level(queued));
         }
         if (gs) return NBH_OK;
         CHK(read_counters(h));
