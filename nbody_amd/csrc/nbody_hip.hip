@@ -847,9 +847,11 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
         F.far_cap = (uint32_t)std::min<unsigned long long>(nx, 0xffffffffull);
         F.far_cnt = &h->counters.as<Counters>()->far_pairs.v;
     }
-    // side stream, overlapping M2L and L2L: the near field (raw sums)
-    if (!for_vjp) {
-        HIPCHK(h, hipEventRecord(h->ev_walk, h->stream));
+    // side stream, overlapping M2L and L2L: the near field (raw sums), queued
+    // behind the cross-level kernels, whose chain is the longer one
+    HIPCHK(h, hipEventRecord(h->ev_walk, h->stream));
+    auto near_field = [&]() -> int {
+        if (for_vjp) return NBH_OK;
         HIPCHK(h, hipStreamWaitEvent(h->stream2, h->ev_walk, 0));
         record_side(h, 2);
         if (gs) {
@@ -864,18 +866,21 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
         }
         record_side(h, 3);
         HIPCHK(h, hipEventRecord(h->ev_near, h->stream2));
-    }
+        return NBH_OK;
+    };
     HIPCHK(h, hipStreamWaitEvent(h->stream, h->ev_side, 0));
     if (em.on) {
         // the same-level kernels run beside the walk; the other-level pairs
         // (into Lx) beside them; L2L waits for both
         launch_m2l_parts(p, q, F, gs ? graph_plan(h, *gs) : m2l_plan(h), M2L_REST, -1, h->stream);
+        CHK(near_field());
         HIPCHK(h, hipEventRecord(h->ev_same, h->stream3));
         HIPCHK(h, hipEventRecord(h->ev_same4, h->stream4));
         HIPCHK(h, hipStreamWaitEvent(h->stream, h->ev_same, 0));
         HIPCHK(h, hipStreamWaitEvent(h->stream, h->ev_same4, 0));
     } else {
         launch_m2l(p, q, F, gs ? graph_plan(h, *gs) : m2l_plan(h), h->stream);
+        CHK(near_field());
     }
     record(h, 3);
     launch_l2l(p, F, depth, h->hc->level_count, h->hc->level_off, h->stream, gs ? gs->level_items : nullptr);
