@@ -2,9 +2,10 @@
 //
 // Replaces OpenClSimulation's host side (open_cl_simulation.cpp:15-616): the
 // constructor's upload and octree build, step()'s phase sequence, and
-// particles().  All per-step phases run on one HIP stream; the host reads the
-// device counters twice per force evaluation (after the tree count, to size
-// the node arrays, and after the walk's counting phase, to size the lists).
+// particles().  An evaluation runs on four HIP streams ordered by events; the
+// host reads the device counters after the tree count (to size the node
+// arrays), after the walk (overflowed pools grow and the walk is repeated) and
+// at the end.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

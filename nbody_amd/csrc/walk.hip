@@ -23,11 +23,11 @@
 // one depth: rows of depth s are the level-s cells (in id order) followed by
 // the leaves carried from depth s-1.  Every row of depth s-1 is a group: its
 // candidate set expand(SL(row)) is shared by all of its targets at depth s --
-// the cell's children, or the carried leaf itself.  One wavefront takes one
-// group, loads each candidate once and classifies it against every target
-// (up to 8), in two passes: count, reserve, write.  Each row's M2L, P2P and
-// split entries land as contiguous segments carved from per-wave chunks of
-// three pools; a node's rows are chained in depth order (first row = its
+// the cell's children, or the carried leaf itself.  One workgroup takes one
+// group, each of its wavefronts a slice of the split list: a candidate is
+// loaded once and classified against every target (up to 8); then count,
+// reserve, write.  Each row's M2L, P2P and split entries land as contiguous
+// segments carved from per-workgroup chunks of three pools; a node's rows are chained in depth order (first row = its
 // level row, next = its carried row one depth deeper), and the force kernels
 // follow the chain, so no compaction pass is needed.
 //
@@ -50,8 +50,7 @@ __device__ __forceinline__ uint32_t depth_base(const Counters* C, int s) {
     return b;
 }
 
-
-// Per-wave LDS cache of one split list (SL_CACHE entries at a time): the
+// A workgroup's LDS cache of one split list (SL_CACHE entries at a time): the
 // entry's node id, geometry and first child.  Loading it once, coalesced,
 // leaves one global round trip (the children's geometry) per candidate chunk.
 constexpr int SL_CACHE = 512;
