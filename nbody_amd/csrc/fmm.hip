@@ -108,9 +108,13 @@ __global__ __launch_bounds__(256) void l2p_kernel(FmmParams F, State S, uint32_t
     }
 }
 
-// M2M (replaces moment.cl:72-160, which sums untranslated moments): one
-// thread per cell of the level; children's moments shifted to the parent
-// centre.  Levels run bottom-up.
+// M2M (replaces moment.cl:72-160, which sums untranslated moments): eight
+// lanes per cell of the level, a child's moments each, shifted to the parent
+// centre and summed by shuffles.  Levels run bottom-up.  A level of a small
+// tree lasts as long as one cell's chain of loads and products: with a child a
+// lane instead of a cell a lane, forces at N = 30,011 (order 5) 964 -> 911 us,
+// gradient at N = 16,384 (two chains of levels a step) 54.9 -> 53.6 ms, the
+// large cases the same.
 template <int P>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void m2m_kernel(FmmParams F, uint32_t count,
                                                                                            uint32_t off) {
@@ -120,25 +124,32 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
         count = F.C->level_count[off];
         off = F.C->level_off[off];
     }
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < count; t += gridDim.x * blockDim.x) {
-    const int A = (int)(off + t);
-    const int4 g = F.nodes.geo[A];
-    const int nch = g.w >> 8;
-    if (nch == 0) continue;
-    const int4 lk = F.nodes.link[A];
-    const float unit = F.unit[F.nodes.sys[A]];
-    float Mp[NC];
+    const uint32_t c = threadIdx.x & 7;
+    for (uint32_t t0 = blockIdx.x * 8; t0 < count; t0 += gridDim.x * 8) {  // uniform
+        const uint32_t t = t0 + threadIdx.x / 8;
+        const int A = (int)(off + min(t, count - 1));
+        const int4 g = F.nodes.geo[A];
+        const uint32_t nch = t < count ? (uint32_t)(g.w >> 8) : 0u;
+        float Mp[NC];
 #pragma unroll
-    for (int k = 0; k < NC; ++k) Mp[k] = 0.f;
-    for (int c = 0; c < nch; ++c) {
-        const int ch = lk.z + c;
-        const int4 gc = F.nodes.geo[ch];
-        const float3 d = centre_diff(g, gc, F.bits, unit);  // c_child - c_parent
-        m2m_apply<P>(d.x, d.y, d.z, F.M + (size_t)ch * F.ncp, Mp);
-    }
-    float* out = F.M + (size_t)A * F.ncp;
+        for (int k = 0; k < NC; ++k) Mp[k] = 0.f;
+        if (c < nch) {
+            const int ch = F.nodes.link[A].z + (int)c;
+            const int4 gc = F.nodes.geo[ch];
+            const float3 d = centre_diff(g, gc, F.bits, F.unit[F.nodes.sys[A]]);  // c_child - c_parent
+            m2m_apply<P>(d.x, d.y, d.z, F.M + (size_t)ch * F.ncp, Mp);
+        }
 #pragma unroll
-    for (int k = 0; k < NC; ++k) out[k] = Mp[k];
+        for (int k = 0; k < NC; ++k) {
+            Mp[k] += __shfl_xor(Mp[k], 1, WAVE);
+            Mp[k] += __shfl_xor(Mp[k], 2, WAVE);
+            Mp[k] += __shfl_xor(Mp[k], 4, WAVE);
+        }
+        if (c == 0 && nch) {
+            float* out = F.M + (size_t)A * F.ncp;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) out[k] = Mp[k];
+        }
     }
 }
 
@@ -1264,7 +1275,7 @@ static void launch_l2p_t(const FmmParams& F, const State& S, uint32_t n, double 
 }
 template <int P>
 static void launch_m2m_t(const FmmParams& F, uint32_t count, uint32_t off, uint32_t items, hipStream_t st) {
-    hipLaunchKernelGGL((m2m_kernel<P>), dim3(ceil_div(items, 64)), dim3(64), 0, st, F, count, off);
+    hipLaunchKernelGGL((m2m_kernel<P>), dim3(ceil_div(items, 8)), dim3(64), 0, st, F, count, off);
 }
 template <int P>
 static void launch_l2l_t(const FmmParams& F, uint32_t count, uint32_t off, uint32_t items, hipStream_t st) {
