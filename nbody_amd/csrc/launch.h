@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "common.h"
+#include "rules.h"
 
 namespace nbh {
 
@@ -48,11 +49,7 @@ void launch_tree_link(const uint64_t* keys, uint32_t n, const uint32_t* sys_off,
                       NodeView nodes, hipStream_t st);
 
 // ---- walk (walk.hip)
-// Chunk sizes of the walk's segment pools (entries).  A workgroup starts with
-// a chunk of its own, reserves more with one atomic each and carves row
-// segments from them; the host sizes the pools for one unused tail per
-// workgroup and depth.
-constexpr uint32_t POOL_CHUNK_M = 2048, POOL_CHUNK_P = 512, POOL_CHUNK_S = 512;
+// (chunk and pool sizes: rules.h)
 // A depth of at most this many workgroups (two a compute unit) is walked with
 // eight wavefronts a workgroup instead of four
 constexpr uint32_t WALK_WIDE = 512;

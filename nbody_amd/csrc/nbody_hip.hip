@@ -535,23 +535,19 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
     }
     const unsigned long long waste_m = blocks * POOL_CHUNK_M, waste_p = blocks * POOL_CHUNK_P;
     const unsigned long long waste_s = blocks * POOL_CHUNK_S;
-    // pools: sized from the last evaluation (or a per-node guess: a cell keeps
-    // about 1000 M2L and 230 P2P sources at theta = 1/2, in proportion to
-    // 1/theta^3, and no more than there are cells) and grown on overflow, which
-    // repeats the walk (a captured step's were sized beforehand)
+    // pools: sized from the last evaluation (or a per-node guess) and grown on
+    // overflow, which repeats the walk (a captured step's were sized beforehand)
     if (!gs && h->sl_cap < 64ull * nn + waste_s) {
         h->sl_cap = (uint32_t)std::min<unsigned long long>(64ull * nn + waste_s, 0xffff0000ull);
         HIPCHK(h, h->sl.ensure((size_t)h->sl_cap * 4));
     }
-    const double near = std::pow(0.5 * h->theta_den / h->theta_num, 3.0);
-    const unsigned long long mguess = (unsigned long long)(nn * std::min((double)nn, 1024.0 * near)) + waste_m;
-    const unsigned long long pguess = (unsigned long long)(nn * std::min((double)nn, 256.0 * near)) + waste_p;
-    if (!gs && h->m2l_pool_cap < mguess) {
-        h->m2l_pool_cap = std::min<unsigned long long>(mguess, 0xffff0000ull);
+    const PoolSizes guess = pool_guess(nn, h->theta_num, h->theta_den, blocks);
+    if (!gs && h->m2l_pool_cap < guess.m2l) {
+        h->m2l_pool_cap = guess.m2l;
         HIPCHK(h, h->m2l_pool.ensure((size_t)h->m2l_pool_cap * 4));
     }
-    if (!gs && h->p2p_pool_cap < pguess) {
-        h->p2p_pool_cap = std::min<unsigned long long>(pguess, 0xffff0000ull);
+    if (!gs && h->p2p_pool_cap < guess.p2p) {
+        h->p2p_pool_cap = guess.p2p;
         HIPCHK(h, h->p2p_pool.ensure((size_t)h->p2p_pool_cap * 4));
     }
     WalkParams W{};

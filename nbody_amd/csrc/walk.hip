@@ -163,7 +163,7 @@ __global__ __launch_bounds__(64) void walk_root_kernel(WalkParams W) {
         C->sl_used.v = W.blocks * POOL_CHUNK_S;
         // the same-level M2L kernel's lanes past their lists load entry 0 and
         // the node it names: it lies in a chunk that may stay empty
-        W.m2l_pool[0] = (int)C->level_off[0];
+        if (W.m2l_pool_cap > 0) W.m2l_pool[0] = (int)C->level_off[0];
     }
     __syncthreads();
     for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n_roots; r += gridDim.x * blockDim.x) {
