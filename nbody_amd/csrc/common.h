@@ -38,7 +38,12 @@ struct alignas(256) LineTotals {
 };
 
 // Device-side counters of one force evaluation.  Written by kernels, read by
-// the host once after the tree build and once after the walk's first phase.
+// the host once after the tree build (the part up to carried), once after the
+// walk's first phase and once at the end (the part up to tot, whose copies a
+// kernel has summed).  The host's reads are kept below 16 KiB: a larger copy
+// goes to a DMA engine, which waits for the kernel before it another 7 us (8
+// copies of 64 B after a kernel 13.4 us, of 17 KiB 20.0), and at times until
+// the next timer tick (a step of 8 particles 0.39 ms instead of 0.16).
 struct Counters {
     uint32_t num_nodes;
     uint32_t num_leaves;
@@ -46,18 +51,18 @@ struct Counters {
     uint32_t overflow;                 // bit flags, see OVF_*
     uint32_t level_count[MAX_LEVELS + 1];
     uint32_t level_off[MAX_LEVELS + 2];
-    // (from here to far_pairs: cleared before each walk)
+    uint32_t nonfinite;
+    uint32_t outside;                  // fixed root box: a particle lies outside it
+    // sums over tot
+    unsigned long long m2l_total, p2p_total, p2p_inter, split_total, m2lx_total;
+    // (from here on: cleared before each walk)
     alignas(256) uint32_t carried[MAX_LEVELS + 2];  // walk: carried leaf rows per depth
     LineU32 sl_used;                   // walk: split-list entries used
     LineU32 m2l_pool_used;             // walk: phase-1 segment pools used
     LineU32 p2p_pool_used;
-    LineTotals tot[CNT_COPIES];
     alignas(256) unsigned long long near_used;  // near field: work items (low half), slots asked for (high half)
     LineU32 far_pairs;                 // M2L: deferred pairs (level gap >= 2)
-    uint32_t nonfinite;
-    uint32_t outside;                  // fixed root box: a particle lies outside it
-    // sums over tot, made by the host when it has read the counters
-    unsigned long long m2l_total, p2p_total, p2p_inter, split_total, m2lx_total;
+    LineTotals tot[CNT_COPIES];
 };
 
 // OVF_GEOM: a same-level M2L block found a pair count or a source position

@@ -229,6 +229,20 @@ __global__ void zero_u32_kernel(uint32_t* p, size_t n) {
     if (i < n) p[i] = 0;
 }
 
+__global__ __launch_bounds__(WAVE) void sum_totals_kernel(Counters* C) {
+    static_assert(CNT_COPIES == WAVE, "one copy per lane");
+    const LineTotals& t = C->tot[threadIdx.x];
+    const unsigned long long m2l = wave_sum(t.m2l), p2p = wave_sum(t.p2p), inter = wave_sum(t.p2p_inter);
+    const unsigned long long split = wave_sum(t.split), m2lx = wave_sum(t.m2lx);
+    if (threadIdx.x == 0) {
+        C->m2l_total = m2l;
+        C->p2p_total = p2p;
+        C->p2p_inter = inter;
+        C->split_total = split;
+        C->m2lx_total = m2lx;
+    }
+}
+
 // A captured step processes levels 0..depth_cap: a deeper tree is flagged
 // like one that outgrew its node arrays, so that every later kernel of the
 // step stands down (those levels have no rows) and the host reruns it.
@@ -328,19 +342,19 @@ static int alloc_nodes(nbh_handle* h, uint32_t need) {
     return NBH_OK;
 }
 
-static int read_counters(nbh_handle* h) {
-    HIPCHK(h, hipMemcpyAsync(h->hc, h->counters.p, sizeof(Counters), hipMemcpyDeviceToHost, h->stream));
+// the first `bytes` of the counters to the host
+static int read_counters(nbh_handle* h, size_t bytes) {
+    HIPCHK(h, hipMemcpyAsync(h->hc, h->counters.p, bytes, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    Counters& c = *h->hc;
-    c.m2l_total = c.p2p_total = c.p2p_inter = c.split_total = c.m2lx_total = 0;
-    for (const LineTotals& t : c.tot) {
-        c.m2l_total += t.m2l;
-        c.p2p_total += t.p2p;
-        c.p2p_inter += t.p2p_inter;
-        c.split_total += t.split;
-        c.m2lx_total += t.m2lx;
-    }
     return NBH_OK;
+}
+// after the bounding box and the tree: what they count
+static int read_tree_counters(nbh_handle* h) { return read_counters(h, offsetof(Counters, carried)); }
+// after the walk or the evaluation: everything, the totals summed
+static int read_all_counters(nbh_handle* h) {
+    static_assert(offsetof(Counters, tot) < 16384, "the copy stays off the DMA engine");
+    hipLaunchKernelGGL(sum_totals_kernel, dim3(1), dim3(WAVE), 0, h->stream, h->counters.as<Counters>());
+    return read_counters(h, offsetof(Counters, tot));
 }
 
 static NodeView node_view(nbh_handle* h) {
@@ -404,7 +418,7 @@ static int build_tree(nbh_handle* h, const GraphShape* gs = nullptr) {
         hipLaunchKernelGGL(graph_guard_kernel, dim3(1), dim3(64), 0, h->stream, dC, gs->depth_cap);
         return NBH_OK;
     }
-    CHK(read_counters(h));
+    CHK(read_tree_counters(h));
     if (h->hc->nonfinite) return h->fail(NBH_E_NONFINITE, "non-finite particle position");
     if (h->hc->outside)
         return h->fail(NBH_E_OUTSIDE, "a particle lies outside the fixed root box [%g, %g) x [%g, %g) x [%g, %g)",
@@ -608,7 +622,7 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
         if (gs && !side_done) CHK(run_side());
         if (side_done) CHK(fork_same());
         // reset the walk part of the counters (the tree build cleared all of them)
-        if (attempt) zero_u32(&dC->carried[0], (offsetof(Counters, nonfinite) - offsetof(Counters, carried)) / 4, h->stream);
+        if (attempt) zero_u32(&dC->carried[0], (sizeof(Counters) - offsetof(Counters, carried)) / 4, h->stream);
         launch_walk_root(W, h->stream);
         // the same-level kernel of a level, once its walk depth is queued
         auto tabled = [&](uint32_t l) {
@@ -643,7 +657,7 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
                 for (; queued <= s; ++queued) CHK(same_level(queued));
         }
         if (gs) return NBH_OK;
-        CHK(read_counters(h));
+        CHK(read_all_counters(h));
         const uint32_t ovf = h->hc->overflow;
         const uint32_t walk_bits = OVF_SL | OVF_ROWS | OVF_M2L | OVF_P2P;
         if (ovf & walk_bits)
@@ -896,7 +910,7 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
     HIPCHK(h, hipGetLastError());
     if (gs) return NBH_OK;
     // stats (read at the end of the evaluation; one more sync)
-    CHK(read_counters(h));
+    CHK(read_all_counters(h));
     if (h->hc->overflow) return h->fail(NBH_E_INTERNAL, "overflow flags %u", h->hc->overflow);
     h->stats.num_nodes = h->num_nodes;
     h->stats.num_leaves = h->num_leaves;
@@ -951,7 +965,7 @@ static int force_direct(nbh_handle* h, double kick_dt) {
     launch_direct_f32(S, (uint32_t)h->n, h->max_sys_n, h->sys_off.as<uint32_t>(), h->nsys, h->box.as<double4>(), (float)h->cfg.G,
                       (float)(h->cfg.eps * h->cfg.eps), (int)h->cfg.force_law, kick_dt, h->pf.as<float>(), h->stream);
     HIPCHK(h, hipGetLastError());
-    CHK(read_counters(h));
+    CHK(read_tree_counters(h));
     if (h->hc->nonfinite) return h->fail(NBH_E_NONFINITE, "non-finite particle position");
     return NBH_OK;
 }
@@ -1109,7 +1123,7 @@ static int graph_step(nbh_handle* h) {
     if (!h->gexec[h->cur]) CHK(graph_capture(h));
     const int cur0 = h->cur;
     HIPCHK(h, hipGraphLaunch(h->gexec[cur0], h->stream));
-    CHK(read_counters(h));
+    CHK(read_all_counters(h));
     const Counters& c = *h->hc;
     if (c.nonfinite) return h->fail(NBH_E_NONFINITE, "non-finite particle position");
     if (c.outside) return h->fail(NBH_E_OUTSIDE, "a particle lies outside the fixed root box");
