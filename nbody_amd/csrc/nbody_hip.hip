@@ -127,6 +127,7 @@ struct nbh_handle {
     DevBuf row_node, row_first, row_next, row_sl_start, row_sl_cnt, sl, row_m_start, row_m_cnt, row_mx_cnt,
         row_p_start, row_p_cnt, m2l_pool, p2p_pool;
     unsigned long long m2l_pool_cap = 0, p2p_pool_cap = 0;
+    bool small_pools = false;  // the device had no room for pools of the usual sizes
     DevBuf counters, diag, tmp_small;
     Counters* hc = nullptr;  // pinned host copy
     uint32_t* bad = nullptr;  // pinned: nbh_set_state's values were not finite
@@ -323,6 +324,7 @@ static int alloc_nodes(nbh_handle* h, uint32_t need) {
     if (need <= h->node_cap) return NBH_OK;
     uint32_t cap = std::max<uint32_t>(need + need / 4, 1024);
     const int ncp = ncp_of((int)h->cfg.order);
+    h->node_cap = 0;  // (until every array is there)
     HIPCHK(h, h->geo.ensure((size_t)cap * 16));
     HIPCHK(h, h->link.ensure((size_t)cap * 16));
     HIPCHK(h, h->nsys_of.ensure((size_t)cap * 4));
@@ -480,11 +482,39 @@ static FmmParams fmm_params(nbh_handle* h) {
 }
 
 static int grow_rows(nbh_handle* h, uint32_t cap) {
-    h->row_cap = cap;
+    h->row_cap = 0;  // (until every array is there)
     DevBuf* rows[] = {&h->row_node, &h->row_next, &h->row_sl_start, &h->row_sl_cnt,
                       &h->row_m_start, &h->row_m_cnt, &h->row_mx_cnt, &h->row_p_start, &h->row_p_cnt};
     for (DevBuf* b : rows) HIPCHK(h, b->ensure((size_t)cap * 4));
+    h->row_cap = cap;
     return NBH_OK;
+}
+
+// A pool of at least `want` entries of 4 bytes.  Without room for it the pool
+// is gone and its capacity 0, so that no later call writes to it.
+template <typename T>
+static int ensure_pool(nbh_handle* h, DevBuf& buf, T& cap, unsigned long long want) {
+    if (cap >= want) return NBH_OK;
+    cap = 0;
+    HIPCHK(h, buf.ensure((size_t)want * 4));
+    cap = (T)want;
+    return NBH_OK;
+}
+
+// The M2L and P2P pools before an evaluation's first walk.  A device without
+// room for the usual sizes gets the small ones, from then on.
+static int guess_pools(nbh_handle* h, unsigned long long blocks) {
+    auto both = [&]() -> int {
+        const PoolSizes g =
+            pool_guess(h->num_nodes, h->max_sys_n, h->n, h->theta_num, h->theta_den, blocks, h->small_pools);
+        CHK(ensure_pool(h, h->m2l_pool, h->m2l_pool_cap, g.m2l));
+        return ensure_pool(h, h->p2p_pool, h->p2p_pool_cap, g.p2p);
+    };
+    const int rc = both();
+    if (rc != NBH_E_NOMEM || h->small_pools) return rc;
+    (void)hipGetLastError();  // the failed allocation's, which a launch check would report
+    h->small_pools = true;
+    return both();
 }
 
 static M2LPlan m2l_plan(const nbh_handle* h);
@@ -551,19 +581,8 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
     const unsigned long long waste_s = blocks * POOL_CHUNK_S;
     // pools: sized from the last evaluation (or a per-node guess) and grown on
     // overflow, which repeats the walk (a captured step's were sized beforehand)
-    if (!gs && h->sl_cap < 64ull * nn + waste_s) {
-        h->sl_cap = (uint32_t)std::min<unsigned long long>(64ull * nn + waste_s, 0xffff0000ull);
-        HIPCHK(h, h->sl.ensure((size_t)h->sl_cap * 4));
-    }
-    const PoolSizes guess = pool_guess(nn, h->theta_num, h->theta_den, blocks);
-    if (!gs && h->m2l_pool_cap < guess.m2l) {
-        h->m2l_pool_cap = guess.m2l;
-        HIPCHK(h, h->m2l_pool.ensure((size_t)h->m2l_pool_cap * 4));
-    }
-    if (!gs && h->p2p_pool_cap < guess.p2p) {
-        h->p2p_pool_cap = guess.p2p;
-        HIPCHK(h, h->p2p_pool.ensure((size_t)h->p2p_pool_cap * 4));
-    }
+    if (!gs) CHK(ensure_pool(h, h->sl, h->sl_cap, std::min(64ull * nn + waste_s, POOL_MAX)));
+    if (!gs) CHK(guess_pools(h, blocks));
     WalkParams W{};
     W.nodes = node_view(h);
     W.C = dC;
@@ -669,10 +688,8 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
             HIPCHK(h, hipStreamSynchronize(h->stream4));
         }
         if (ovf & OVF_SL) {
-            h->sl_cap = (uint32_t)std::min<unsigned long long>(
-                std::max<unsigned long long>(2ull * h->sl_cap, h->hc->sl_used.v + h->hc->sl_used.v / 4 + waste_s),
-                0xffff0000ull);
-            HIPCHK(h, h->sl.ensure((size_t)h->sl_cap * 4));
+            const unsigned long long need = h->hc->sl_used.v + h->hc->sl_used.v / 4 + waste_s;
+            CHK(ensure_pool(h, h->sl, h->sl_cap, std::min(std::max<unsigned long long>(2ull * h->sl_cap, need), POOL_MAX)));
         }
         if (ovf & OVF_ROWS) {
             uint64_t need = 0;
@@ -680,14 +697,12 @@ static int run_walk(nbh_handle* h, const EarlyM2L* em = nullptr, const GraphShap
             CHK(grow_rows(h, (uint32_t)std::max<uint64_t>((uint64_t)h->row_cap * 2, need + need / 4)));
         }
         if (ovf & OVF_M2L) {
-            h->m2l_pool_cap = std::min<unsigned long long>(
-                std::max<unsigned long long>(h->m2l_pool_cap * 2, h->hc->m2l_pool_used.v + waste_m), 0xffff0000ull);
-            HIPCHK(h, h->m2l_pool.ensure((size_t)h->m2l_pool_cap * 4));
+            const unsigned long long need = h->hc->m2l_pool_used.v + waste_m;
+            CHK(ensure_pool(h, h->m2l_pool, h->m2l_pool_cap, std::min(std::max(2 * h->m2l_pool_cap, need), POOL_MAX)));
         }
         if (ovf & OVF_P2P) {
-            h->p2p_pool_cap = std::min<unsigned long long>(
-                std::max<unsigned long long>(h->p2p_pool_cap * 2, h->hc->p2p_pool_used.v + waste_p), 0xffff0000ull);
-            HIPCHK(h, h->p2p_pool.ensure((size_t)h->p2p_pool_cap * 4));
+            const unsigned long long need = h->hc->p2p_pool_used.v + waste_p;
+            CHK(ensure_pool(h, h->p2p_pool, h->p2p_pool_cap, std::min(std::max(2 * h->p2p_pool_cap, need), POOL_MAX)));
         }
         if (ovf & walk_bits) {
             uint32_t keep = ovf & ~walk_bits;
@@ -1012,7 +1027,7 @@ static void graph_shape_update(nbh_handle* h) {
         }
     }
     // every workgroup may leave one unused chunk tail per depth
-    const unsigned long long cap32 = 0xffff0000ull;
+    const unsigned long long cap32 = POOL_MAX;
     g.m2l_cap = std::min(std::max<unsigned long long>(h->m2l_pool_cap,
                                                       c.m2l_pool_used.v + c.m2l_pool_used.v / 4 + blocks * POOL_CHUNK_M),
                          cap32);
@@ -1042,18 +1057,9 @@ static int graph_prepare(nbh_handle* h) {
     const GraphShape& g = h->gshape;
     CHK(alloc_nodes(h, g.node_cap));
     if (h->row_cap < g.row_cap) CHK(grow_rows(h, g.row_cap));
-    if (h->sl_cap < g.sl_cap) {
-        h->sl_cap = g.sl_cap;
-        HIPCHK(h, h->sl.ensure((size_t)h->sl_cap * 4));
-    }
-    if (h->m2l_pool_cap < g.m2l_cap) {
-        h->m2l_pool_cap = g.m2l_cap;
-        HIPCHK(h, h->m2l_pool.ensure((size_t)h->m2l_pool_cap * 4));
-    }
-    if (h->p2p_pool_cap < g.p2p_cap) {
-        h->p2p_pool_cap = g.p2p_cap;
-        HIPCHK(h, h->p2p_pool.ensure((size_t)h->p2p_pool_cap * 4));
-    }
+    CHK(ensure_pool(h, h->sl, h->sl_cap, g.sl_cap));
+    CHK(ensure_pool(h, h->m2l_pool, h->m2l_pool_cap, g.m2l_cap));
+    CHK(ensure_pool(h, h->p2p_pool, h->p2p_pool_cap, g.p2p_cap));
     // the tables (as force_fmm sizes them) and the deferred pairs
     const int q = m2l_q(h);
     const int Kp = (int)std::floor(std::sqrt(3.0) * h->theta_den / h->theta_num);

@@ -17,25 +17,35 @@ constexpr uint32_t POOL_CHUNK_M = 2048, POOL_CHUNK_P = 512, POOL_CHUNK_S = 512;
 // the most entries of a pool (its counter has 32 bits)
 constexpr unsigned long long POOL_MAX = 0xffff0000ull;
 
-// First sizes (entries) of the M2L and P2P pools for `nodes` cells walked by
-// `blocks` workgroups at theta = num / den: a cell keeps about 1000 M2L and
-// 230 P2P sources at theta = 1/2, in proportion to 1/theta^3, and no more than
-// there are cells.  One chunk at least, whatever the tree and theta: the
-// walk's first kernel stores entry 0 of the M2L pool, also of a tree without
-// a list (one cell, no workgroup of the walk), where the product below is less
-// than one entry from theta = 5.1 on.
+// First sizes (entries) of the M2L and P2P pools for `nodes` cells of a handle
+// whose largest system holds max_sys_n of its n particles, walked by `blocks`
+// workgroups at theta = num / den.  A cell keeps about 1000 M2L and 230 P2P
+// sources at theta = 1/2, in proportion to 1/theta^3, and no more than its own
+// system has cells or, since a cell's sources are disjoint, particles.  What
+// theta < 1/2 adds stays within POOL_GUESS_MAX: a pool that is too small is
+// grown after the walk, which is then repeated.  `small`: 256 and 64 sources a
+// cell, for a device without room for more.  One chunk at least, whatever the
+// tree and theta: the walk's first kernel stores entry 0 of the M2L pool, also
+// of a tree without a list (one cell, no workgroup of the walk), where the
+// product below is less than one entry from theta = 5.1 on.
+constexpr double POOL_GUESS_MAX = 1u << 29;  // entries, 2 GiB
 struct PoolSizes {
     unsigned long long m2l, p2p;
 };
-inline PoolSizes pool_guess(uint32_t nodes, int num, int den, unsigned long long blocks) {
+inline PoolSizes pool_guess(uint32_t nodes, uint32_t max_sys_n, uint64_t n, int num, int den,
+                            unsigned long long blocks, bool small) {
     const double near = std::pow(0.5 * den / num, 3.0);
-    auto pool = [&](double per_cell, uint32_t chunk) {
-        const double entries = nodes * std::min((double)nodes, per_cell * near);
+    const double cells = std::min(std::ceil((double)nodes * max_sys_n / n), (double)max_sys_n);
+    auto pool = [&](double usual, double few, uint32_t chunk) {
+        const double at_half = nodes * std::min(cells, usual * std::min(near, 1.0));
+        const double at_theta = nodes * std::min(cells, usual * near);
+        const double entries =
+            small ? nodes * std::min(cells, few) : std::max(at_half, std::min(at_theta, POOL_GUESS_MAX));
         const unsigned long long want =
             (unsigned long long)std::min(entries, (double)POOL_MAX) + blocks * chunk;
         return std::min(std::max<unsigned long long>(want, chunk), POOL_MAX);
     };
-    return {pool(1024.0, POOL_CHUNK_M), pool(256.0, POOL_CHUNK_P)};
+    return {pool(1024.0, 256.0, POOL_CHUNK_M), pool(256.0, 64.0, POOL_CHUNK_P)};
 }
 
 }  // namespace nbh
