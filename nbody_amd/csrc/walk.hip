@@ -360,7 +360,6 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
             }
             // the split list, cached for the workgroup (a section of it at a
             // time if it is longer than the cache) and sliced over the wavefronts
-            const bool whole = sl_n <= (uint32_t)SL_CACHE;
             auto section = [&](uint32_t p0) -> uint32_t {  // entries cached
                 const uint32_t pn = min((uint32_t)SL_CACHE, sl_n - p0);
                 for (uint32_t k = threadIdx.x; k < pn; k += blockDim.x) {
@@ -522,6 +521,9 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
                     const uint32_t tm = __builtin_amdgcn_readlane(em, MAXT - 1);
                     const uint32_t tp = __builtin_amdgcn_readlane(ep, MAXT - 1);
                     const uint32_t ts = __builtin_amdgcn_readlane(es, MAXT - 1);
+                    // (here, with every lane active: under a condition on the lane the
+                    // last sums of lane 7 may be left out)
+                    const uint32_t tx = __builtin_amdgcn_readlane(ex, MAXT - 1);
                     // reserve one block per pool for all targets of the group (lanes
                     // 0..2 of the first wavefront, a pool each) and a carried leaf's
                     // row (lane 3): the atomics go out together
@@ -541,7 +543,7 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
                             }
                         }
                         const bool fail = __ballot(lane < 4 && at == 0xffffffffu) != 0;
-                        if (!fail) acc += lane == 3 ? __builtin_amdgcn_readlane(ex, MAXT - 1) : need;
+                        if (!fail) acc += lane == 3 ? tx : need;
                         if (lane < 4) bcast[lane] = at;
                         if (lane == 4) bcast[4] = fail;
                     }
