@@ -35,6 +35,7 @@ struct alignas(256) LineTotals {
     unsigned long long m2l, p2p, split;
     unsigned long long m2lx;       // M2L entries between different levels
     unsigned long long p2p_inter;  // particle pairs of the P2P kernels
+    unsigned long long near_work;  // near field: batches of the P2P lists times their target chunks
 };
 
 // Device-side counters of one force evaluation.  Written by kernels, read by
@@ -54,13 +55,13 @@ struct Counters {
     uint32_t nonfinite;
     uint32_t outside;                  // fixed root box: a particle lies outside it
     // sums over tot
-    unsigned long long m2l_total, p2p_total, p2p_inter, split_total, m2lx_total;
+    unsigned long long m2l_total, p2p_total, p2p_inter, split_total, m2lx_total, near_work;
     // (from here on: cleared before each walk)
     alignas(256) uint32_t carried[MAX_LEVELS + 2];  // walk: carried leaf rows per depth
     LineU32 sl_used;                   // walk: split-list entries used
     LineU32 m2l_pool_used;             // walk: phase-1 segment pools used
     LineU32 p2p_pool_used;
-    alignas(256) unsigned long long near_used;  // near field: work items (low half), slots asked for (high half)
+    alignas(256) unsigned long long near_used;  // near field: work items (low half), slots taken (high half)
     LineU32 far_pairs;                 // M2L: deferred pairs (level gap >= 2)
     LineTotals tot[CNT_COPIES];
 };

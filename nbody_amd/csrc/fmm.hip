@@ -368,9 +368,9 @@ __global__ __launch_bounds__(256) void p2p_kernel(FmmParams F, State S, uint32_t
 // wavefront per leaf the longest list was the kernel's time.  So a list of more
 // than G batches is cut into items of at most G, G = the evaluation's batches
 // / NEAR_BATCHES (about three rounds of resident wavefronts; 1 for small
-// systems), and each item leaves its partial sums in a slot that the join
-// kernel adds up in order (no atomics: the sums do not depend on which item
-// ran first).  P2P kernel, one wavefront per leaf -> items, with the pair
+// systems) or more where the slots ask for it (rules.h), and each item leaves
+// its partial sums in a slot that the join kernel adds up in order (no atomics:
+// the sums do not depend on which item ran first).  P2P kernel, one wavefront per leaf -> items, with the pair
 // count's atomics spread over CNT_COPIES lines: Plummer 5003 100 -> 21 us,
 // 30,011 (p = 5) 682 -> 86 us, two spheres of 150,001 (p = 6, theta = 0.4)
 // 5.65 -> 1.1 ms, the adjoint's kernel at 16,384 590 -> 190 us; 1,048,576
@@ -385,8 +385,8 @@ __global__ __launch_bounds__(256) void near_plan_kernel(FmmParams F, uint32_t nu
     __shared__ uint32_t wsum[NW][2];
     __shared__ unsigned long long first;
     static_assert(CNT_COPIES == WAVE, "one copy per lane");
-    const unsigned long long entries = wave_sum(C->tot[lane].p2p);
-    const uint32_t G = (uint32_t)max(1ull, (entries / WAVE + NEAR_BATCHES - 1) / NEAR_BATCHES);
+    const uint32_t G =
+        near_item_batches(wave_sum(C->tot[lane].p2p), wave_sum(C->tot[lane].near_work), F.near_slot_cap);
     for (uint32_t t0 = blockIdx.x * 256; t0 < num_leaves; t0 += gridDim.x * 256) {  // uniform over the workgroup
         const uint32_t t = t0 + threadIdx.x;
         int A = 0;
@@ -398,10 +398,9 @@ __global__ __launch_bounds__(256) void near_plan_kernel(FmmParams F, uint32_t nu
             tc = ((uint32_t)F.nodes.link[A].y + WAVE - 1) / WAVE;
             k = max(1u, (nb + G - 1) / G);
         }
-        // items, and slots for the leaves that are cut; items are reserved for
-        // every leaf as if it found its slots, which is at most what they all
-        // take uncut, and the slots there are
-        uint32_t want = k > 1 ? tc * k : 0u;
+        // slots for the leaves that are cut, and uncut items for every leaf (empty
+        // ones for a leaf that is cut)
+        const uint32_t want = k > 1 ? tc * k : 0u;
         const uint32_t wpre = wave_prefix(want), ipre = wave_prefix(tc);
         if (lane == WAVE - 1) {
             wsum[wave][0] = wpre;
@@ -421,7 +420,6 @@ __global__ __launch_bounds__(256) void near_plan_kernel(FmmParams F, uint32_t nu
         __syncthreads();
         // uncut items from 0 on; the items of a cut leaf stand beside its slots
         const uint32_t s0 = (uint32_t)(first >> 32) + wb, i0 = (uint32_t)first + ib;
-        if (want && (unsigned long long)s0 + want > F.near_slot_cap) k = 1;
         if (t < num_leaves) {
             F.near_k[A] = k;
             F.near_first[A] = s0;
@@ -435,9 +433,6 @@ __global__ __launch_bounds__(256) void near_plan_kernel(FmmParams F, uint32_t nu
                     F.near_items[s0 + c * k + j] = NearItem{A, c * WAVE, b0, b1, s0 + c * k + j, {0, 0, 0}};
                 }
             }
-            // slots that this leaf asked for beyond the last: nothing to do
-            if (want && k == 1)
-                for (uint32_t j = s0; j < F.near_slot_cap; ++j) F.near_items[j] = NearItem{A, 0, 0, 0, NO_SLOT, {0, 0, 0}};
         }
         __syncthreads();
     }

@@ -116,13 +116,8 @@ struct alignas(16) NearItem {
     uint32_t slot;
     uint32_t pad[3];
 };
-// Batches that an evaluation's lists are cut towards, and the most slots
-// (1 KiB each): the items of a split leaf hold more than half of
-// (batches / NEAR_BATCHES) batches each, so that they stay below NEAR_SLOTS
-// (a leaf that finds no slot left is not split).  The items of split leaves
-// stand at the index of their slot, those of the others from the slot
-// capacity on.
-constexpr uint32_t NEAR_BATCHES = 16384, NEAR_SLOTS = 2 * NEAR_BATCHES;
+// (how lists are cut: rules.h.  The items of cut leaves stand at the index of
+// their slot, those of the others from the slot capacity on.)
 
 // ---- particle state in sorted order (FP64 positions/velocities)
 struct State {

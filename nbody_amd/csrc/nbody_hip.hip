@@ -234,13 +234,14 @@ __global__ __launch_bounds__(WAVE) void sum_totals_kernel(Counters* C) {
     static_assert(CNT_COPIES == WAVE, "one copy per lane");
     const LineTotals& t = C->tot[threadIdx.x];
     const unsigned long long m2l = wave_sum(t.m2l), p2p = wave_sum(t.p2p), inter = wave_sum(t.p2p_inter);
-    const unsigned long long split = wave_sum(t.split), m2lx = wave_sum(t.m2lx);
+    const unsigned long long split = wave_sum(t.split), m2lx = wave_sum(t.m2lx), near = wave_sum(t.near_work);
     if (threadIdx.x == 0) {
         C->m2l_total = m2l;
         C->p2p_total = p2p;
         C->p2p_inter = inter;
         C->split_total = split;
         C->m2lx_total = m2lx;
+        C->near_work = near;
     }
 }
 
@@ -308,8 +309,8 @@ int validate_config(const nbh_config* c, std::string& why) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// partial-sum slots of a handle (1 KiB each): NEAR_SLOTS, fewer for a small
-// system, whose lists have fewer batches
+// the most partial-sum slots (1 KiB each) of an evaluation: NEAR_SLOTS, fewer
+// for a small system, whose lists have fewer batches
 static uint32_t near_slot_cap(const nbh_handle* h) {
     return (uint32_t)std::min<size_t>(NEAR_SLOTS, std::max<size_t>(4 * h->n, 1024));
 }
@@ -318,6 +319,16 @@ static uint32_t near_slot_cap(const nbh_handle* h) {
 static uint32_t near_grid_items(const nbh_handle* h, uint64_t leaves, uint64_t entries) {
     const uint64_t cut = std::min<uint64_t>(near_slot_cap(h), 2 * (entries / 64 + leaves));
     return (uint32_t)std::min<uint64_t>(leaves + h->n / 64 + cut, 1u << 24);
+}
+
+// the slots of the evaluation whose walk has just been read back (with room
+// for the next ones to need a few more)
+static int ensure_near_slots(nbh_handle* h) {
+    const uint32_t cap = near_slot_cap(h);
+    const uint64_t need = near_slots_bound(h->hc->p2p_total, h->hc->near_work, cap);
+    if (h->near_part.bytes >= need * 1024) return NBH_OK;
+    HIPCHK(h, h->near_part.ensure(std::min<uint64_t>(need + need / 4, cap) * 1024));
+    return NBH_OK;
 }
 
 static int alloc_nodes(nbh_handle* h, uint32_t need) {
@@ -338,7 +349,6 @@ static int alloc_nodes(nbh_handle* h, uint32_t need) {
     HIPCHK(h, h->near_first.ensure((size_t)cap * 4));
     // items: every leaf's target chunks, and the slots of the leaves that are cut
     HIPCHK(h, h->near_items.ensure((std::min<size_t>(cap, h->n) + h->n / 64 + near_slot_cap(h)) * sizeof(NearItem)));
-    HIPCHK(h, h->near_part.ensure((size_t)near_slot_cap(h) * 1024));
     HIPCHK(h, h->scan_tmp.ensure(scan_tmp_bytes(cap + 1) + 256));
     h->node_cap = cap;
     return NBH_OK;
@@ -859,6 +869,7 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
     em.T = T;
     CHK(run_walk(h, &em, gs, &side));
     record(h, 2);
+    if (!gs && !for_vjp && h->cfg.p2p == NBH_P2P_LANE) CHK(ensure_near_slots(h));
     F = fmm_params(h);
     if (tables) {
         copy_tables(F, T);
@@ -1069,6 +1080,7 @@ static int graph_prepare(nbh_handle* h) {
     HIPCHK(h, h->xtab.ensure((size_t)E * E * E * g.depth_cap * dcp * 4 * h->nsys));
     HIPCHK(h, h->far_src.ensure((size_t)g.far_cap * 4));
     HIPCHK(h, h->far_tgt.ensure((size_t)g.far_cap * 4));
+    HIPCHK(h, h->near_part.ensure((size_t)near_slot_cap(h) * 1024));
     HIPCHK(h, h->gsnap.ensure(h->n * 48));
     return NBH_OK;
 }
@@ -1835,6 +1847,7 @@ static int vjp_device(nbh_handle* h, const double* w_dev) {
     HIPCHK(h, h->pw.ensure(n * 16));
     HIPCHK(h, h->gbuf.ensure(n * 32));
     FmmParams F = h->lastF;
+    CHK(ensure_near_slots(h));
     set_near(h, F);
     FmmParams Fw = F;
     Fw.M = h->Mw.as<float>();

@@ -16,7 +16,7 @@ struct NearCount {
 __device__ __forceinline__ NearCount near_count(const FmmParams& F) {
     if (F.C->overflow & OVF_WALK) return NearCount{0, 0};
     const unsigned long long u = F.C->near_used;
-    return NearCount{min((uint32_t)(u >> 32), F.near_slot_cap), (uint32_t)u};
+    return NearCount{(uint32_t)(u >> 32), (uint32_t)u};
 }
 __device__ __forceinline__ NearItem near_item(const FmmParams& F, const NearCount& c, uint32_t w) {
     return F.near_items[w < c.cut ? w : F.near_slot_cap + (w - c.cut)];

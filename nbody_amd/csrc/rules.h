@@ -48,4 +48,26 @@ inline PoolSizes pool_guess(uint32_t nodes, uint32_t max_sys_n, uint64_t n, int 
     return {pool(1024.0, 256.0, POOL_CHUNK_M), pool(256.0, 64.0, POOL_CHUNK_P)};
 }
 
+// Near field: batches (of up to 64 entries of a row of a P2P list) that a list
+// is cut towards, and the most partial-sum slots.  A leaf of nb batches and tc
+// chunks of 64 targets is cut if nb > G, into k = ceil(nb / G) items a chunk,
+// and takes tc k slots.  G keeps an item near 1 / NEAR_BATCHES of all batches
+// (entries / 64), and the slots of every leaf within `slots` whatever the
+// lists: with work = the sum of tc nb over the leaves, G = 1 takes at most work
+// slots, and G > 1 at most 2 work / (G + 1), since k <= 2 nb / (G + 1) for nb >
+// G.  So which lists are cut depends on the tree and the lists alone.
+constexpr uint32_t NEAR_BATCHES = 16384, NEAR_SLOTS = 2 * NEAR_BATCHES;
+constexpr uint32_t NEAR_WHOLE = 0x7fffffffu;  // more batches than any list has
+constexpr uint32_t near_item_batches(uint64_t entries, uint64_t work, uint32_t slots) {
+    const uint64_t by_size = (entries / 64 + NEAR_BATCHES - 1) / NEAR_BATCHES;
+    const uint64_t by_slots = (2 * work + slots - 1) / slots;  // G + 1
+    const uint64_t g = by_slots > by_size + 1 ? by_slots - 1 : by_size;
+    return (uint32_t)(g < 1 ? 1 : g > NEAR_WHOLE ? NEAR_WHOLE : g);
+}
+// at least the slots that are then taken
+constexpr uint64_t near_slots_bound(uint64_t entries, uint64_t work, uint32_t slots) {
+    const uint64_t g = near_item_batches(entries, work, slots);
+    return g == 1 ? work : g == NEAR_WHOLE ? 0 : 2 * work / (g + 1);
+}
+
 }  // namespace nbh

@@ -149,6 +149,9 @@ __device__ __forceinline__ uint32_t pool_take(uint2& ch, uint32_t n, uint32_t ch
     return r;
 }
 
+// 64-target chunks of a leaf
+__device__ __forceinline__ uint32_t target_chunks(int4 link) { return ((uint32_t)link.y + WAVE - 1) / WAVE; }
+
 // Depth 0: one row per root (one per system), the candidate being the root
 // itself: a childless root is its own P2P source, otherwise (root, root) is
 // split.  One thread per root.
@@ -186,6 +189,7 @@ __global__ __launch_bounds__(64) void walk_root_kernel(WalkParams W) {
                 W.p2p_pool[ps] = A;
                 pc = 1;
                 atomicAdd(&C->tot[0].p2p, 1ull);
+                atomicAdd(&C->tot[0].near_work, (unsigned long long)target_chunks(W.nodes.link[A]));
             } else {
                 atomicOr(&C->overflow, (uint32_t)OVF_P2P);
                 ps = 0;
@@ -306,7 +310,8 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
     chunk.x = (W.first_block + blockIdx.x) * pool_chunk;
     chunk.y = chunk.x + pool_chunk;
     if (chunk.y > pool_cap) chunk = make_uint2(0, 0);
-    unsigned long long acc = 0;  // totals, lanes 0..3 of the first wavefront: M2L, P2P, split, M2L of other levels
+    // totals, lanes 0..4 of the first wavefront: M2L, P2P, split, M2L of other levels, near-field work
+    unsigned long long acc = 0;
     for (uint64_t j0 = 0; (uint64_t)blockIdx.x + j0 * nblk < n_groups; j0 += WAVE) {
         // headers of the next 64 rows of this workgroup (identical in every wavefront)
         const uint64_t gl = (uint64_t)blockIdx.x + (j0 + lane) * nblk;
@@ -335,9 +340,10 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
             const int nch = gpw >> 8;
             int nt, A0;
             uint32_t row0 = 0;
+            const int4 lp = W.nodes.link[P];
             if (nch > 0) {  // the cell's children: level-s rows in id order
                 nt = nch;
-                A0 = W.nodes.link[P].z;
+                A0 = lp.z;
                 row0 = base + (uint32_t)(A0 - (int)loff);
             } else {  // a leaf with sources left to split: carried to depth s (its row is taken below)
                 nt = 1;
@@ -372,17 +378,20 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
             };
             // targets: lane o < 8 holds the child of octant o (of a carried leaf,
             // lane 0 the leaf): its index among the children, which are in
-            // octant order, and whether it is a leaf
-            int tgt = 0;  // index | leaf << 3 | present << 4
+            // octant order, whether it is a leaf, and its 64-target chunks
+            int tgt = 0;  // index | leaf << 3 | present << 4 | chunks << 5
             if (nch > 0) {
-                int4 gt = make_int4(0, 0, 0, 0);
-                if (lane < nt) gt = W.nodes.geo[A0 + lane];
+                int4 gt = make_int4(0, 0, 0, 0), lk = make_int4(0, 0, 0, 0);
+                if (lane < nt) {
+                    gt = W.nodes.geo[A0 + lane];
+                    lk = W.nodes.link[A0 + lane];
+                }
                 const int oct = (gt.x & 1) << 2 | (gt.y & 1) << 1 | (gt.z & 1);
                 // (lanes without a child push past the octants)
                 tgt = __builtin_amdgcn_ds_permute((lane < nt ? oct : 8 + (lane & 31)) << 2,
-                                                  lane | ((gt.w >> 8) == 0) << 3 | 1 << 4);
+                                                  lane | ((gt.w >> 8) == 0) << 3 | 1 << 4 | target_chunks(lk) << 5);
             } else {
-                tgt = 1 << 3 | 1 << 4;
+                tgt = 1 << 3 | 1 << 4 | target_chunks(lp) << 5;
             }
             const bool pres_l = lane < (nch > 0 ? MAXT : 1) && (tgt >> 4 & 1);
             const bool leaf_l = tgt >> 3 & 1;
@@ -528,6 +537,10 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
                     // 0..2 of the first wavefront, a pool each) and a carried leaf's
                     // row (lane 3): the atomics go out together
                     if (wv == 0) {
+                        // (only leaves have P2P entries)
+                        unsigned long long near = (unsigned long long)((uint32_t)tgt >> 5) * ((T.p + WAVE - 1) / WAVE);
+#pragma unroll
+                        for (int o = 1; o < MAXT; o <<= 1) near += __shfl_xor(near, o, WAVE);
                         const uint32_t need = lane == 0 ? tm : lane == 1 ? tp : lane == 2 ? ts : 0u;
                         const uint32_t ovf = lane == 0 ? OVF_M2L : lane == 1 ? OVF_P2P : OVF_SL;
                         uint32_t at = 0;
@@ -543,7 +556,7 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
                             }
                         }
                         const bool fail = __ballot(lane < 4 && at == 0xffffffffu) != 0;
-                        if (!fail) acc += lane == 3 ? tx : need;
+                        if (!fail) acc += lane == 3 ? tx : lane == 4 ? near : need;
                         if (lane < 4) bcast[lane] = at;
                         if (lane == 4) bcast[4] = fail;
                     }
@@ -585,9 +598,14 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
             }
         }
     }
-    if (threadIdx.x < 4 && acc) {
+    if (threadIdx.x < 5 && acc) {
         LineTotals& tot = C->tot[blockIdx.x % CNT_COPIES];
-        atomicAdd(lane == 0 ? &tot.m2l : lane == 1 ? &tot.p2p : lane == 2 ? &tot.split : &tot.m2lx, acc);
+        atomicAdd(lane == 0   ? &tot.m2l
+                  : lane == 1 ? &tot.p2p
+                  : lane == 2 ? &tot.split
+                  : lane == 3 ? &tot.m2lx
+                              : &tot.near_work,
+                  acc);
     }
 }
 

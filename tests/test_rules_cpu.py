@@ -4,6 +4,7 @@ import os
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -20,6 +21,8 @@ void pool_sizes(uint32_t nodes, uint32_t max_sys_n, uint64_t n, int num, int den
     out[0] = s.m2l;
     out[1] = s.p2p;
 }
+uint32_t item_batches(uint64_t entries, uint64_t work, uint32_t slots) { return near_item_batches(entries, work, slots); }
+uint64_t slots_bound(uint64_t entries, uint64_t work, uint32_t slots) { return near_slots_bound(entries, work, slots); }
 }
 """
 
@@ -31,7 +34,10 @@ def rules(tmp_path_factory):
     so = d / "librules.so"
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC",
                     "-I" + os.path.join(ROOT, "nbody_amd", "csrc"), str(d / "shim.cpp"), "-o", str(so)], check=True)
-    return ctypes.CDLL(str(so))
+    lib = ctypes.CDLL(str(so))
+    lib.item_batches.argtypes = lib.slots_bound.argtypes = [ctypes.c_uint64, ctypes.c_uint64, ctypes.c_uint32]
+    lib.item_batches.restype, lib.slots_bound.restype = ctypes.c_uint32, ctypes.c_uint64
+    return lib
 
 
 CHUNK_M, CHUNK_P, POOL_MAX = 2048, 512, 0xFFFF0000
@@ -81,3 +87,40 @@ def test_pools_at_small_theta(rules):
                 assert h <= g <= max(h, 1 << 29)
                 assert g == max(h, min(1 << 29, nodes * min(nodes, usual * den**3 // 8))) or den % 2
             assert _pools(rules, nodes, 1, den, 0, max_sys_n=10 * nodes, small=True) == (nodes * 256, nodes * 64)
+
+
+def _slots(nb, tc, g):
+    """Slots of leaves of nb batches and tc chunks of targets, cut at g."""
+    return int(np.where(nb > g, tc * -(-nb // g), 0).sum())
+
+
+@pytest.mark.parametrize("slots", [1024, 6148, 32768])
+def test_near_field_slots_suffice(rules, slots):
+    """No lists ask for more slots than there are, nor than the bound that they
+    are allocated by; lists short of it are cut to single batches."""
+    rng = np.random.default_rng(slots)
+    for trial in range(400):
+        leaves = int(10 ** rng.uniform(0, 5))
+        rows = rng.integers(1, 6, leaves)
+        entries = np.ceil(10 ** rng.uniform(0, rng.uniform(0.5, 4.5), leaves)).astype(np.int64)
+        nb = rows - 1 + -(-entries // 64)  # rows of a list are rounded up on their own
+        tc = np.ceil(2 ** rng.uniform(0, rng.choice([0.01, 1, 5, 15]), leaves)).astype(np.int64)
+        work = int((tc * nb).sum())
+        g = rules.item_batches(int(entries.sum()), work, slots)
+        used = _slots(nb, tc, g)
+        assert used <= rules.slots_bound(int(entries.sum()), work, slots) <= max(slots, 0)
+        if work <= slots and entries.sum() <= 64 * 16384:
+            assert g == 1
+    # a leaf at the depth limit that holds a million particles, and the largest work
+    for tc, nb in ((1 << 14, 1 << 14), (1 << 25, 1 << 25)):
+        work = tc * nb
+        g = rules.item_batches(64 * nb, work, slots)
+        assert (tc * -(-nb // g) if nb > g else 0) <= rules.slots_bound(64 * nb, work, slots) <= slots
+
+
+def test_large_leaves_asked_for_more_slots_than_there_are(rules):
+    """512 leaves of 10 chunks with 8 batches: 40,960 slots when the cut looked
+    at the entries alone."""
+    nb, tc = np.full(512, 8), np.full(512, 10)
+    assert _slots(nb, tc, 1) > 32768
+    assert _slots(nb, tc, rules.item_batches(64 * 8 * 512, int((nb * tc).sum()), 32768)) <= 32768
