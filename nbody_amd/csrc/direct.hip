@@ -131,6 +131,59 @@ __global__ __launch_bounds__(WAVE * DS_WAVES) void direct_f32_kernel(State S, co
     }
 }
 
+// The same sums with one thread per target that does all of a pair's work,
+// source tiles in LDS: about 12 issue slots a pair where the pipeline takes 20,
+// once there are targets enough to fill the GPU with (direct_by_pipeline).
+constexpr int DT_THREADS = 256;
+template <bool NORMAL>
+__global__ __launch_bounds__(DT_THREADS) void direct_thread_kernel(State S, const uint32_t* __restrict__ sys_off,
+                                                                   const double4* __restrict__ box, float G,
+                                                                   float eps2, double kick_dt) {
+    __shared__ float4 tile[DT_THREADS];
+    const uint32_t b = sys_off[blockIdx.y], e = sys_off[blockIdx.y + 1];
+    const uint32_t i = b + blockIdx.x * DT_THREADS + threadIdx.x;
+    if (b + blockIdx.x * DT_THREADS >= e) return;
+    const double4 bx = box[blockIdx.y];
+    const double h = 0.5 * bx.w, cx = bx.x + h, cy = bx.y + h, cz = bx.z + h;
+    const bool valid = i < e;
+    auto offset = [&](uint32_t j) {
+        return make_float4((float)(S.x[j] - cx), (float)(S.y[j] - cy), (float)(S.z[j] - cz), (float)S.charge[j]);
+    };
+    const float4 me = offset(valid ? i : e - 1);
+    float ax = 0.f, ay = 0.f, az = 0.f, ph = 0.f;
+    for (uint32_t j0 = b; j0 < e; j0 += DT_THREADS) {
+        const uint32_t j = j0 + threadIdx.x;
+        __syncthreads();
+        if (j < e) tile[threadIdx.x] = offset(j);
+        __syncthreads();
+        const uint32_t jn = min((uint32_t)DT_THREADS, e - j0);
+        if (!valid) continue;
+        for (uint32_t k = 0; k < jn; ++k) {
+            const float4 q = tile[k];
+            const float rx = q.x - me.x, ry = q.y - me.y, rz = q.z - me.z;
+            const float r2 = fmaf(rx, rx, fmaf(ry, ry, fmaf(rz, rz, eps2)));
+            // the self pair contributes nothing (r2 = 0 when unsoftened)
+            const float inv = j0 + k == i ? 0.f : NORMAL ? __builtin_amdgcn_rsqf(r2) : rsqrtf(r2);
+            const float w = q.w * inv;
+            const float w3 = w * inv * inv;
+            ax = fmaf(rx, w3, ax);
+            ay = fmaf(ry, w3, ay);
+            az = fmaf(rz, w3, az);
+            ph += w;
+        }
+    }
+    if (!valid) return;
+    const float fac = (float)(S.charge[i] / S.mass[i]) * G;
+    ax *= fac; ay *= fac; az *= fac;
+    S.ax[i] = ax; S.ay[i] = ay; S.az[i] = az;
+    S.pot[i] = -G * ph;
+    if (kick_dt != 0.0) {
+        S.vx[i] += (double)ax * kick_dt;
+        S.vy[i] += (double)ay * kick_dt;
+        S.vz[i] += (double)az * kick_dt;
+    }
+}
+
 // The reference's naive force law (compat): separation (dx, dx, dx), no
 // softening (naive_simulation.cpp:10-17), with each pair's term formed as the
 // reference forms it in FP32 (uncentred x difference, r = sqrt(d d + d d +
@@ -181,6 +234,23 @@ __global__ __launch_bounds__(DC_THREADS) void direct_compat_kernel(State S, cons
     }
 }
 
+// The pipeline shortens the chain of each target, the thread-per-target form
+// takes fewer slots a pair: the first wins while there are few targets, in
+// systems large enough to fill and drain its chunks.  Sum kernels, us, pipeline
+// and threads (eps > 0), either side of the line:
+//   size x systems
+//   128 x 1     11.1  9.5     200 x 1      11.0  12.4
+//   200 x 128   14.3 13.3     200 x 64     12.5  13.1
+//   512 x 128   33.6 28.0     512 x 64     20.3  26.8
+//   1000 x 64   52.2 50.7     1000 x 48    39.6  46.2
+//   4096 x 64    612  435     4096 x 20     182   215
+//   65536 x 2   4070 3362     65536 x 1    2092  2732
+//   131072 x 1  8144 6667     90000 x 1    4005  4548
+//   262144 x 1 31960 24905    16384 x 1     174   675
+static bool direct_by_pipeline(uint32_t n, uint32_t max_sys_n) {
+    return max_sys_n >= 192 && n <= std::min<uint64_t>(24576u + 24ull * max_sys_n, 98304u);
+}
+
 void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uint32_t* sys_off, int nsys,
                        const double4* box, float G, float eps2, int compat_law, double kick_dt, float* pk,
                        hipStream_t st) {
@@ -189,10 +259,19 @@ void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uin
                            S, sys_off, G, kick_dt);
         return;
     }
+    const bool normal = eps2 >= 1.17549435e-38f;
+    if (!direct_by_pipeline(n, max_sys_n)) {
+        const dim3 grid(ceil_div(max_sys_n, DT_THREADS), nsys), block(DT_THREADS);
+        if (normal)
+            hipLaunchKernelGGL(direct_thread_kernel<true>, grid, block, 0, st, S, sys_off, box, G, eps2, kick_dt);
+        else
+            hipLaunchKernelGGL(direct_thread_kernel<false>, grid, block, 0, st, S, sys_off, box, G, eps2, kick_dt);
+        return;
+    }
     hipLaunchKernelGGL(direct_pack_kernel, dim3(ceil_div(n + DS_PAD, 256)), dim3(256), 0, st, S, n, sys_off, nsys, box,
                        pk);
     const dim3 grid(ceil_div(max_sys_n, WAVE), nsys), block(WAVE * DS_WAVES);
-    if (eps2 >= 1.17549435e-38f)
+    if (normal)
         hipLaunchKernelGGL(direct_f32_kernel<true>, grid, block, 0, st, S, pk, n, sys_off, G, eps2, kick_dt);
     else
         hipLaunchKernelGGL(direct_f32_kernel<false>, grid, block, 0, st, S, pk, n, sys_off, G, eps2, kick_dt);

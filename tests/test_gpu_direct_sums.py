@@ -83,3 +83,31 @@ def test_fp64_sums_of_coincident_particles():
     assert pot[0] == -np.inf and np.isnan(acc[0]).any()
     assert acc[1][0] == -2.0 and pot[1] == -2.0
     assert np.all(acc[2] == 0.0) and pot[2] == 0.0
+
+
+# (particles, systems) either side of the rules that choose the kernel: systems
+# of 192 particles, and total targets against 24,576 + 24 size, at most 98,304
+@pytest.mark.parametrize("size,systems", [(191, 1), (192, 1), (191, 7), (192, 151), (192, 152), (257, 3), (8, 1031),
+                                          (1, 65), (40000, 1), (98304, 1), (98305, 1)])
+@pytest.mark.parametrize("eps", [1e-2, 0.0])
+def test_direct_solver_forms(size, systems, eps):
+    rng = np.random.default_rng(size)
+    n = size * systems
+    x, m = rng.standard_normal((n, 3)), rng.uniform(0.5, 1.5, n) / size
+    off = (np.arange(systems + 1) * size).astype(np.uint32)
+    cfg = nb.default_config(solver=nb.SOLVER_DIRECT, eps=eps)
+    with nb.HipSimulation.from_arrays(x, np.zeros_like(x), m, m, config=cfg,
+                                      sys_off=off if systems > 1 else None) as sim:
+        acc, pot = sim.forces()
+        sim.step(1)
+        moved = sim.state()[1]
+    for s in {0, systems // 2, systems - 1}:
+        a, b = size * s, size * (s + 1)
+        t = np.arange(a, b, max(1, size // 61))
+        ar, pr = _sum64(_packed(x[a:b]), m[a:b], eps, t - a)
+        # FP32 terms and sums of n of them in order: n half ulps of the largest partial sum
+        tol = 2e-5 if size < 5000 else 1e-4
+        assert np.max(np.abs(acc[t] - ar)) <= tol * np.abs(ar).max() + 1e-30
+        assert np.max(np.abs(pot[t] - pr)) <= tol * np.abs(pr).max() + 1e-30
+    # v after a step of dt from rest, to first order (the closing kick reaches every system)
+    assert np.all(np.isfinite(moved)) and (size == 1 or np.all(np.any(moved != 0.0, axis=1)))
