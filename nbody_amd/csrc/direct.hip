@@ -10,29 +10,35 @@ namespace nbh {
 // ---------------------------------------------------------------------------
 // Direct sum on the GPU (replaces NaiveSimulation::step's O(N^2) loop,
 // naive_simulation.cpp:8-35), softened law: FP32 positions relative to the
-// system's box centre, packed once: x, y, z and charge in arrays of n + DS_PAD
-// (zeros past the particles).
+// system's box centre, packed once: x, y, z and charge in arrays in which every
+// system is followed by DS_PAD zeros, so that a chunk past its end reads no
+// other system's values (which may overflow FP32, and 0 times infinity is NaN).
 __global__ void direct_pack_kernel(State S, uint32_t n, const uint32_t* sys_off, int nsys, const double4* box,
                                    float* pk) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t m = (size_t)n + DS_PAD;
-    if (i >= m) return;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t m = direct_pack_len(n, nsys);
+    if (t >= m) return;
+    uint32_t at;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i < n) {
+    if (t < n) {
         int lo = 0, hi = nsys - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
-            if (sys_off[mid] <= i) lo = mid; else hi = mid - 1;
+            if (sys_off[mid] <= t) lo = mid; else hi = mid - 1;
         }
         const double4 bx = box[lo];
         const double h = 0.5 * bx.w;
-        v = make_float4((float)(S.x[i] - (bx.x + h)), (float)(S.y[i] - (bx.y + h)), (float)(S.z[i] - (bx.z + h)),
-                        (float)S.charge[i]);
+        v = make_float4((float)(S.x[t] - (bx.x + h)), (float)(S.y[t] - (bx.y + h)), (float)(S.z[t] - (bx.z + h)),
+                        (float)S.charge[t]);
+        at = t + lo * DS_PAD;
+    } else {
+        const uint32_t s = (t - n) / DS_PAD;
+        at = sys_off[s + 1] + (t - n);
     }
-    pk[i] = v.x;
-    pk[m + i] = v.y;
-    pk[2 * m + i] = v.z;
-    pk[3 * m + i] = v.w;
+    pk[at] = v.x;
+    pk[m + at] = v.y;
+    pk[2 * m + at] = v.z;
+    pk[3 * m + at] = v.w;
 }
 
 // One workgroup per 64 targets (one per lane).  Each target's force is one
@@ -52,7 +58,7 @@ __global__ void direct_pack_kernel(State S, uint32_t n, const uint32_t* sys_off,
 constexpr int DS_PROD = 13, DS_PER = 8, DS_CH = DS_PROD * DS_PER, DS_WAVES = DS_PROD + 3;
 static_assert(DS_PAD >= DS_CH, "a chunk past the particles reads the padding");
 template <bool NORMAL>
-__global__ __launch_bounds__(WAVE * DS_WAVES) void direct_f32_kernel(State S, const float* __restrict__ pk, uint32_t n,
+__global__ __launch_bounds__(WAVE * DS_WAVES) void direct_f32_kernel(State S, const float* __restrict__ pk, uint32_t m,
                                                                      const uint32_t* __restrict__ sys_off, float G,
                                                                      float eps2, double kick_dt) {
     __shared__ float4 w3s[2][DS_CH / 4][WAVE];  // q / r^3 of four sources
@@ -63,11 +69,13 @@ __global__ __launch_bounds__(WAVE * DS_WAVES) void direct_f32_kernel(State S, co
     const int lane = lane_id();
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const uint32_t i = i0 + lane, it = min(i, e - 1);
-    const size_t m = (size_t)n + DS_PAD;
+    // (m: the arrays' length, in 32 bits: with 64-bit strides the kernel took half
+    // as long again at N = 65,536)
+    const uint32_t pad = blockIdx.y * DS_PAD;  // the system's particles stand so much further on
     const uint32_t nch = (e - b + DS_CH - 1) / DS_CH;
     if (wv < 3) {  // consumers: component wv
-        const float* src = pk + wv * m + b;
-        const float me = pk[wv * m + it];
+        const float* src = pk + wv * m + (b + pad);
+        const float me = pk[wv * m + it + pad];
         float acc = 0.f;
         for (uint32_t c = 0; c <= nch; ++c) {
             if (c > 0) {
@@ -86,12 +94,12 @@ __global__ __launch_bounds__(WAVE * DS_WAVES) void direct_f32_kernel(State S, co
         part[DS_PROD + wv][lane] = acc;
     } else {
         const int pw = wv - 3;
-        const float px = pk[it], py = pk[m + it], pz = pk[2 * m + it];
+        const float px = pk[it + pad], py = pk[m + it + pad], pz = pk[2 * m + it + pad];
         float ph = 0.f;
         for (uint32_t c = 0; c <= nch; ++c) {
             if (c < nch) {
                 const uint32_t j0 = b + c * DS_CH + pw * DS_PER;  // uniform
-                const float *sx = pk + j0, *sy = sx + m, *sz = sy + m, *sq = sz + m;
+                const float *sx = pk + (j0 + pad), *sy = sx + m, *sz = sy + m, *sq = sz + m;
                 float w3[DS_PER];
                 auto pairs = [&](auto&& skip) {
 #pragma unroll
@@ -247,8 +255,12 @@ __global__ __launch_bounds__(DC_THREADS) void direct_compat_kernel(State S, cons
 //   65536 x 2   4070 3362     65536 x 1    2092  2732
 //   131072 x 1  8144 6667     90000 x 1    4005  4548
 //   262144 x 1 31960 24905    16384 x 1     174   675
-static bool direct_by_pipeline(uint32_t n, uint32_t max_sys_n) {
-    return max_sys_n >= 192 && n <= std::min<uint64_t>(24576u + 24ull * max_sys_n, 98304u);
+// (every system has a workgroup, also one of few particles)
+static bool direct_by_pipeline(uint32_t n, uint32_t max_sys_n, int nsys) {
+    return max_sys_n >= 192 && n <= std::min<uint64_t>(24576u + 24ull * max_sys_n, 98304u) && nsys <= 512;
+}
+size_t direct_pack_bytes(uint32_t n, uint32_t max_sys_n, int nsys) {
+    return direct_by_pipeline(n, max_sys_n, nsys) ? 16 * (size_t)direct_pack_len(n, nsys) : 0;
 }
 
 void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uint32_t* sys_off, int nsys,
@@ -260,7 +272,7 @@ void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uin
         return;
     }
     const bool normal = eps2 >= 1.17549435e-38f;
-    if (!direct_by_pipeline(n, max_sys_n)) {
+    if (!direct_by_pipeline(n, max_sys_n, nsys)) {
         const dim3 grid(ceil_div(max_sys_n, DT_THREADS), nsys), block(DT_THREADS);
         if (normal)
             hipLaunchKernelGGL(direct_thread_kernel<true>, grid, block, 0, st, S, sys_off, box, G, eps2, kick_dt);
@@ -268,13 +280,13 @@ void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uin
             hipLaunchKernelGGL(direct_thread_kernel<false>, grid, block, 0, st, S, sys_off, box, G, eps2, kick_dt);
         return;
     }
-    hipLaunchKernelGGL(direct_pack_kernel, dim3(ceil_div(n + DS_PAD, 256)), dim3(256), 0, st, S, n, sys_off, nsys, box,
-                       pk);
+    const uint32_t m = direct_pack_len(n, nsys);
+    hipLaunchKernelGGL(direct_pack_kernel, dim3(ceil_div(m, 256)), dim3(256), 0, st, S, n, sys_off, nsys, box, pk);
     const dim3 grid(ceil_div(max_sys_n, WAVE), nsys), block(WAVE * DS_WAVES);
     if (normal)
-        hipLaunchKernelGGL(direct_f32_kernel<true>, grid, block, 0, st, S, pk, n, sys_off, G, eps2, kick_dt);
+        hipLaunchKernelGGL(direct_f32_kernel<true>, grid, block, 0, st, S, pk, m, sys_off, G, eps2, kick_dt);
     else
-        hipLaunchKernelGGL(direct_f32_kernel<false>, grid, block, 0, st, S, pk, n, sys_off, G, eps2, kick_dt);
+        hipLaunchKernelGGL(direct_f32_kernel<false>, grid, block, 0, st, S, pk, m, sys_off, G, eps2, kick_dt);
 }
 
 // ---------------------------------------------------------------------------

@@ -267,8 +267,10 @@ void launch_m2l_parts(int p, int q, const FmmParams& F, const M2LPlan& plan, int
 void launch_integrate(const State& S, uint32_t n, int mode, double dt_k, double dt_d, hipStream_t st);
 
 // direct sums
-// (direct.hip) pk: scratch, 4 (n + DS_PAD) floats
+// (direct.hip) pk: scratch of direct_pack_bytes
 constexpr uint32_t DS_PAD = 128;
+__host__ __device__ constexpr uint32_t direct_pack_len(uint32_t n, int nsys) { return n + nsys * DS_PAD; }
+size_t direct_pack_bytes(uint32_t n, uint32_t max_sys_n, int nsys);
 void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uint32_t* sys_off, int nsys,
                        const double4* box, float G, float eps2, int compat_law, double kick_dt, float* pk,
                        hipStream_t st);

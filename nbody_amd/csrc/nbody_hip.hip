@@ -1359,7 +1359,7 @@ static int create_impl(const nbh_config* cfg, size_t nsys, const uint32_t* sys_o
     CCHK(h->unit.ensure(nsys * 4));
     CCHK(h->bbox_part.ensure(bbox_part_bytes(h->max_sys_n, (int)nsys)));
     CCHK(h->leaf_ids.ensure(n * 4));
-    CCHK(h->pf.ensure((n + DS_PAD) * 16));
+    CCHK(h->pf.ensure(std::max(n * 16, direct_pack_bytes((uint32_t)n, h->max_sys_n, (int)nsys))));
     CCHK(h->pleaf.ensure(n * 4));
     CCHK(h->counters.ensure(sizeof(Counters)));
     CCHK(h->diag.ensure(1024 * 8 * 8));

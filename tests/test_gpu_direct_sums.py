@@ -111,3 +111,41 @@ def test_direct_solver_forms(size, systems, eps):
         assert np.max(np.abs(pot[t] - pr)) <= tol * np.abs(pr).max() + 1e-30
     # v after a step of dt from rest, to first order (the closing kick reaches every system)
     assert np.all(np.isfinite(moved)) and (size == 1 or np.all(np.any(moved != 0.0, axis=1)))
+
+
+@pytest.mark.parametrize("what", ["charge", "position"])
+@pytest.mark.parametrize("size", [192, 200, 208, 311])
+def test_direct_solver_keeps_systems_apart(size, what):
+    """A system beside one whose values overflow FP32 has the forces that it has alone."""
+    rng = np.random.default_rng(size)
+    x, m = rng.standard_normal((2 * size, 3)), rng.uniform(0.5, 1.5, 2 * size)
+    cfg = nb.default_config(solver=nb.SOLVER_DIRECT, eps=1e-2)
+    with nb.HipSimulation.from_arrays(x[:size], 0 * x[:size], m[:size], m[:size], config=cfg) as sim:
+        alone = sim.forces()
+    if what == "charge":
+        m[size:] = 1e39
+    else:
+        x[size:] *= 1e39
+    with nb.HipSimulation.from_arrays(x, 0 * x, m, m, config=cfg, sys_off=np.array([0, size, 2 * size])) as sim:
+        acc, pot = sim.forces()
+    assert np.array_equal(acc[:size], alone[0]) and np.array_equal(pot[:size], alone[1])
+
+
+@pytest.mark.parametrize("small", [510, 511, 512])
+def test_direct_solver_many_small_systems(small):
+    """A system among many of two particles, 511 to 513 in all."""
+    rng = np.random.default_rng(small)
+    size = np.array([2] * (small // 2) + [333] + [2] * (small - small // 2))
+    off = np.concatenate([[0], np.cumsum(size)])
+    n, a = int(off[-1]), int(off[small // 2])
+    x, m = rng.standard_normal((n, 3)), rng.uniform(0.5, 1.5, n)
+    cfg = nb.default_config(solver=nb.SOLVER_DIRECT, eps=1e-2)
+    with nb.HipSimulation.from_arrays(x[a:a + 333], 0 * x[a:a + 333], m[a:a + 333], m[a:a + 333], config=cfg) as sim:
+        alone = sim.forces()[0]
+    with nb.HipSimulation.from_arrays(x, 0 * x, m, m, config=cfg, sys_off=off) as sim:
+        acc = sim.forces()[0]
+    assert np.array_equal(acc[a:a + 333], alone)
+    for i in range(20):
+        j = i ^ 1
+        ar, _ = _sum64(_packed(x[[i, j]]), m[[i, j]], 1e-2, [0])
+        assert np.max(np.abs(acc[i] - ar[0])) <= 2e-5 * np.abs(ar).max()
