@@ -124,8 +124,8 @@ constexpr int rs_len(int n, int s) {
 // the S steps v[0, rs_len(N, S)) of a lane holds group sums; rs_slot names
 // which.  It takes sum(rs_len(N, 1..S)) shuffles where a sum per value
 // (wave_sum) takes N S.
-template <int N, int S>
-__device__ __forceinline__ void group_reduce_scatter(float* v) {
+template <int N, int S, typename T>
+__device__ __forceinline__ void group_reduce_scatter(T* v) {
     const int lane = __lane_id();
 #pragma unroll
     for (int t = 0; t < S; ++t) {
@@ -134,7 +134,7 @@ __device__ __forceinline__ void group_reduce_scatter(float* v) {
         const bool up = (lane >> b) & 1;
 #pragma unroll
         for (int i = 0; i < h; ++i) {
-            const float lo = v[i], hi = h + i < n ? v[h + i] : 0.f;
+            const T lo = v[i], hi = h + i < n ? v[h + i] : T(0);
             v[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, 1 << b, WAVE);
         }
     }

@@ -290,25 +290,26 @@ void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uin
 }
 
 // ---------------------------------------------------------------------------
-// FP64 direct sum for selected targets (sorted slots).  A workgroup takes T
-// targets; its 8 wavefronts stride over the sources with one source per lane,
-// so each source is loaded once for T targets (one target per wavefront read
-// 32 bytes per pair from L2, 12 TB/s at 262,144 sources x 4096 targets, which
-// bound it).  1/r is v_rsq_f64 (relative error e/2 ~ 2^-27) and one third-order
-// step y (1 + e/2 + 3/8 e^2), e = 1 - r^2 y^2, whose remainder ~e^3 is below
-// the rounding; 1/sqrt took ~50 instructions of the pair's ~70.  262,144 x
-// 4096: 2.7 -> 1.0 ms, of 0.68 ms that the pairs' FP64 instructions take.
+// FP64 direct sum for selected targets (sorted slots).  NW of a workgroup's 8
+// wavefronts take T targets together and stride over the sources with one
+// source per lane, so that each source is loaded once for T targets (one
+// target per wavefront read 32 bytes per pair from L2, 12 TB/s at 262,144
+// sources x 4096 targets, which bound it).  1/r is v_rsq_f64 (relative error
+// e/2 ~ 2^-27) and one third-order step y (1 + e/2 + 3/8 e^2), e = 1 - r^2 y^2,
+// whose remainder ~e^3 is below the rounding; 1/sqrt took ~50 instructions of
+// the pair's ~70.  262,144 x 4096: 2.5 -> 1.06 ms, of 0.68 ms that the pairs'
+// FP64 instructions take.
 constexpr int DD_WAVES = 8;
-template <int T>
+template <int T, int NW>
 __global__ __launch_bounds__(WAVE * DD_WAVES) void direct_fp64_kernel(State S, const uint32_t* __restrict__ sys_off,
                                                                       int nsys, const uint32_t* __restrict__ targets,
                                                                       uint32_t nt, double G, double eps2, double* acc,
                                                                       double* pot) {
     __shared__ double part[DD_WAVES][T][4];
-    const uint32_t w0 = blockIdx.x * T;
-    const uint32_t n = sys_off[nsys];
-    const uint32_t wv = threadIdx.x / WAVE;
     const int lane = lane_id();
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t w0 = (blockIdx.x * (DD_WAVES / NW) + wv / NW) * T;  // the group's targets
+    const uint32_t n = sys_off[nsys];
     uint32_t id[T];
     double px[T], py[T], pz[T], a[T][4];
 #pragma unroll
@@ -328,7 +329,8 @@ __global__ __launch_bounds__(WAVE * DD_WAVES) void direct_fp64_kernel(State S, c
         b = sys_off[lo];
         e = sys_off[lo + 1];
     }
-    for (uint32_t j = b + wv * WAVE + lane; j < e; j += WAVE * DD_WAVES) {
+    if (w0 >= nt) e = b;
+    for (uint32_t j = b + (wv % NW) * WAVE + lane; j < e; j += WAVE * NW) {
         const double sx = S.x[j], sy = S.y[j], sz = S.z[j], q = S.charge[j];
 #pragma unroll
         for (int t = 0; t < T; ++t) {
@@ -347,41 +349,58 @@ __global__ __launch_bounds__(WAVE * DD_WAVES) void direct_fp64_kernel(State S, c
             a[t][3] += w;
         }
     }
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const double v = wave_sum(a[t][k]);
-            if (lane == 0) part[wv][t][k] = v;
-        }
+    {
+        // (a sum a lane: the 4 T sums one after the other took 24 T shuffles, and
+        // half of the kernel's time at n = 5003)
+        group_reduce_scatter<4 * T, 6>(&a[0][0]);
+        int at, cnt;
+        rs_slot(4 * T, 6, lane, at, cnt);
+        if (cnt > 0) (&part[wv][0][0])[at] = a[0][0];
+    }
     __syncthreads();
-    if (threadIdx.x < 4 * T) {
-        const int t = threadIdx.x / 4, k = threadIdx.x % 4;
-        const uint32_t w = w0 + t;
-        if (w >= nt) return;
+    for (uint32_t v = threadIdx.x; v < 4 * T * (DD_WAVES / NW); v += WAVE * DD_WAVES) {
+        const int g = v / (4 * T), t = v / 4 % T, k = v % 4;
+        const uint32_t w = (blockIdx.x * (DD_WAVES / NW) + g) * T + t;
+        if (w >= nt) continue;
         const uint32_t i = targets[w];
-        double v = 0.0;
-        for (int q = 0; q < DD_WAVES; ++q) v += part[q][t][k];
+        double sum = 0.0;
+        for (int q = 0; q < NW; ++q) sum += part[g * NW + q][t][k];
         // no such particle: report NaN
-        if (k < 3) acc[3 * (size_t)w + k] = i < n ? S.charge[i] / S.mass[i] * G * v : NAN;
-        else pot[w] = i < n ? -G * v : NAN;
+        if (k < 3) acc[3 * (size_t)w + k] = i < n ? S.charge[i] / S.mass[i] * G * sum : NAN;
+        else pot[w] = i < n ? -G * sum : NAN;
     }
 }
 
-void launch_direct_fp64(const State& S, const uint32_t* sys_off, int nsys, const uint32_t* targets, uint32_t nt,
-                        double G, double eps2, double* acc, double* pot, hipStream_t st) {
+template <int T, int NW>
+static void launch_direct_fp64_t(const State& S, const uint32_t* sys_off, int nsys, const uint32_t* targets,
+                                 uint32_t nt, double G, double eps2, double* acc, double* pot, hipStream_t st) {
+    hipLaunchKernelGGL((direct_fp64_kernel<T, NW>), dim3(ceil_div(nt, T * (DD_WAVES / NW))), dim3(WAVE * DD_WAVES), 0,
+                       st, S, sys_off, nsys, targets, nt, G, eps2, acc, pot);
+}
+void launch_direct_fp64(const State& S, uint32_t n, const uint32_t* sys_off, int nsys, const uint32_t* targets,
+                        uint32_t nt, double G, double eps2, double* acc, double* pot, hipStream_t st) {
     if (!nt) return;
-    // eight targets a workgroup where that still leaves two workgroups per
-    // CU; of several systems each target has its own sources
-    if (nsys == 1 && nt >= 4096)
-        hipLaunchKernelGGL(direct_fp64_kernel<8>, dim3(ceil_div(nt, 8)), dim3(WAVE * DD_WAVES), 0, st, S, sys_off,
-                           nsys, targets, nt, G, eps2, acc, pot);
-    else if (nsys == 1 && nt >= 1024)
-        hipLaunchKernelGGL(direct_fp64_kernel<4>, dim3(ceil_div(nt, 4)), dim3(WAVE * DD_WAVES), 0, st, S, sys_off,
-                           nsys, targets, nt, G, eps2, acc, pot);
+    if (nsys == 1) {
+        // eight targets where that leaves two workgroups a CU, four where it
+        // leaves one, us with 1, 4 and 8 at 262,144 sources: 512 targets 244,
+        // 284, 606; 1024 491, 307, 613; 2048 929, 562, 630; 4096 1810, 1047,
+        // 1056; 16,384 7172, 3999, 3871; at 5003 sources: 1024 16, 12, 18;
+        // 4096 45, 29, 29
+        if (nt >= 4096) launch_direct_fp64_t<8, 8>(S, sys_off, nsys, targets, nt, G, eps2, acc, pot, st);
+        else if (nt >= 1024) launch_direct_fp64_t<4, 8>(S, sys_off, nsys, targets, nt, G, eps2, acc, pot, st);
+        else launch_direct_fp64_t<1, 8>(S, sys_off, nsys, targets, nt, G, eps2, acc, pot, st);
+        return;
+    }
+    // of several systems each target has its own sources, and one wavefront
+    // does where there are targets enough and their systems are small, us with
+    // one and eight, size x targets: 8 x 65,536 35, 241; 512 x 4096 11, 20;
+    // 2048 x 2048 14, 16; 2048 x 1024 13, 11; 1000 x 1024 9.4, 9.0; 8192 x 8192
+    // 133, 122; 40,000 x 2048 245, 151
+    const uint32_t mean = n / (uint32_t)nsys;
+    if (nt >= 1024 && mean <= (nt < 2048 ? 1024u : 4096u))
+        launch_direct_fp64_t<1, 1>(S, sys_off, nsys, targets, nt, G, eps2, acc, pot, st);
     else
-        hipLaunchKernelGGL(direct_fp64_kernel<1>, dim3(nt), dim3(WAVE * DD_WAVES), 0, st, S, sys_off, nsys, targets,
-                           nt, G, eps2, acc, pot);
+        launch_direct_fp64_t<1, 8>(S, sys_off, nsys, targets, nt, G, eps2, acc, pot, st);
 }
 
 // slots[k] = slot_of[targets[k]] (targets checked by the host)

@@ -274,8 +274,8 @@ size_t direct_pack_bytes(uint32_t n, uint32_t max_sys_n, int nsys);
 void launch_direct_f32(const State& S, uint32_t n, uint32_t max_sys_n, const uint32_t* sys_off, int nsys,
                        const double4* box, float G, float eps2, int compat_law, double kick_dt, float* pk,
                        hipStream_t st);
-void launch_direct_fp64(const State& S, const uint32_t* sys_off, int nsys, const uint32_t* targets, uint32_t nt,
-                        double G, double eps2, double* acc, double* pot, hipStream_t st);
+void launch_direct_fp64(const State& S, uint32_t n, const uint32_t* sys_off, int nsys, const uint32_t* targets,
+                        uint32_t nt, double G, double eps2, double* acc, double* pot, hipStream_t st);
 void launch_map_slots(const uint32_t* slot_of, const int64_t* targets, uint32_t nt, uint32_t* slots, hipStream_t st);
 void launch_find_slots(const uint32_t* id, uint32_t n, const int64_t* targets, uint32_t nt, uint32_t* slots,
                        hipStream_t st);

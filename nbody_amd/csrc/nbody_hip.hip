@@ -1693,7 +1693,7 @@ int nbh_direct_fp64(nbh_handle* h, size_t nt, const int64_t* targets, double* ac
     HIPCHK(h, h->staging.to_device(&in, 1, dtg, h->stream));
     launch_inverse_perm(S.id, h->slot_of.as<uint32_t>(), (uint32_t)n, h->stream);
     launch_map_slots(h->slot_of.as<uint32_t>(), dtg, (uint32_t)nt, dslot, h->stream);
-    launch_direct_fp64(S, h->sys_off.as<uint32_t>(), h->nsys, dslot, (uint32_t)nt, h->cfg.G,
+    launch_direct_fp64(S, (uint32_t)n, h->sys_off.as<uint32_t>(), h->nsys, dslot, (uint32_t)nt, h->cfg.G,
                        h->cfg.eps * h->cfg.eps, dacc, dpot, h->stream);
     HIPCHK(h, hipGetLastError());
     const Staging::Part out[2] = {{acc, nt * 24}, {pot, nt * 8}};
@@ -1759,7 +1759,7 @@ int nbh_direct_fp64_noalloc(nbh_handle* h, size_t nt, const int64_t* targets, do
     State S = h->st[h->cur].view();
     HIPCHK(h, hipMemcpyAsync(dtg, targets, nt * 8, hipMemcpyHostToDevice, h->stream));
     launch_find_slots(S.id, (uint32_t)n, dtg, (uint32_t)nt, dslot, h->stream);
-    launch_direct_fp64(S, h->sys_off.as<uint32_t>(), h->nsys, dslot, (uint32_t)nt, h->cfg.G,
+    launch_direct_fp64(S, (uint32_t)n, h->sys_off.as<uint32_t>(), h->nsys, dslot, (uint32_t)nt, h->cfg.G,
                        h->cfg.eps * h->cfg.eps, dacc, dpot, h->stream);
     HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipMemcpyAsync(acc, dacc, nt * 24, hipMemcpyDeviceToHost, h->stream));

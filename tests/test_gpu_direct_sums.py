@@ -149,3 +149,27 @@ def test_direct_solver_many_small_systems(small):
         j = i ^ 1
         ar, _ = _sum64(_packed(x[[i, j]]), m[[i, j]], 1e-2, [0])
         assert np.max(np.abs(acc[i] - ar[0])) <= 2e-5 * np.abs(ar).max()
+
+
+# systems x size and targets either side of the rule for ensembles: 1024 and
+# 2048 targets, mean sizes 1024 and 4096, and a last workgroup that is not full
+@pytest.mark.parametrize("systems,size,nt", [(3, 500, 1023), (3, 500, 1024), (2, 1024, 1027), (2, 1025, 2047),
+                                             (2, 1025, 2048), (2, 4096, 4099), (2, 4097, 4099), (700, 3, 2100),
+                                             (65, 64, 1)])
+def test_fp64_sums_of_ensembles(systems, size, nt):
+    rng = np.random.default_rng(systems * size)
+    n = systems * size
+    x, m = rng.standard_normal((n, 3)), rng.uniform(0.5, 1.5, n) / size
+    off = np.arange(systems + 1) * size
+    t = rng.permutation(n)[:nt]
+    cfg = nb.default_config(eps=1e-3)
+    with nb.HipSimulation.from_arrays(x, np.zeros_like(x), m, m, config=cfg, sys_off=off) as sim:
+        acc, pot = sim.direct_fp64(t)
+        acc2, pot2 = sim.direct_fp64_noalloc(t)
+    assert np.array_equal(acc, acc2) and np.array_equal(pot, pot2)
+    for k in range(0, nt, max(1, nt // 97)):
+        s = t[k] // size
+        ar, pr = _sum64(x[size * s:size * (s + 1)], m[size * s:size * (s + 1)], 1e-3, [t[k] - size * s])
+        # 64-bit sums of up to 4097 terms, each to a few ulps; a sum that cancels has the terms' errors
+        assert np.max(np.abs(acc[k] - ar[0])) <= 1e-12 * max(np.abs(ar).max(), np.abs(pr[0]))
+        assert abs(pot[k] - pr[0]) <= 1e-13 * abs(pr[0])
