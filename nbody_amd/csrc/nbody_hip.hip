@@ -57,24 +57,51 @@ struct DevBuf {
     template <typename T> T* as() const { return (T*)p; }
 };
 
+// Arrays that are sized together share one allocation: what a device has beyond
+// the 64 MiB that the runtime keeps for reuse goes back to the system at a
+// handle's end and comes from it at the next one's start, which takes ~0.25 ms
+// an allocation of 2 MiB or more.
+struct Slice {
+    void* p = nullptr;
+    size_t bytes = 0;
+    template <typename T> T* as() const { return (T*)p; }
+};
+struct SliceSize {
+    Slice* s;
+    size_t bytes;
+};
+template <size_t N>
+hipError_t ensure_slices(DevBuf& mem, const SliceSize (&part)[N]) {
+    auto place = [](size_t bytes) { return (bytes + 4095) / 4096 * 4096; };
+    size_t total = 0;
+    for (const SliceSize& q : part) {
+        total += place(q.bytes);
+        *q.s = Slice{};
+    }
+    const hipError_t e = mem.ensure(total);
+    if (e != hipSuccess) return e;
+    char* at = mem.as<char>();
+    for (const SliceSize& q : part) {
+        *q.s = Slice{at, q.bytes};
+        at += place(q.bytes);
+    }
+    return hipSuccess;
+}
+
 struct StateBufs {
-    DevBuf x, y, z, vx, vy, vz, mass, charge, ax, ay, az, pot, id;
+    DevBuf mem;
+    Slice x, y, z, vx, vy, vz, mass, charge, ax, ay, az, pot, id;
     hipError_t alloc(size_t n) {
-        DevBuf* d[] = {&x, &y, &z, &vx, &vy, &vz, &mass, &charge};
-        for (DevBuf* b : d) { hipError_t e = b->ensure(n * 8); if (e) return e; }
-        DevBuf* f[] = {&ax, &ay, &az, &pot, &id};
-        for (DevBuf* b : f) { hipError_t e = b->ensure(n * 4); if (e) return e; }
-        return hipSuccess;
+        return ensure_slices(mem, {{&x, n * 8}, {&y, n * 8}, {&z, n * 8}, {&vx, n * 8}, {&vy, n * 8}, {&vz, n * 8},
+                                   {&mass, n * 8}, {&charge, n * 8}, {&ax, n * 4}, {&ay, n * 4}, {&az, n * 4},
+                                   {&pot, n * 4}, {&id, n * 4}});
     }
     State view() const {
         return State{x.as<double>(), y.as<double>(), z.as<double>(), vx.as<double>(), vy.as<double>(),
                      vz.as<double>(), mass.as<double>(), charge.as<double>(), ax.as<float>(), ay.as<float>(),
                      az.as<float>(), pot.as<float>(), id.as<uint32_t>()};
     }
-    void release() {
-        DevBuf* all[] = {&x, &y, &z, &vx, &vy, &vz, &mass, &charge, &ax, &ay, &az, &pot, &id};
-        for (DevBuf* b : all) b->release();
-    }
+    void release() { mem.release(); }
 };
 
 // Launch shapes of a captured step, taken from the last uncaptured step with
@@ -121,11 +148,14 @@ struct nbh_handle {
 
     StateBufs st[2];
     int cur = 0;
-    DevBuf sys_off, keys, keys_alt, perm, perm_alt, sort_tmp, tree_tmp, scan_tmp;
+    DevBuf sys_off, scan_tmp, part_mem;
+    Slice keys, keys_alt, perm, perm_alt, sort_tmp, tree_tmp, leaf_ids, pf, pleaf;  // part_mem
     DevBuf box, inv, unit, bbox_part;
-    DevBuf geo, link, nsys_of, node_begin, leaf_ids, M, L, Lx, Lt, pf, pleaf, dtab, xtab, far_src, far_tgt, near_items, near_k, near_first, near_part;
-    DevBuf row_node, row_first, row_next, row_sl_start, row_sl_cnt, sl, row_m_start, row_m_cnt, row_mx_cnt,
-        row_p_start, row_p_cnt, m2l_pool, p2p_pool;
+    DevBuf dtab, xtab, far_src, far_tgt, near_part;
+    DevBuf node_mem, row_mem, sl, m2l_pool, p2p_pool;
+    Slice geo, link, nsys_of, node_begin, M, L, Lx, Lt, row_first, near_items, near_k, near_first;  // node_mem
+    Slice row_node, row_next, row_sl_start, row_sl_cnt, row_m_start, row_m_cnt, row_mx_cnt, row_p_start,
+        row_p_cnt;  // row_mem
     unsigned long long m2l_pool_cap = 0, p2p_pool_cap = 0;
     bool small_pools = false;  // the device had no room for pools of the usual sizes
     DevBuf counters, diag, tmp_small;
@@ -336,19 +366,13 @@ static int alloc_nodes(nbh_handle* h, uint32_t need) {
     uint32_t cap = std::max<uint32_t>(need + need / 4, 1024);
     const int ncp = ncp_of((int)h->cfg.order);
     h->node_cap = 0;  // (until every array is there)
-    HIPCHK(h, h->geo.ensure((size_t)cap * 16));
-    HIPCHK(h, h->link.ensure((size_t)cap * 16));
-    HIPCHK(h, h->nsys_of.ensure((size_t)cap * 4));
-    HIPCHK(h, h->node_begin.ensure((size_t)cap * 4));
-    HIPCHK(h, h->M.ensure((size_t)cap * ncp * 4));
-    HIPCHK(h, h->L.ensure((size_t)cap * ncp * 4));
-    HIPCHK(h, h->Lx.ensure((size_t)cap * ncp * 4));
-    HIPCHK(h, h->Lt.ensure((size_t)cap * ncp * 4));
-    HIPCHK(h, h->row_first.ensure((size_t)cap * 4));
-    HIPCHK(h, h->near_k.ensure((size_t)cap * 4));
-    HIPCHK(h, h->near_first.ensure((size_t)cap * 4));
     // items: every leaf's target chunks, and the slots of the leaves that are cut
-    HIPCHK(h, h->near_items.ensure((std::min<size_t>(cap, h->n) + h->n / 64 + near_slot_cap(h)) * sizeof(NearItem)));
+    const size_t c = cap, exp = c * ncp * 4;
+    const size_t items = std::min<size_t>(c, h->n) + h->n / 64 + near_slot_cap(h);
+    HIPCHK(h, ensure_slices(h->node_mem, {{&h->geo, c * 16}, {&h->link, c * 16}, {&h->nsys_of, c * 4},
+                                          {&h->node_begin, c * 4}, {&h->M, exp}, {&h->L, exp}, {&h->Lx, exp},
+                                          {&h->Lt, exp}, {&h->row_first, c * 4}, {&h->near_k, c * 4},
+                                          {&h->near_first, c * 4}, {&h->near_items, items * sizeof(NearItem)}}));
     HIPCHK(h, h->scan_tmp.ensure(scan_tmp_bytes(cap + 1) + 256));
     h->node_cap = cap;
     return NBH_OK;
@@ -493,9 +517,10 @@ static FmmParams fmm_params(nbh_handle* h) {
 
 static int grow_rows(nbh_handle* h, uint32_t cap) {
     h->row_cap = 0;  // (until every array is there)
-    DevBuf* rows[] = {&h->row_node, &h->row_next, &h->row_sl_start, &h->row_sl_cnt,
-                      &h->row_m_start, &h->row_m_cnt, &h->row_mx_cnt, &h->row_p_start, &h->row_p_cnt};
-    for (DevBuf* b : rows) HIPCHK(h, b->ensure((size_t)cap * 4));
+    const size_t b = (size_t)cap * 4;
+    HIPCHK(h, ensure_slices(h->row_mem, {{&h->row_node, b}, {&h->row_next, b}, {&h->row_sl_start, b},
+                                         {&h->row_sl_cnt, b}, {&h->row_m_start, b}, {&h->row_m_cnt, b},
+                                         {&h->row_mx_cnt, b}, {&h->row_p_start, b}, {&h->row_p_cnt, b}}));
     h->row_cap = cap;
     return NBH_OK;
 }
@@ -1092,9 +1117,9 @@ static int graph_prepare(nbh_handle* h) {
 static int graph_snapshot(nbh_handle* h, bool save) {
     const size_t n = h->n;
     StateBufs& sb = h->st[h->cur];
-    DevBuf* d[] = {&sb.x, &sb.y, &sb.z, &sb.vx, &sb.vy, &sb.vz};
+    Slice* d[] = {&sb.x, &sb.y, &sb.z, &sb.vx, &sb.vy, &sb.vz};
     char* o = (char*)h->gsnap.p;
-    for (DevBuf* b : d) {
+    for (Slice* b : d) {
         HIPCHK(h, save ? hipMemcpyAsync(o, b->p, n * 8, hipMemcpyDeviceToDevice, h->stream)
                        : hipMemcpyAsync(b->p, o, n * 8, hipMemcpyDeviceToDevice, h->stream));
         o += n * 8;
@@ -1348,19 +1373,20 @@ static int create_impl(const nbh_config* cfg, size_t nsys, const uint32_t* sys_o
     CCHK(h->st[0].alloc(n));
     CCHK(h->st[1].alloc(n));
     CCHK(h->sys_off.ensure((nsys + 1) * 4));
-    CCHK(h->keys.ensure(n * 8));
-    CCHK(h->keys_alt.ensure(n * 8));
-    CCHK(h->perm.ensure(n * 4));
-    CCHK(h->perm_alt.ensure(n * 4));
-    CCHK(h->sort_tmp.ensure(radix_tmp_bytes((uint32_t)n)));
-    CCHK(h->tree_tmp.ensure(tree_tmp_bytes((uint32_t)n, (int)h->cfg.max_depth)));
+    CCHK(ensure_slices(h->part_mem,
+                       {{&h->keys, n * 8},
+                        {&h->keys_alt, n * 8},
+                        {&h->perm, n * 4},
+                        {&h->perm_alt, n * 4},
+                        {&h->sort_tmp, radix_tmp_bytes((uint32_t)n)},
+                        {&h->tree_tmp, tree_tmp_bytes((uint32_t)n, (int)h->cfg.max_depth)},
+                        {&h->leaf_ids, n * 4},
+                        {&h->pf, std::max(n * 16, direct_pack_bytes((uint32_t)n, h->max_sys_n, (int)nsys))},
+                        {&h->pleaf, n * 4}}));
     CCHK(h->box.ensure(nsys * sizeof(double4)));
     CCHK(h->inv.ensure(nsys * 8));
     CCHK(h->unit.ensure(nsys * 4));
     CCHK(h->bbox_part.ensure(bbox_part_bytes(h->max_sys_n, (int)nsys)));
-    CCHK(h->leaf_ids.ensure(n * 4));
-    CCHK(h->pf.ensure(std::max(n * 16, direct_pack_bytes((uint32_t)n, h->max_sys_n, (int)nsys))));
-    CCHK(h->pleaf.ensure(n * 4));
     CCHK(h->counters.ensure(sizeof(Counters)));
     CCHK(h->diag.ensure(1024 * 8 * 8));
     CCHK(h->tmp_small.ensure(64));
@@ -1505,14 +1531,12 @@ void nbh_destroy(nbh_handle* h) {
     h->gsnap.release();
     h->st[0].release();
     h->st[1].release();
-    DevBuf* all[] = {&h->sys_off, &h->keys, &h->keys_alt, &h->perm, &h->perm_alt, &h->sort_tmp, &h->tree_tmp,
-                     &h->scan_tmp, &h->box, &h->inv, &h->unit, &h->bbox_part, &h->geo, &h->link, &h->nsys_of,
-                     &h->node_begin, &h->leaf_ids, &h->M, &h->L, &h->Lx, &h->Lt, &h->Lwt, &h->pf, &h->pleaf, &h->dtab, &h->xtab, &h->far_src, &h->far_tgt, &h->near_items, &h->near_k, &h->near_first,
-                     &h->near_part, &h->row_node, &h->row_first,
-                     &h->row_next, &h->row_sl_start, &h->row_sl_cnt, &h->row_m_start, &h->row_m_cnt,
-                     &h->row_mx_cnt, &h->row_p_start, &h->row_p_cnt, &h->m2l_pool, &h->p2p_pool, &h->sl, &h->counters, &h->diag,
+    DevBuf* all[] = {&h->sys_off, &h->part_mem, &h->scan_tmp, &h->box, &h->inv, &h->unit, &h->bbox_part,
+                     &h->node_mem, &h->row_mem, &h->Lwt, &h->dtab, &h->xtab, &h->far_src, &h->far_tgt,
+                     &h->near_part, &h->m2l_pool, &h->p2p_pool, &h->sl, &h->counters, &h->diag,
                      &h->tmp_small, &h->Mw, &h->Lw, &h->pw, &h->wbuf, &h->gbuf, &h->mb, &h->mbw, &h->d2tab,
-                     &h->cand, &h->hank, &h->opar, &h->sl_offs, &h->sl_map, &h->acc_save, &h->slot_of, &h->direct_buf, &h->io};
+                     &h->cand, &h->hank, &h->opar, &h->sl_offs, &h->sl_map, &h->acc_save, &h->slot_of,
+                     &h->direct_buf, &h->io};
     for (DevBuf* b : all) b->release();
     for (DevBuf& b : h->adj_ckpt) b.release();
     for (DevBuf& b : h->adj_seg) b.release();
@@ -1784,14 +1808,14 @@ int nbh_diagnostics(nbh_handle* h, double* out) {
         char* o = (char*)h->acc_save.p;
         {
             const StateBufs& sb = h->st[h->cur];
-            const DevBuf* a[3] = {&sb.ax, &sb.ay, &sb.az};
+            const Slice* a[3] = {&sb.ax, &sb.ay, &sb.az};
             for (int k = 0; k < 3; ++k)
                 HIPCHK(h, hipMemcpyAsync(o + k * n * 4, a[k]->p, n * 4, hipMemcpyDeviceToDevice, h->stream));
         }
         CHK(force_eval(h, 0.0, true));
         {
             const StateBufs& sb = h->st[h->cur];
-            const DevBuf* a[3] = {&sb.ax, &sb.ay, &sb.az};
+            const Slice* a[3] = {&sb.ax, &sb.ay, &sb.az};
             for (int k = 0; k < 3; ++k)
                 HIPCHK(h, hipMemcpyAsync(a[k]->p, o + k * n * 4, n * 4, hipMemcpyDeviceToDevice, h->stream));
         }
@@ -1892,22 +1916,22 @@ static int snapshot_save(nbh_handle* h, DevBuf& dst) {
     const size_t n = h->n;
     HIPCHK(h, dst.ensure(snapshot_bytes(n)));
     const StateBufs& sb = h->st[h->cur];
-    const DevBuf* d8[] = {&sb.x, &sb.y, &sb.z, &sb.vx, &sb.vy, &sb.vz, &sb.mass, &sb.charge};
-    const DevBuf* d4[] = {&sb.ax, &sb.ay, &sb.az, &sb.pot, &sb.id};
+    const Slice* d8[] = {&sb.x, &sb.y, &sb.z, &sb.vx, &sb.vy, &sb.vz, &sb.mass, &sb.charge};
+    const Slice* d4[] = {&sb.ax, &sb.ay, &sb.az, &sb.pot, &sb.id};
     char* o = (char*)dst.p;
-    for (const DevBuf* b : d8) { HIPCHK(h, hipMemcpyAsync(o, b->p, n * 8, hipMemcpyDeviceToDevice, h->stream)); o += n * 8; }
-    for (const DevBuf* b : d4) { HIPCHK(h, hipMemcpyAsync(o, b->p, n * 4, hipMemcpyDeviceToDevice, h->stream)); o += n * 4; }
+    for (const Slice* b : d8) { HIPCHK(h, hipMemcpyAsync(o, b->p, n * 8, hipMemcpyDeviceToDevice, h->stream)); o += n * 8; }
+    for (const Slice* b : d4) { HIPCHK(h, hipMemcpyAsync(o, b->p, n * 4, hipMemcpyDeviceToDevice, h->stream)); o += n * 4; }
     return NBH_OK;
 }
 
 static int snapshot_restore(nbh_handle* h, const DevBuf& src, double t) {
     const size_t n = h->n;
     StateBufs& sb = h->st[h->cur];
-    DevBuf* d8[] = {&sb.x, &sb.y, &sb.z, &sb.vx, &sb.vy, &sb.vz, &sb.mass, &sb.charge};
-    DevBuf* d4[] = {&sb.ax, &sb.ay, &sb.az, &sb.pot, &sb.id};
+    Slice* d8[] = {&sb.x, &sb.y, &sb.z, &sb.vx, &sb.vy, &sb.vz, &sb.mass, &sb.charge};
+    Slice* d4[] = {&sb.ax, &sb.ay, &sb.az, &sb.pot, &sb.id};
     const char* o = (const char*)src.p;
-    for (DevBuf* b : d8) { HIPCHK(h, hipMemcpyAsync(b->p, o, n * 8, hipMemcpyDeviceToDevice, h->stream)); o += n * 8; }
-    for (DevBuf* b : d4) { HIPCHK(h, hipMemcpyAsync(b->p, o, n * 4, hipMemcpyDeviceToDevice, h->stream)); o += n * 4; }
+    for (Slice* b : d8) { HIPCHK(h, hipMemcpyAsync(b->p, o, n * 8, hipMemcpyDeviceToDevice, h->stream)); o += n * 8; }
+    for (Slice* b : d4) { HIPCHK(h, hipMemcpyAsync(b->p, o, n * 4, hipMemcpyDeviceToDevice, h->stream)); o += n * 4; }
     h->time = t;
     h->acc_valid = true;  // the snapshot carries the accelerations of its positions
     h->pot_valid = false;  // (and the potentials only if that evaluation computed them)
@@ -2116,7 +2140,7 @@ int nbh_debug_expansions(nbh_handle* h, float* M, float* L) {
     const int nc = ncoef((int)h->cfg.order), ncp = ncp_of((int)h->cfg.order);
     std::vector<float> buf(nn * ncp);
     float* outs[2] = {M, L};
-    DevBuf* srcs[2] = {&h->M, &h->Lt};
+    const Slice* srcs[2] = {&h->M, &h->Lt};
     for (int k = 0; k < 2; ++k) {
         if (!outs[k]) continue;
         HIPCHK(h, hipMemcpyAsync(buf.data(), srcs[k]->p, buf.size() * 4, hipMemcpyDeviceToHost, h->stream));
