@@ -1396,6 +1396,9 @@ static int create_impl(const nbh_config* cfg, size_t nsys, const uint32_t* sys_o
     if (cfg->solver == NBH_SOLVER_FMM) {
         int r = alloc_nodes(h, (uint32_t)std::min<size_t>(n / 2 + 64, 0x7fffffff));
         if (r) return bail(r);
+        // the slots that a small system's lists usually take (allocated with the
+        // rest, not between the launches of its first evaluation)
+        if (n <= 16384) CCHK(h->near_part.ensure(std::min<size_t>(near_slot_cap(h), n + n / 4) * 1024));
         // candidate same-level offsets o of the matrix-core M2L, with the mask of
         // the target classes c (position in the parent) that take them: the
         // criterion accepts o and rejects the parent offset floor((c + o) / 2)

@@ -61,26 +61,27 @@ def test_items_match_whole_lists(name, ic, n, opt, chunk):
     assert np.max(np.abs(p.astype(np.float64) - pr)) <= tol * np.max(np.abs(pr)) + 1e-30
 
 
-def test_more_items_than_slots():
-    """512 leaves of ten target chunks that all meet each other in eight batches:
-    cut to single batches they would take 40,960 slots of the 32,768.  No
-    far-field pairs, so that every evaluation is the same sum to the bit."""
-    n = 300000
+@pytest.mark.parametrize("n,cap,slots", [(300000, 1024, 32768), (600000, 2048, 65536)])
+def test_more_items_than_slots(n, cap, slots):
+    """512 leaves of ten (19) target chunks that all meet each other in eight
+    batches: cut to single batches they would take 40,960 (77,824) slots, of
+    65,536.  No far-field pairs, so that every evaluation is the same sum to the
+    bit."""
     x, v, m = nb.ics.uniform(n, 5)
     got = []
     for p2p in (nb.P2P_LANE, nb.P2P_LANE, nb.P2P_LEAF):
-        cfg = nb.default_config(eps=1e-2, theta=0.125, leaf_capacity=1024, order=2, p2p=p2p)
+        cfg = nb.default_config(eps=1e-2, theta=0.125, leaf_capacity=cap, order=2, p2p=p2p)
         with nb.HipSimulation.from_arrays(x, v, m, m, config=cfg) as sim:
             got += [sim.forces() for _ in range(3 if p2p == nb.P2P_LANE else 1)]
             s, off = sim.debug_sizes(), sim.debug_lists()[2]
             count = np.array(sim.debug_tree()["count"])
     assert s["m2l"] == 0 and s["leaves"] == 512
     leaf = np.diff(off) > 0
-    assert np.sum(np.ceil(np.diff(off)[leaf] / 64) * np.ceil(count[leaf] / 64)) > 32768
+    assert np.sum(np.ceil(np.diff(off)[leaf] / 64) * np.ceil(count[leaf] / 64)) > slots
     for a, p in got[1:6]:
         assert np.array_equal(a, got[0][0]) and np.array_equal(p, got[0][1])
-    # sums of 75,000 terms added up are no further from the 64-bit sum than
-    # single ones of 300,000
+    # sums of a part of the sources added up are no further from the 64-bit sum
+    # than single ones of all n
     t = np.arange(0, n, 149)
     with nb.HipSimulation.from_arrays(x, v, m, m, config=cfg) as sim:
         exact = sim.direct_fp64(t)
