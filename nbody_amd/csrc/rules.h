@@ -17,6 +17,20 @@ constexpr uint32_t POOL_CHUNK_M = 2048, POOL_CHUNK_P = 512, POOL_CHUNK_S = 512;
 // the most entries of a pool (its counter has 32 bits)
 constexpr unsigned long long POOL_MAX = 0xffff0000ull;
 
+// The walk's criterion 3 den^2 (d_A + d_B)^2 < 4 num^2 |c_B - c_A|^2 in units of
+// half the finer cell of the pair, `gap` levels apart: the largest squared
+// centre offset that it does not accept, 3 den^2 (2 + 2 2^gap)^2 / 4 num^2
+// rounded down (2^32 - 1: not below 2^32 - 1).
+constexpr uint32_t walk_threshold(uint32_t num4, uint32_t den3, int gap) {
+    const uint64_t side = 2ull + (2ull << gap);
+    return (uint32_t)std::min<uint64_t>((uint64_t)den3 * side * side / num4, 0xffffffffu);
+}
+// Offsets of octant 0's centre whose squares, and those of the other octants'
+// (2 less), are products of 24 bits with a sum of three in 32 bits.
+constexpr int WALK_SMALL = 32000;
+constexpr bool walk_small(int d) { return (uint32_t)(d + WALK_SMALL) <= 2u * WALK_SMALL; }
+static_assert(WALK_SMALL + 2 < 1 << 23 && 3ull * (WALK_SMALL + 2) * (WALK_SMALL + 2) < 1ull << 32, "squares fit");
+
 // First sizes (entries) of the M2L and P2P pools for `nodes` cells of a handle
 // whose largest system holds max_sys_n of its n particles, walked by `blocks`
 // workgroups at theta = num / den.  A cell keeps about 1000 M2L and 230 P2P

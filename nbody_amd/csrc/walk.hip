@@ -271,7 +271,7 @@ __device__ __forceinline__ void cat_add(CatCount& c, uint64_t a, uint64_t v, uin
 // of them less 2 for the others, so a candidate takes six squares, eight sums
 // and eight compares with a threshold that depends on the level gap alone
 // (floor of 3 den^2 (d_A + d_B)^2 / 4 num^2, exact).  Squares are 24-bit
-// products in 32 bits where every offset of the chunk is below 32,000 (all but
+// products in 32 bits where every offset of the chunk is small (rules.h; all but
 // level gaps of ten and more, which take the 64-bit form).  A chunk's
 // accepted candidates are one 64-bit mask per target; the categories follow
 // from it and three masks of the candidates (valid, leaf, target's level) by
@@ -421,8 +421,7 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
                 const int dx = ((2 * gb.x + 1) << sb) - (tx << sa), dy = ((2 * gb.y + 1) << sb) - (ty << sa);
                 const int dz = ((2 * gb.z + 1) << sb) - (tz << sa);
                 const uint32_t thr = thr_s[sa + sb];
-                const bool big = (uint32_t)(dx + 32000) > 64000u || (uint32_t)(dy + 32000) > 64000u ||
-                                 (uint32_t)(dz + 32000) > 64000u || thr == 0xffffffffu;
+                const bool big = !walk_small(dx) || !walk_small(dy) || !walk_small(dz) || thr == 0xffffffffu;
                 uint64_t a = 0;
                 if (!(__ballot(big) & v)) {
                     const uint32_t x[2] = {(uint32_t)__mul24(dx, dx), (uint32_t)__mul24(dx - 2, dx - 2)};
@@ -621,14 +620,8 @@ __global__ __launch_bounds__(WAVE * NW) void walk_group_kernel(WalkParams W, int
     }
 }
 
-// thr[gap]: the largest squared centre offset, in half cells of the finer of
-// two cells `gap` levels apart, that the criterion does not accept (2^32 - 1:
-// not below 2^32 - 1)
 void walk_thresholds(uint32_t num4, uint32_t den3, uint32_t* thr) {
-    for (int g = 0; g < MAX_LEVELS; ++g) {
-        const uint64_t side = 2ull + (2ull << g);
-        thr[g] = (uint32_t)std::min<uint64_t>((uint64_t)den3 * side * side / num4, 0xffffffffu);
-    }
+    for (int g = 0; g < MAX_LEVELS; ++g) thr[g] = walk_threshold(num4, den3, g);
 }
 
 void launch_walk_root(const WalkParams& W, hipStream_t st) {

@@ -22,6 +22,7 @@ void pool_sizes(uint32_t nodes, uint32_t max_sys_n, uint64_t n, int num, int den
     out[1] = s.p2p;
 }
 uint32_t item_batches(uint64_t entries, uint64_t work, uint32_t slots) { return near_item_batches(entries, work, slots); }
+int small_offset(int d) { return walk_small(d); }
 uint64_t slots_bound(uint64_t entries, uint64_t work, uint32_t slots) { return near_slots_bound(entries, work, slots); }
 }
 """
