@@ -51,9 +51,9 @@ __global__ void direct_pack_kernel(State S, uint32_t n, const uint32_t* sys_off,
 // bit those of the one-thread chain.  Per source and 64 targets the producers
 // issue 14 slots (the rsq takes four) and the consumers 6: 150 us at N =
 // 16,384 if the four SIMDs of a CU never wait; measured 190 us.  (The sum cut
-// into 16 slices takes 129 us, but rounds differently.)  Sources are the same for every lane of
-// a wavefront and come through scalar loads.  The potential has no such order:
-// each producer keeps a partial sum.  NORMAL: eps^2 is a normal float, so that
+// into 16 slices takes 129 us, but rounds differently.)  Sources are the same
+// for every lane of a wavefront and come through scalar loads.  The potential
+// has no such order: each producer keeps a partial sum.  NORMAL: eps^2 is a normal float, so that
 // v_rsq_f32 needs no denormal scaling (rsqrtf's).
 constexpr int DS_PROD = 13, DS_PER = 8, DS_CH = DS_PROD * DS_PER, DS_WAVES = DS_PROD + 3;
 static_assert(DS_PAD >= DS_CH, "a chunk past the particles reads the padding");

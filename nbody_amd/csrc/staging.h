@@ -60,8 +60,9 @@ private:
 
     hipError_t ensure(size_t bytes) {
         if (bytes <= cap_) return hipSuccess;
-        // (the last use of the ring may still be in flight)
-        hipError_t e = hipDeviceSynchronize();
+        // (the last upload may still be in flight; a device-wide wait would also
+        // wait for other handles, and meet a stream that another thread captures)
+        hipError_t e = drain();
         if (e != hipSuccess) return e;
         if (pin_) (void)hipHostFree(pin_);
         pin_ = nullptr;

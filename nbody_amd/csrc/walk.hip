@@ -27,9 +27,10 @@
 // group, each of its wavefronts a slice of the split list: a candidate is
 // loaded once and classified against every target (up to 8); then count,
 // reserve, write.  Each row's M2L, P2P and split entries land as contiguous
-// segments carved from per-workgroup chunks of three pools; a node's rows are chained in depth order (first row = its
-// level row, next = its carried row one depth deeper), and the force kernels
-// follow the chain, so no compaction pass is needed.
+// segments carved from per-workgroup chunks of three pools; a node's rows are
+// chained in depth order (first row = its level row, next = its carried row one
+// depth deeper), and the force kernels follow the chain, so no compaction pass
+// is needed.
 //
 // Each target's entries come out in ascending source id, chain order included:
 // split lists are ascending, kept leaves (coarser levels) precede children,

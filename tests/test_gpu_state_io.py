@@ -48,3 +48,19 @@ def test_set_state_refuses_and_keeps():
         assert after[4] == t and all(np.array_equal(a, b) for a, b in zip(before, after))
         sim.set_state(x, v)
         assert np.array_equal(sim.positions(), x)
+
+
+def test_ring_grows_behind_an_upload():
+    """A transfer that needs a larger ring than the upload before it, which may
+    still be on its way: targets (8 bytes each) up, their sums (32) down."""
+    x, v, m = nb.ics.plummer(9001, 4)
+    with nb.HipSimulation.from_arrays(x, v, m, m, config=nb.default_config()) as sim:
+        t = np.arange(9001)
+        whole = sim.direct_fp64(t)
+    for nt in (1, 2049, 8191):
+        with nb.HipSimulation.from_arrays(x[:100], v[:100], m[:100], m[:100], config=nb.default_config()) as small:
+            few = small.direct_fp64(np.arange(nt) % 100)
+            assert np.array_equal(few[0], few[0][np.arange(nt) % 100])
+        with nb.HipSimulation.from_arrays(x, v, m, m, config=nb.default_config()) as sim:
+            acc, pot = sim.direct_fp64(t[:nt])
+        assert np.allclose(acc, whole[0][:nt], rtol=1e-12, atol=0) and np.allclose(pot, whole[1][:nt], rtol=1e-12)
