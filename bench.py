@@ -263,7 +263,7 @@ def workload_uniform4096(nb, args):
         res[label] = {"particle_steps_per_s": n * K / wall, "ms_per_step": wall / K * 1e3, "force_err": err}
         if graph:
             res[label]["graph"] = {k: st[k] for k in ("graph_captures", "graph_replays", "graph_fallbacks")}
-    # the value: the tuned kernels with captured steps (the fastest at this size)
+    # the value: the tuned kernels with captured steps (the launched ones take the same time at this size)
     out = {"metric": "particle-steps/s, N=4096 uniform, 10 KDK steps; force error vs FP64 direct",
            "value": res["tuned_graph"]["particle_steps_per_s"], "unit": "particle-steps/s", "n_gpus": 1, "steps": K,
            "warmup": 2, "ms_per_step": res["tuned_graph"]["ms_per_step"], "higher_is_better": True, "scaling": "weak",
