@@ -1203,7 +1203,7 @@ static void launch_m2l_pq_pot(const FmmParams& F, const M2LPlan& plan, int parts
         if (!(parts & M2L_LEVELS) || (level >= 0 && l != level)) continue;
         const uint32_t cnt = plan.level_count[l];
         if (!cnt) continue;
-        if (plan.mfma) {
+        if (plan.mfma && l >= 2) {
             // by translation offset on the matrix cores: one workgroup per
             // level-(l-2) cell, its level-l descendants as the targets
             launch_m2l_offset_level(P, plan.mfma == 1, F, plan.off, plan.level_off[l - 2], plan.level_count[l - 2],

@@ -759,6 +759,13 @@ static int m2l_q(const nbh_handle* h) {
     return (h->cfg.m2l_terms == NBH_M2L_TERMS_ALL && p < q && q < 2 * p) ? (q | M2L_ALL) : q;
 }
 
+// First level of the same-level tables.  Cells of level 1 are at most the cube's
+// diagonal apart, which is the sum of their radii: some pairs are well separated
+// for every theta above 1, none at or below it.  The matrix-core forms group
+// targets by an ancestor two levels up and start at level 2; level 1's eight
+// cells go to the grouped kernel there.
+static int table_level0(const nbh_handle* h) { return h->theta_num > h->theta_den ? 1 : 2; }
+
 // P2P tile: sources staged per wavefront round
 static int p2p_chunk(const nbh_handle* h) { return h->cfg.p2p_chunk == 128 ? 128 : 64; }
 
@@ -826,18 +833,19 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
     int K = 0, nlev = 0, E = 0, xn = 0;
     const bool off = tables && use_offset_m2l(h), bf3 = h->cfg.m2l == NBH_M2L_BF16X3;
     if (tables) {
-        // derivative tensors of the same-level offsets [0, K]^3 of levels
-        // 2..depth (cells of levels 0 and 1 are never well separated), per
-        // system, since the tensors depend on each system's root size
+        // derivative tensors of the same-level offsets [0, K]^3 of the levels
+        // from table_level0 down to depth, per system, since the tensors depend
+        // on each system's root size
         const int Kp = (int)std::floor(std::sqrt(3.0) * h->theta_den / h->theta_num);
         K = 2 * Kp + 1;
         const int dsz = h->sl_rows, dcp = ncp_of(m2l_deg(q));
-        nlev = (int)depth - 1;
+        const int level0 = table_level0(h);
+        nlev = (int)depth - level0 + 1;
         HIPCHK(h, h->dtab.ensure((size_t)dsz * nlev * dcp * 4 * h->nsys));
         T = F;
         T.dtab = h->dtab.as<float>();
         T.dK = K;
-        T.dlevel0 = 2;
+        T.dlevel0 = level0;
         T.dnlev = nlev;
         T.dcp = dcp;
         T.dsz = dsz;
@@ -858,7 +866,7 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
             // dense tensors (orders <= 2p) of the offsets [0, K]^3, levels 2..depth
             HIPCHK(h, h->mb.ensure(off_moment_bytes(p, bf3, h->num_nodes)));
             const size_t cube = (size_t)(K + 1) * (K + 1) * (K + 1);  // every offset of [0, K]^3
-            HIPCHK(h, h->d2tab.ensure(cube * nlev * off_table_words(p) * 4));
+            HIPCHK(h, h->d2tab.ensure(cube * (depth - 1) * off_table_words(p) * 4));
         }
     }
     const std::function<int()> side = [&]() -> int {
@@ -875,12 +883,13 @@ static int force_fmm(nbh_handle* h, double kick_dt, bool for_vjp = false, const 
         }
         record_side(h, 1);
         if (tables) {
-            launch_dtable(m2l_deg(q), T, T.dtab, 2, nlev, K + 1, 0, 1, 0, (int)h->nsys, T.doffs, T.dsz, h->stream2);
+            launch_dtable(m2l_deg(q), T, T.dtab, T.dlevel0, nlev, K + 1, 0, 1, 0, (int)h->nsys, T.doffs, T.dsz,
+                          h->stream2);
             launch_dtable(m2l_deg(q), T, T.xtab, 1, xn, E, 1, 2, 1, (int)h->nsys, nullptr, 0, h->stream2);
             if (off) {
                 launch_off_moments(p, bf3, F.M, F.ncp, h->num_nodes, h->geo.as<int4>(), h->box.as<double4>(),
                                    h->mb.p, h->stream2);
-                launch_off_dtable(p, bf3, h->box.as<double4>(), h->cfg.eps * h->cfg.eps, 2, nlev, K + 1,
+                launch_off_dtable(p, bf3, h->box.as<double4>(), h->cfg.eps * h->cfg.eps, 2, (int)depth - 1, K + 1,
                                   h->d2tab.as<uint32_t>(), h->stream2);
             }
         }
@@ -1101,7 +1110,7 @@ static int graph_prepare(nbh_handle* h) {
     const int Kp = (int)std::floor(std::sqrt(3.0) * h->theta_den / h->theta_num);
     const int E = 2 * Kp + 1;
     const size_t dsz = (size_t)h->sl_rows, dcp = (size_t)ncp_of(m2l_deg(q));
-    HIPCHK(h, h->dtab.ensure(dsz * (g.depth_cap - 1) * dcp * 4 * h->nsys));
+    HIPCHK(h, h->dtab.ensure(dsz * (g.depth_cap + 1 - table_level0(h)) * dcp * 4 * h->nsys));
     HIPCHK(h, h->xtab.ensure((size_t)E * E * E * g.depth_cap * dcp * 4 * h->nsys));
     HIPCHK(h, h->far_src.ensure((size_t)g.far_cap * 4));
     HIPCHK(h, h->far_tgt.ensure((size_t)g.far_cap * 4));
